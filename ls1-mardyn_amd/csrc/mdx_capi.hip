@@ -31,7 +31,7 @@ __global__ void k_bin_gather(int, MolArrays, MolArrays, const int *, const int *
                              int *);
 __global__ void k_bin_gather_point(int, MolArrays, MolArrays, const int *, const int *,
                                    const int *, int *, const int *, int *, const Component *, Reps,
-                                   float *, float *, float *, int *);
+                                   float4 *, int *);
 __global__ void k_scan_block(ScanArgs);
 __global__ void k_scan_add(ScanArgs);
 __global__ void k_scan_total(ScanArgs);
@@ -57,6 +57,17 @@ using namespace mdx;
 namespace {
 thread_local std::string g_create_error;
 constexpr int kBlock = 256;
+// Boxes of at most this many cells (one-centre systems: kSmallCellsPoint) run
+// the block pair kernels, four waves per cell. A box alone gains up to 512
+// cells and beyond (9001 mixture molecules, 512 cells, FP32: 310 -> 75 us; 500 LJ
+// molecules, 64 cells: 34 -> 13.5 us), but a batch of boxes fills the chip, where
+// a cell kernel does less work per pair, and the choice may depend on the box
+// alone (a replica gives the bits it gives alone). Full batches, block kernel
+// against cell kernel: multi-site 64 x 4000 molecules 924 / 914 us, 64 x 16000
+// (beyond the line) 3760 / 2613; one-centre 512 x 500 (64 cells) 175 / 113, 512
+// x 1500 (125 cells) 607 / 251: the one-centre line lies where a lone box gains
+// more than a full batch loses.
+constexpr long kSmallCells = 512, kSmallCellsPoint = 64;
 inline int nblk(long n, int b = kBlock) { return (int)std::max<long>(1, (n + b - 1) / b); }
 
 // Scratch of the entry points that allocate nothing (mdx_adjoint_noalloc):
@@ -125,6 +136,8 @@ struct mdx_context {
     std::vector<int64_t> rep_n;  // molecules per replica (nrep > 1)
     Geom *d_geoms = nullptr;
     int *d_cell_off = nullptr, *d_cell_rep = nullptr;  // cell_rep: null for one replica
+    int nsmall = 0;              // cells of small boxes (block pair kernels)
+    int *d_small_cell = nullptr;
     int *d_mol_rep = nullptr;                          // state; null for one replica
     int *d_lf_chunk = nullptr, *d_lf_chunk_end = nullptr, *d_lf_off = nullptr;
     int lf_nchunk = 0;
@@ -445,6 +458,7 @@ int make_geom(mdx_context *c, const double *box, double rc, int periodic, int ce
         g.reflect[d] = 0;
     }
     g.wall_rc = rc;
+    g.small = ncell <= (c->point_lj ? kSmallCellsPoint : kSmallCells);
     ncell_out = ncell;
     return MDX_OK;
 }
@@ -603,6 +617,16 @@ int upload_reps(mdx_context *c) {
         TRY(dalloc(c, &c->d_cell_rep, c->ncell));
         HIPCHK(c, hipMemcpy(c->d_cell_rep, cr.data(), 4 * cr.size(), hipMemcpyHostToDevice));
     }
+    std::vector<int> small;
+    for (int r = 0; r < R; ++r)
+        if (c->geoms[r].small)
+            for (int k = c->cell_off[r]; k < c->cell_off[r + 1]; ++k) small.push_back(k);
+    c->nsmall = (int)small.size();
+    c->d_small_cell = nullptr;
+    if (c->nsmall > 0 && c->nsmall < c->ncell) {
+        TRY(dalloc(c, &c->d_small_cell, small.size()));
+        HIPCHK(c, hipMemcpy(c->d_small_cell, small.data(), 4 * small.size(), hipMemcpyHostToDevice));
+    }
     return MDX_OK;
 }
 
@@ -612,6 +636,7 @@ Reps reps(const mdx_context *c) {
     r.cell_off = c->d_cell_off;
     r.mol_rep = c->d_mol_rep;
     r.cell_rep = c->d_cell_rep;
+    r.small_cell = c->d_small_cell;
     r.nrep = c->nrep;
     return r;
 }
@@ -638,8 +663,7 @@ int alloc_sites(mdx_context *c, SiteArrays &s, int cap, int ncell, int n, int ty
     memset(&s, 0, sizeof(s));
     if (c->point_lj) {  // the rest are views of molecule arrays (site_view)
         if (type != T_LJ || cap == 0) return MDX_OK;
-        float **fp[] = {&s.fx, &s.fy, &s.fz};
-        for (float **p : fp) TRY(dalloc(c, p, cap, true));
+        TRY(dalloc(c, &s.f, cap, true));
         return dalloc(c, &s.ljid, cap, true);
     }
     TRY(dalloc(c, &s.cstart, ncell + 1, true));
@@ -649,20 +673,18 @@ int alloc_sites(mdx_context *c, SiteArrays &s, int cap, int ncell, int n, int ty
     double **dp[] = {&s.x, &s.y, &s.z, &s.mx, &s.my, &s.mz,
                      &s.Fx, &s.Fy, &s.Fz, &s.Vx, &s.Vy, &s.Vz};
     for (double **p : dp) TRY(dalloc(c, p, cap, true));
-    float **fp[] = {&s.fx, &s.fy, &s.fz, &s.fmx, &s.fmy, &s.fmz};
-    for (float **p : fp) TRY(dalloc(c, p, cap, true));
+    TRY(dalloc(c, &s.f, cap, true));
+    TRY(dalloc(c, &s.fm, cap, true));
     if (type == T_LJ) {
         TRY(dalloc(c, &s.ljid, cap, true));
     } else {
         TRY(dalloc(c, &s.p, cap, true));
-        TRY(dalloc(c, &s.fp, cap, true));
     }
     if (type == T_C) TRY(dalloc(c, &s.nhead, cap, true));
     if (type >= T_D) {
         double **ep[] = {&s.ex, &s.ey, &s.ez, &s.Mx, &s.My, &s.Mz};
         for (double **p : ep) TRY(dalloc(c, p, cap, true));
-        float **fe[] = {&s.fex, &s.fey, &s.fez};
-        for (float **p : fe) TRY(dalloc(c, p, cap, true));
+        TRY(dalloc(c, &s.fe, cap, true));
     }
     return MDX_OK;
 }
@@ -708,15 +730,15 @@ int scan_exclusive(mdx_context *c, const ScanArgs &a, int na, int level = 0) {
     return MDX_OK;
 }
 
-// Work items of cpb consecutive cells in 8 contiguous ranges (one per XCD);
-// one block per item, or blocks_per_xcd persistent blocks per XCD.
-// The quadrupole kernel takes cells two at a time, so its items are twice as
-// long (same number of cell pairs per item as single cells per item).
+// Work items in 8 contiguous ranges (one per XCD); one block per item, or
+// blocks_per_xcd persistent blocks per XCD. Items of the cell kernels: cpb
+// consecutive cells; the quadrupole kernel takes cells two at a time, so its
+// items are twice as long (same number of cell pairs per item as single cells
+// per item). Items of the block kernels: one cell of a small box.
 int cells_per_item(const mdx_context *c, int t) { return t == T_Q ? 2 * c->cpb : c->cpb; }
 
-int pair_grid(const mdx_context *c, int *items_per_xcd, int t = T_LJ) {
-    const int cpb = cells_per_item(c, t);
-    const int items = (c->ncell + cpb - 1) / cpb;
+int item_grid(const mdx_context *c, int cells, int per_item, int *items_per_xcd) {
+    const int items = (cells + per_item - 1) / per_item;
     *items_per_xcd = (items + 7) / 8;
     int per = *items_per_xcd;
     if (c->blocks_per_xcd > 0) per = std::min(per, c->blocks_per_xcd);
@@ -756,9 +778,7 @@ SiteArrays site_view(const mdx_context *c, int t) {
     s.x = s.mx = m.rx;
     s.y = s.my = m.ry;
     s.z = s.mz = m.rz;
-    s.fmx = s.fx;
-    s.fmy = s.fy;
-    s.fmz = s.fz;
+    s.fm = s.f;
     s.mol = s.mstart = c->ident;
     s.cstart = c->start;
     s.Fx = c->F;
@@ -798,7 +818,7 @@ int launch_update(mdx_context *c) {
         const SiteArrays &s = c->sites[T_LJ];
         hipLaunchKernelGGL(k_bin_gather_point, dim3(nblk(n)), dim3(kBlock), 0, c->stream, n, src,
                            dst, c->cell, c->perm, c->start, c->mcell, c->ls1id, c->mls1id,
-                           c->d_comps, reps(c), s.fx, s.fy, s.fz, s.ljid);
+                           c->d_comps, reps(c), s.f, s.ljid);
         c->cur = 1 - c->cur;
         c->binned = true;
         HIPCHK(c, hipGetLastError());
@@ -899,6 +919,8 @@ int launch_traverse(mdx_context *c, double kick = 0.0) {
     a.pp.fpar = c->d_fpar;
     a.pp.nlj = c->model.nlj;
     a.ncell = c->ncell;
+    a.nsmall = c->nsmall;
+    a.others = c->nsmall > 0;
     if (c->timing) HIPCHK(c, hipEventRecord(c->ev[0], c->stream));
     // one [ncell][4] partial array: the first i-site type writes each cell's
     // row, later types add to it (the launches are ordered on the stream)
@@ -909,14 +931,21 @@ int launch_traverse(mdx_context *c, double kick = 0.0) {
         a.accumulate = slot > 0;
         a.counters = c->d_counters + 8 * t;  // each kernel its own row
         a.cpb = cells_per_item(c, t);
-        const int grid = pair_grid(c, &a.items_per_xcd, t);
-        PairKernel k = pair_kernel(t, c->precision == MDX_PREC_FP32_FP64ACC, c->counting,
-                                   t == T_LJ && c->lj_at_origin, c->model.nlj > 1);
+        const bool fp32 = c->precision == MDX_PREC_FP32_FP64ACC, centre = t == T_LJ && c->lj_at_origin;
         if (c->timing) {
             HIPCHK(c, hipEventRecord(c->kev[slot], c->stream));
             c->kev_order[slot] = t;
         }
-        hipLaunchKernelGGL(k, dim3(grid), dim3(64), 0, c->stream, a);
+        if (c->nsmall < c->ncell) {
+            const int grid = item_grid(c, c->ncell, a.cpb, &a.items_per_xcd);
+            PairKernel k = pair_kernel(t, fp32, c->counting, centre, c->model.nlj > 1);
+            hipLaunchKernelGGL(k, dim3(grid), dim3(64), 0, c->stream, a);
+        }
+        if (c->nsmall > 0) {
+            const int grid = item_grid(c, c->nsmall, 1, &a.items_per_xcd);
+            PairKernel k = block_kernel(t, fp32, c->counting, centre, c->model.nlj);
+            hipLaunchKernelGGL(k, dim3(grid), dim3(kPairBlock), 0, c->stream, a);
+        }
         ++slot;
     }
     if (c->timing) {
@@ -1447,7 +1476,7 @@ int mdx_autotune(mdx_context *c, int reps, int32_t *chosen, double *best_ms) {
             c->cpb = cp;
             c->blocks_per_xcd = b;
             int ipx = 0;
-            (void)pair_grid(c, &ipx);
+            (void)item_grid(c, c->ncell, cells_per_item(c, T_LJ), &ipx);
             if (b > 0 && b >= ipx) continue;  // same as one block per item
             cand.push_back({cp, b});
         }

@@ -9,8 +9,8 @@
 //  * per site type t in {LJ, charge, dipole, quadrupole}: contiguous site
 //    arrays in molecule order; cell c owns sites [cstart_t[c], cstart_t[c+1]).
 //    Each site carries its position and its molecule's position (the mask is
-//    on molecule centres), FP64 absolute and FP32 relative to its cell's lower
-//    corner, its orientation (dipoles, quadrupoles) and its scalar parameter
+//    on molecule centres), FP64 absolute and FP32 relative to its cell's
+//    centre, its orientation (dipoles, quadrupoles) and its scalar parameter
 //    (LJ lookup id, charge, |mu|, |Q|), plus FP64 force / virial / torque
 //    outputs of the pair kernels.
 #pragma once
@@ -55,6 +55,7 @@ struct Geom {
                        // next re-bin moves them behind the last cell)
     double wall_rc;    // width of the wall slab checked for leaving molecules (rc)
     double rc2, rclj2, epsRFInvrc3;
+    int small;         // few cells: the block pair kernels' (mdx_pairs_block.hip)
 };
 
 // Site arrays of one type (device pointers).
@@ -62,12 +63,13 @@ struct SiteArrays {
     int *mol;                  // molecule index (current order)
     double *x, *y, *z;         // site position, FP64 absolute
     double *mx, *my, *mz;      // molecule position, FP64 absolute
-    float *fx, *fy, *fz;       // site position relative to the cell corner
-    float *fmx, *fmy, *fmz;    // molecule position relative to the cell corner
     double *ex, *ey, *ez;      // orientation (D, Q)
-    float *fex, *fey, *fez;
     double *p;                 // C: q, D: |mu|, Q: |Q|
-    float *fp;
+    float4 *f;                 // FP32 form: site position relative to the cell's corner;
+                               // w = C, D, Q parameter, or 4 * LJ lookup id as bits
+    float4 *fm;                // molecule position relative to the cell's corner; w of
+                               // charges = nhead as bits
+    float4 *fe;                // orientation (D, Q)
     int *ljid;                 // LJ lookup id
     int *nhead;                // charges: the molecule's charge count at its first
                                // charge site, 0 at the others (per-molecule tests)
@@ -115,6 +117,7 @@ struct Reps {
     const int *cell_off;   // [nrep + 1]
     const int *mol_rep;    // [n] replica of each molecule, or null
     const int *cell_rep;   // [ncell] replica of each global cell, or null
+    const int *small_cell; // global cells of the small boxes, or null where all boxes are
     int nrep;
 };
 
@@ -138,13 +141,15 @@ struct PairArgs {
     double rc2, rclj2, epsRFInvrc3;   // shared by all replicas
     SiteArrays s[kTypes];
     PairParams pp;
-    int ncell;          // global cells
-    int cpb;            // cells per work item (consecutive cells, one block)
+    int nsmall;         // cells of small boxes (block kernels: one per work item)
     int items_per_xcd;  // work items of each XCD's contiguous range
     int present[kTypes];
-    double *macro_part; // [ncell][4] sums {u6 (LJ), uXpoles, virial, rf}: each work item
-                        // stores its cells' sums in the row of its last non-empty cell
-                        // (per replica) and zeros in the others
+    int ncell;          // global cells
+    int cpb;            // cells per work item of the cell kernels
+    int others;         // some boxes are small: the cell kernels skip them
+    double *macro_part; // [ncell][4] sums {u6 (LJ), uXpoles, virial, rf}: a work item of
+                        // the cell kernels stores its cells' sums in the row of its last
+                        // non-empty cell (per replica), the block kernels each cell's
     int accumulate;     // add to macro_part rows (a later i-site type) instead of writing
     double vscale;      // factor on the written site virial: 1, or 0.5 where the site
                         // arrays are the molecule arrays (calcFM's Vi = 0.5 sum V_site)
@@ -156,7 +161,9 @@ struct PairArgs {
     unsigned long long *counters;  // [8] or null
 };
 
+constexpr int kPairBlock = 256;  // threads per block of the block kernels
 typedef void (*PairKernel)(PairArgs);
 PairKernel pair_kernel(int ti, bool fp32, bool count, bool molsite, bool multi);
+PairKernel block_kernel(int ti, bool fp32, bool count, bool molsite, int nlj);
 
 }  // namespace mdx

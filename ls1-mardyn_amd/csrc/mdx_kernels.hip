@@ -508,7 +508,7 @@ __global__ __launch_bounds__(256) void k_bin_gather_point(
     int n, MolArrays src, MolArrays dst, const int *__restrict__ cell,
     const int *__restrict__ perm, const int *__restrict__ start, int *newcell,
     const int *__restrict__ ls1id, int *newls1id, const Component *__restrict__ comps, Reps R,
-    float *fx, float *fy, float *fz, int *ljid) {
+    float4 *f, int *ljid) {
     __shared__ int win[kGatherWin];
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     int i, c;
@@ -519,10 +519,12 @@ __global__ __launch_bounds__(256) void k_bin_gather_point(
     const Geom &g = R.geom[rep];
     const int local = c - R.cell_off[rep];
     const int cx = local % g.n[0], cy = (local / g.n[0]) % g.n[1], cz = local / (g.n[0] * g.n[1]);
-    fx[d] = (float)(src.rx[i] - (g.bbmin[0] + cx * g.cl[0]));
-    fy[d] = (float)(src.ry[i] - (g.bbmin[1] + cy * g.cl[1]));
-    fz[d] = (float)(src.rz[i] - (g.bbmin[2] + cz * g.cl[2]));
-    ljid[d] = comps[src.cid[i]].lj_base;
+    const int id = comps[src.cid[i]].lj_base;
+    f[d] = make_float4((float)(src.rx[i] - (g.bbmin[0] + cx * g.cl[0])),
+                       (float)(src.ry[i] - (g.bbmin[1] + cy * g.cl[1])),
+                       (float)(src.rz[i] - (g.bbmin[2] + cz * g.cl[2])),
+                       __int_as_float(4 * id));
+    ljid[d] = id;
 }
 
 // q <- N^k(q), N = Quaternion::normalize (q scaled by 1/sqrt(|q|^2)), for
@@ -695,17 +697,18 @@ __global__ __launch_bounds__(256) void k_build_sites(int n, MolArrays s, Reps R,
                 if (t != T_LJ) A.p[j] = c.param[t][k];
             }
             if (f32) {
-                A.fx[j] = (float)(pos[0] - corner[0]);
-                A.fy[j] = (float)(pos[1] - corner[1]);
-                A.fz[j] = (float)(pos[2] - corner[2]);
-                A.fmx[j] = mrel[0]; A.fmy[j] = mrel[1]; A.fmz[j] = mrel[2];
-                if (t != T_LJ) A.fp[j] = (float)c.param[t][k];
+                A.f[j] = make_float4((float)(pos[0] - corner[0]), (float)(pos[1] - corner[1]),
+                                     (float)(pos[2] - corner[2]),
+                                     t == T_LJ ? __int_as_float(4 * (c.lj_base + k))
+                                               : (float)c.param[t][k]);
+                A.fm[j] = make_float4(mrel[0], mrel[1], mrel[2],
+                                      __int_as_float(t == T_C && k == 0 ? c.n[T_C] : 0));
             }
             if (t >= T_D) {
                 double e[3];
                 qrot(q, c.e[t][k], e);
                 if (f64) { A.ex[j] = e[0]; A.ey[j] = e[1]; A.ez[j] = e[2]; }
-                if (f32) { A.fex[j] = (float)e[0]; A.fey[j] = (float)e[1]; A.fez[j] = (float)e[2]; }
+                if (f32) A.fe[j] = make_float4((float)e[0], (float)e[1], (float)e[2], 0.f);
             }
         }
     }

@@ -1,7 +1,7 @@
 // mdx_pair_common.h -- pieces shared by the pair kernels (mdx_pairs.hip) and
 // the adjoint kernel (mdx_adjoint.hip): vector helpers, the seven site-pair
-// bodies, site accessors per precision, the neighbour-image table and the LDS
-// tile of staged neighbour sites.
+// bodies, site accessors per precision, the neighbour images of a cell and the
+// LDS tile of staged neighbour sites.
 #pragma once
 
 #include "mdx_internal.h"
@@ -185,33 +185,69 @@ __device__ __forceinline__ void body_qq(V3<R> d, V3<R> ei, R mi, V3<R> ej, R mj,
 
 // ------------------------------------------------------------- site access
 
+// a[j] with a 32-bit byte offset (at most 2^27 sites of 16 bytes): one scalar
+// base and one vector offset register instead of a 64-bit address per lane.
+template <typename T> __device__ __forceinline__ const T &item(const T *a, int j) {
+    return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(a) +
+                                        (unsigned)j * (unsigned)sizeof(T));
+}
+
+template <typename R> struct alignas(4 * sizeof(R)) Q4 {
+    R x, y, z, w;
+};
+
+// Site j of an array: site and molecule position, orientation, parameter
+// (charge, moment), LJ column (four times the lookup id), and the molecule's
+// charge count at its first charge site, 0 at the others.
 template <typename R> struct SiteView;
 
 template <> struct SiteView<double> {
     static __device__ __forceinline__ V3<double> pos(const SiteArrays &A, int j) {
-        return {A.x[j], A.y[j], A.z[j]};
+        return {item(A.x, j), item(A.y, j), item(A.z, j)};
     }
     static __device__ __forceinline__ V3<double> mol(const SiteArrays &A, int j) {
-        return {A.mx[j], A.my[j], A.mz[j]};
+        return {item(A.mx, j), item(A.my, j), item(A.mz, j)};
     }
     static __device__ __forceinline__ V3<double> ori(const SiteArrays &A, int j) {
-        return {A.ex[j], A.ey[j], A.ez[j]};
+        return {item(A.ex, j), item(A.ey, j), item(A.ez, j)};
     }
-    static __device__ __forceinline__ double par(const SiteArrays &A, int j) { return A.p[j]; }
+    static __device__ __forceinline__ double par(const SiteArrays &A, int j) { return item(A.p, j); }
+    static __device__ __forceinline__ int column(const SiteArrays &A, int j) {
+        return 4 * item(A.ljid, j);
+    }
+    static __device__ __forceinline__ int heads(const SiteArrays &A, int j) {
+        return item(A.nhead, j);
+    }
 };
 
 template <> struct SiteView<float> {
     static __device__ __forceinline__ V3<float> pos(const SiteArrays &A, int j) {
-        return {A.fx[j], A.fy[j], A.fz[j]};
+        const float4 v = item(A.f, j);
+        return {v.x, v.y, v.z};
     }
     static __device__ __forceinline__ V3<float> mol(const SiteArrays &A, int j) {
-        return {A.fmx[j], A.fmy[j], A.fmz[j]};
+        const float4 v = item(A.fm, j);
+        return {v.x, v.y, v.z};
     }
     static __device__ __forceinline__ V3<float> ori(const SiteArrays &A, int j) {
-        return {A.fex[j], A.fey[j], A.fez[j]};
+        const float4 v = item(A.fe, j);
+        return {v.x, v.y, v.z};
     }
-    static __device__ __forceinline__ float par(const SiteArrays &A, int j) { return A.fp[j]; }
+    static __device__ __forceinline__ float par(const SiteArrays &A, int j) { return item(A.f, j).w; }
+    static __device__ __forceinline__ int column(const SiteArrays &A, int j) {
+        return __float_as_int(item(A.f, j).w);
+    }
+    static __device__ __forceinline__ int heads(const SiteArrays &A, int j) {
+        return __float_as_int(item(A.fm, j).w);
+    }
 };
+
+// an LJ column as the integer bits of a record's w (FP64: of its low word)
+template <typename R> __device__ __forceinline__ R column_bits(int c);
+template <> __device__ __forceinline__ double column_bits<double>(int c) {
+    return __hiloint2double(0, c);
+}
+template <> __device__ __forceinline__ float column_bits<float>(int c) { return __int_as_float(c); }
 
 // Neighbour k (0..26, dz-major) of cell (cx,cy,cz): index of the cell that
 // holds the image, the FP64 shift of that image (0 or +-L) and the unwrapped
@@ -259,28 +295,17 @@ __device__ __forceinline__ int tile_k(const int *pre, int idx, int nb = 27) {
     return lo;
 }
 
-template <typename R>
-__device__ __forceinline__ V3<R> image_offset(const Geom &g, const Nbr &b);
-
-template <> __device__ __forceinline__ V3<double> image_offset<double>(const Geom &, const Nbr &b) {
-    return {b.s[0], b.s[1], b.s[2]};
-}
-template <> __device__ __forceinline__ V3<float> image_offset<float>(const Geom &g, const Nbr &b) {
-    return {(float)(b.dd[0] * g.cl[0]), (float)(b.dd[1] * g.cl[1]), (float)(b.dd[2] * g.cl[2])};
-}
-
 struct Acc {
     double f[3], v[3], m[3];
-    double u, vir, rf;
+    double u, rf;
 };
 
-// i-site data held in registers for the whole cell
+// i-site data held in registers for a whole pass
 template <typename R> struct ISite {
     V3<R> pos, mol, e;
     R par;
-    int ljid;
-    int ljrow;          // ljid * nlj * 4: the row of the interleaved LJ table
-    int idx;            // site index (FP64 molecule position for the cutoff re-check)
+    int ljrow;          // LJ id * nlj * 4: the row of the interleaved LJ table
+    int idx;            // site index
 };
 
 template <int TI, int TJ> struct Kind;  // 0 LJ,1 CC,2 CD,3 DD,4 CQ,5 DQ,6 QQ
@@ -295,110 +320,188 @@ template <> struct Kind<T_D, T_Q> { static constexpr int k = 5; };
 template <> struct Kind<T_Q, T_D> { static constexpr int k = 5; };
 template <> struct Kind<T_Q, T_Q> { static constexpr int k = 6; };
 
-// LDS tile: the j sites of the 27 neighbour images of one cell, positions
-// already moved into the i cell's frame (FP64: + image shift, exactly the
-// reference's halo copy r + L; FP32: + offset of the neighbour's corner).
-// One 16-byte (FP32) or 32-byte (FP64) record per site and field, so a site
-// is fetched with one or two ds_read_b128.
+// FP32 form: most pair terms a lane of a block kernel sums in FP32 before they
+// go to its FP64 accumulators (a cell kernel's lane: one drained hit list).
+// Charges: the lane meets a molecule's charges in turn with other molecules' (a
+// cell kernel's lane sums whole, neutral molecules), and the unbalanced partial
+// sums round more, so each term goes to FP64 (250 rigid water molecules, rc 12:
+// force error 5.3e-6 -> 4.8e-6, as the cell kernel's; +1.8 us at 9001
+// molecules of the mixture)
+constexpr int kPart = 24, kPartCharge = 1;
+// LJ parameters of a pair: one LJ id (scalar registers), a table in LDS (at
+// most kTableIds ids), a table in global memory
+enum { kTableNone = 0, kTableLds = 1, kTableGlobal = 2 };
+constexpr int kTableIds = 8;
 
-template <typename R> struct alignas(4 * sizeof(R)) Q4 {
-    R x, y, z, w;
-};
+template <typename R> __device__ __forceinline__ V3<R> v3(const Q4<R> &q) { return {q.x, q.y, q.z}; }
 
-template <int TI, typename R, bool MOLSITE, bool MULTI> struct TileCfg {
-    static constexpr bool ORI = TI != T_LJ;  // partners may be dipoles / quadrupoles
-    static constexpr bool MOL = !MOLSITE;    // molecule positions differ from sites
-    static constexpr bool LJID = TI == T_LJ && MULTI;  // several LJ centre types
-    // Per-lane hit list entries (LIST) and sites per LDS chunk (CAP). The
-    // kernels are bound by VALU issue, so the tile is sized for occupancy
-    // first (160 KB of LDS per CU shared by the wavefronts of its 4 SIMDs,
-    // next to the register limit of each instantiation) and chunk count
-    // second; values measured best on the 4 M-molecule LJ slab (one-centre)
-    // and the 1 M-molecule multi-site mixture (2CLJQ + water). The FP64
-    // tiles that carry molecule positions or orientations keep 16-entry
-    // lists for their larger records.
-    static constexpr int LIST = (sizeof(R) == 8 && !(TI == T_LJ && MOLSITE)) ? 16 : 24;
-    static constexpr int CAP =
-        TI == T_LJ ? (MOLSITE ? (sizeof(R) == 4 ? 352 : 192) : (sizeof(R) == 4 ? 192 : 112))
-        : TI == T_C ? (sizeof(R) == 4 ? 112 : 72)
-        : TI == T_Q ? (sizeof(R) == 4 ? 114 : 104)
-                    : (sizeof(R) == 4 ? 192 : 160);
-    // Quadrupole i sites are few per cell (one per 2CLJQ molecule) against
-    // a neighbourhood of many partner sites, so the kernel takes two cells
-    // side by side in x at a time (JOINT): their neighbourhood of 4 x 3 x 3
-    // cells is staged once for both, two thirds of what two 27-cell tiles
-    // load, at the price of tests against the 9 cells that are beyond the
-    // cutoff of one of the two (NB neighbour ranges at most).
-    static constexpr bool JOINT = TI == T_Q;
-    static constexpr int NB = JOINT ? 36 : 27;
-    // Minimum waves per SIMD the kernel's registers are allocated for (1: no
-    // bound, the compiler's choice). Tiles of at most 10 KB of LDS (lists
-    // included) let 16 blocks share a CU, 4 waves per SIMD, when the
-    // registers fit 128: the FP32 quadrupole kernel (114-site tile) and the
-    // FP64 charge kernel (72 sites) get the bound, which makes the compiler
-    // fit them with a few spilled values outside the pair loops; the FP64
-    // multi-site LJ kernel (112 sites) fits without it, and the FP64
-    // quadrupole kernel's 104-site tile (13 KB) reaches 3 waves per SIMD
-    // with its 166 registers. Measured on the mixture against the larger
-    // tiles at fewer waves: FP32 quadrupole kernel -6 %; FP64 LJ -3 %,
-    // charge -4 %, quadrupole -9 %.
-    static constexpr int WAVES =
-        (TI == T_Q && sizeof(R) == 4) || (TI == T_C && sizeof(R) == 8) ? 4 : 1;
-};
-
-template <int TI, typename R, bool MOLSITE, bool MULTI> struct Tile {
-    using C = TileCfg<TI, R, MOLSITE, MULTI>;
-    // CAP slots of the largest record set (site, molecule, orientation,
-    // head index and site count); each partner pass lays out only the records
-    // its partner type needs (PassTile), so a pass with smaller records holds
-    // more sites in the same bytes
-    static constexpr int SLOT =
-        (int)sizeof(Q4<R>) * (1 + C::MOL + C::ORI) + (C::MOL && TI != T_LJ ? 3 : 0);
-    alignas(32) unsigned char raw[C::CAP * SLOT];
-    unsigned short lst[C::LIST][64];  // per-lane hit lists (tile indices)
-    int j0[C::NB], pre[C::NB + 1];
-    double shift[C::NB][3];
-};
-
-// The records of one partner pass (partner type TJ) in a tile's slot bytes:
-// p site position (w = charge / moment, LJ table column, or |x|^2 in FP32
-// one-centre tiles), m molecule position (w = |m|^2 in FP32 tiles), e
-// orientation (dipole and quadrupole partners), h first-site (head) indices
-// and ns site counts at heads (charge partners, tested per molecule).
-template <int TI, int TJ, typename R, bool MOLSITE, bool MULTI> struct PassTile {
-    using C = TileCfg<TI, R, MOLSITE, MULTI>;
-    using TT = Tile<TI, R, MOLSITE, MULTI>;
-    static constexpr bool HEADS = C::MOL && TJ == T_C && TI != T_LJ;
-    static constexpr bool ORIJ = TI != T_LJ && TJ >= T_D;
-    static constexpr int REC = 1 + C::MOL + ORIJ;
-    static constexpr int CAP =
-        (C::CAP * TT::SLOT) / ((int)sizeof(Q4<R>) * REC + (HEADS ? 3 : 0));
-    static_assert(CAP >= C::CAP && CAP < 65536, "pass capacity");
-    Q4<R> *p, *m, *e;
-    unsigned short *h;
-    unsigned char *ns;
-    __device__ __forceinline__ explicit PassTile(TT &t) {
-        p = reinterpret_cast<Q4<R> *>(t.raw);
-        m = p + (C::MOL ? CAP : 0);
-        e = p + CAP * (1 + C::MOL);
-        h = reinterpret_cast<unsigned short *>(p + CAP * REC);
-        ns = reinterpret_cast<unsigned char *>(h + (HEADS ? CAP : 0));
+// FP32 form: partial sums of a few pair terms, added to the FP64
+// accumulators by flush().
+struct Part32 {
+    float f[3], v[3], m[3], u, rf;
+    __device__ __forceinline__ void clear() {
+        for (int k = 0; k < 3; ++k) f[k] = v[k] = m[k] = 0.f;
+        u = rf = 0.f;
+    }
+    __device__ __forceinline__ void flush(Acc &a) const {
+        for (int k = 0; k < 3; ++k) {
+            a.f[k] += (double)f[k];
+            a.v[k] += (double)v[k];
+            a.m[k] += (double)m[k];
+        }
+        a.u += (double)u;
+        a.rf += (double)rf;
     }
 };
 
-template <typename R>
-__device__ __forceinline__ V3<R> tile_offset(const Geom &g, const double (*shift)[3], int k,
-                                             int nxs);
-template <>
-__device__ __forceinline__ V3<double> tile_offset<double>(const Geom &, const double (*shift)[3],
-                                                          int k, int) {
-    return {shift[k][0], shift[k][1], shift[k][2]};
+// LJ pair seen from site i, evaluated on every lane of the wave: a lane whose
+// entry is not accepted (ok false) runs the body at a huge r^2 (FP32: +inf;
+// FP64: 1e300, which keeps the Newton steps of 1/r^2 finite), where force and
+// virial come out exactly 0, and adds no energy; u = 6 U_LJ + shift6
+// (_loopBodyLJ, VectorizedCellProcessor.cpp:171-224). FP64 form: into acc;
+// FP32 form: into the FP32 partial sums pa. tab, par: the interleaved
+// parameter table in LDS (few LJ ids) or in global memory.
+template <typename R, bool MOLSITE, int MULTI>
+__device__ __forceinline__ void eval_lj(const Q4<R> *tab, const R *par, const ISite<R> &I,
+                                        const Q4<R> &pj, const Q4<R> &mj, bool ok, R eps24, R sig2,
+                                        R shift6, Acc &acc, Part32 &pa) {
+    const V3<R> d = {I.pos.x - pj.x, I.pos.y - pj.y, I.pos.z - pj.z};
+    V3<R> dm = d;
+    if constexpr (!MOLSITE) dm = {I.mol.x - mj.x, I.mol.y - mj.y, I.mol.z - mj.z};
+    if constexpr (MULTI != kTableNone) {
+        // pj.w carries the partner's column offset (4 * its LJ id) as integer
+        // bits in the low word
+        int col;
+        if constexpr (sizeof(R) == 8)
+            col = __double2loint(pj.w);
+        else
+            col = __float_as_int(pj.w);
+        const unsigned at = (unsigned)(I.ljrow + col);
+        if constexpr (MULTI == kTableLds) {
+            const Q4<R> &t = tab[at >> 2];
+            eps24 = t.x;
+            sig2 = t.y;
+            shift6 = t.z;
+        } else if constexpr (sizeof(R) == 8) {
+            const double *t = par + at;
+            const double2 es = *reinterpret_cast<const double2 *>(t);
+            eps24 = es.x;
+            sig2 = es.y;
+            shift6 = t[2];
+        } else {
+            const float4 t = *reinterpret_cast<const float4 *>(par + at);
+            eps24 = t.x;
+            sig2 = t.y;
+            shift6 = t.z;
+        }
+    }
+    const R far = sizeof(R) == 4 ? R(__builtin_inff()) : R(1e300);
+    const R r2inv = Math<R>::rcp(ok ? dot3(d, d) : far);
+    const R lj2 = sig2 * r2inv, lj6 = lj2 * lj2 * lj2, lj12 = lj6 * lj6;
+    const R lj12m6 = lj12 - lj6;
+    const R s = eps24 * r2inv * (lj12 + lj12m6);
+    const R fx = d.x * s, fy = d.y * s, fz = d.z * s;
+    const R u = ok ? eps24 * lj12m6 + shift6 : R(0);
+    if constexpr (sizeof(R) == 4) {
+        pa.f[0] += fx;
+        pa.f[1] += fy;
+        pa.f[2] += fz;
+        pa.v[0] += dm.x * fx;
+        pa.v[1] += dm.y * fy;
+        pa.v[2] += dm.z * fz;
+        pa.u += u;
+    } else {
+        acc.f[0] += fx;
+        acc.f[1] += fy;
+        acc.f[2] += fz;
+        acc.v[0] += dm.x * fx;
+        acc.v[1] += dm.y * fy;
+        acc.v[2] += dm.z * fz;
+        acc.u += u;
+    }
 }
-template <>
-__device__ __forceinline__ V3<float> tile_offset<float>(const Geom &g, const double (*)[3], int k,
-                                                        int nxs) {
-    return {(float)((k % nxs - 1) * g.cl[0]), (float)((k / nxs % 3 - 1) * g.cl[1]),
-            (float)((k / (3 * nxs) - 1) * g.cl[2])};
+
+// One electrostatic site pair seen from site i: force on i, virial
+// (m_i - m_j) * f_i, torque on i; roles swapped where the reference swaps.
+// pj, mj, ej: the partner's site, molecule and orientation records (the
+// caller reads them from its pass's tile records; ej only for dipole and
+// quadrupole partners).
+template <int TI, int TJ, typename R, bool MOLSITE>
+__device__ __forceinline__ void eval_pair(R epsRFInvrc3, const ISite<R> &I, const Q4<R> &eq,
+                                          const Q4<R> &pj, const Q4<R> &mj,
+                                          Acc &acc, Part32 &pa) {
+    V3<R> d = {I.pos.x - pj.x, I.pos.y - pj.y, I.pos.z - pj.z};
+    V3<R> dm = d;
+    if constexpr (!MOLSITE) dm = {I.mol.x - mj.x, I.mol.y - mj.y, I.mol.z - mj.z};
+    PO<R> o;
+    o.rf = R(0);
+    R sign = R(1);
+    V3<R> tq = {R(0), R(0), R(0)};
+    static_assert(TI != T_LJ, "LJ pairs go through eval_lj");
+    V3<R> ej = {R(0), R(0), R(0)};
+    if constexpr (TJ >= T_D) ej = v3(eq);
+    const R qj = pj.w;
+    if constexpr (TI == T_C && TJ == T_C) {
+        body_cc<R>(d, I.par, qj, o);
+    } else if constexpr (TI == T_C && TJ == T_D) {
+        body_cd<R>(d, I.par, ej, qj, o);
+    } else if constexpr (TI == T_C && TJ == T_Q) {
+        body_cq<R>(d, I.par, ej, qj, o);
+    } else if constexpr (TI == T_D && TJ == T_C) {
+        V3<R> nd = {-d.x, -d.y, -d.z};
+        body_cd<R>(nd, qj, I.e, I.par, o);
+        sign = R(-1);
+        tq = o.M2;
+    } else if constexpr (TI == T_D && TJ == T_D) {
+        body_dd<R>(d, I.e, I.par, ej, qj, epsRFInvrc3, o);
+        tq = o.M1;
+    } else if constexpr (TI == T_D && TJ == T_Q) {
+        body_dq<R>(d, I.e, I.par, ej, qj, o);
+        tq = o.M1;
+    } else if constexpr (TI == T_Q && TJ == T_C) {
+        V3<R> nd = {-d.x, -d.y, -d.z};
+        body_cq<R>(nd, qj, I.e, I.par, o);
+        sign = R(-1);
+        tq = o.M2;
+    } else if constexpr (TI == T_Q && TJ == T_D) {
+        V3<R> nd = {-d.x, -d.y, -d.z};
+        body_dq<R>(nd, ej, qj, I.e, I.par, o);
+        sign = R(-1);
+        tq = o.M2;
+    } else if constexpr (TI == T_Q && TJ == T_Q) {
+        body_qq<R>(d, I.e, I.par, ej, qj, o);
+        tq = o.M1;
+    }
+    V3<R> f = {sign * o.f.x, sign * o.f.y, sign * o.f.z};
+    if constexpr (sizeof(R) == 4) {
+        pa.f[0] += f.x;
+        pa.f[1] += f.y;
+        pa.f[2] += f.z;
+        pa.v[0] += dm.x * f.x;
+        pa.v[1] += dm.y * f.y;
+        pa.v[2] += dm.z * f.z;
+        pa.u += o.u;
+        if constexpr (TI == T_D && TJ == T_D) pa.rf += o.rf;
+        if constexpr (TI >= T_D) {
+            pa.m[0] += tq.x;
+            pa.m[1] += tq.y;
+            pa.m[2] += tq.z;
+        }
+    } else {
+        acc.f[0] += f.x;
+        acc.f[1] += f.y;
+        acc.f[2] += f.z;
+        acc.v[0] += dm.x * f.x;
+        acc.v[1] += dm.y * f.y;
+        acc.v[2] += dm.z * f.z;
+        acc.u += o.u;
+        if constexpr (TI == T_D && TJ == T_D) acc.rf += o.rf;
+        if constexpr (TI >= T_D) {
+            acc.m[0] += tq.x;
+            acc.m[1] += tq.y;
+            acc.m[2] += tq.z;
+        }
+    }
 }
 
 }  // namespace mdx

@@ -1,5 +1,8 @@
 // mdx_pairs.hip -- site-pair traversal kernels (gfx950, wave64, no MFMA).
 //
+// The cell kernels, for boxes of many cells; mdx_pairs_block.hip holds the block
+// kernels of small boxes.
+//
 // The ten site-pair loops of VectorizedCellProcessor::_calculatePairs
 // (VectorizedCellProcessor.cpp:794-2730) with the seven bodies _loopBodyLJ ..
 // _loopBodyQuadrupole (VectorizedCellProcessor.cpp:171-792), evaluated owner-
@@ -27,164 +30,103 @@
 
 namespace mdx {
 
-template <typename R> __device__ __forceinline__ V3<R> v3(const Q4<R> &q) { return {q.x, q.y, q.z}; }
+// LDS tile: the j sites of the 27 neighbour images of one cell, positions
+// already moved into the i cell's frame (FP64: + image shift, exactly the
+// reference's halo copy r + L; FP32: + offset of the neighbour's corner).
+template <int TI, typename R, bool MOLSITE, bool MULTI> struct TileCfg {
+    static constexpr bool ORI = TI != T_LJ;  // partners may be dipoles / quadrupoles
+    static constexpr bool MOL = !MOLSITE;    // molecule positions differ from sites
+    static constexpr bool LJID = TI == T_LJ && MULTI;  // several LJ centre types
+    // Per-lane hit list entries (LIST) and sites per LDS chunk (CAP). The
+    // kernels are bound by VALU issue, so the tile is sized for occupancy
+    // first (160 KB of LDS per CU shared by the wavefronts of its 4 SIMDs,
+    // next to the register limit of each instantiation) and chunk count
+    // second; values measured best on the 4 M-molecule LJ slab (one-centre)
+    // and the 1 M-molecule multi-site mixture (2CLJQ + water). The FP64
+    // tiles that carry molecule positions or orientations keep 16-entry
+    // lists for their larger records.
+    static constexpr int LIST = (sizeof(R) == 8 && !(TI == T_LJ && MOLSITE)) ? 16 : 24;
+    static constexpr int CAP =
+        TI == T_LJ ? (MOLSITE ? (sizeof(R) == 4 ? 352 : 192) : (sizeof(R) == 4 ? 192 : 112))
+        : TI == T_C ? (sizeof(R) == 4 ? 112 : 72)
+        : TI == T_Q ? (sizeof(R) == 4 ? 114 : 104)
+                    : (sizeof(R) == 4 ? 192 : 160);
+    // Quadrupole i sites are few per cell (one per 2CLJQ molecule) against
+    // a neighbourhood of many partner sites, so the kernel takes two cells
+    // side by side in x at a time (JOINT): their neighbourhood of 4 x 3 x 3
+    // cells is staged once for both, two thirds of what two 27-cell tiles
+    // load, at the price of tests against the 9 cells that are beyond the
+    // cutoff of one of the two (NB neighbour ranges at most).
+    static constexpr bool JOINT = TI == T_Q;
+    static constexpr int NB = JOINT ? 36 : 27;
+    // Minimum waves per SIMD the kernel's registers are allocated for (1: no
+    // bound, the compiler's choice). Tiles of at most 10 KB of LDS (lists
+    // included) let 16 blocks share a CU, 4 waves per SIMD, when the
+    // registers fit 128: the FP32 quadrupole kernel (114-site tile) and the
+    // FP64 charge kernel (72 sites) get the bound, which makes the compiler
+    // fit them with a few spilled values outside the pair loops; the FP64
+    // multi-site LJ kernel (112 sites) fits without it, and the FP64
+    // quadrupole kernel's 104-site tile (13 KB) reaches 3 waves per SIMD
+    // with its 166 registers. Measured on the mixture against the larger
+    // tiles at fewer waves: FP32 quadrupole kernel -6 %; FP64 LJ -3 %,
+    // charge -4 %, quadrupole -9 %.
+    static constexpr int WAVES =
+        (TI == T_Q && sizeof(R) == 4) || (TI == T_C && sizeof(R) == 8) ? 4 : 1;
+};
 
-// FP32 form: partial sums of one drained hit list, folded into the FP64
-// accumulators by flush().
-struct Part32 {
-    float f[3], v[3], m[3], u, rf;
-    __device__ __forceinline__ void clear() {
-        for (int k = 0; k < 3; ++k) f[k] = v[k] = m[k] = 0.f;
-        u = rf = 0.f;
-    }
-    __device__ __forceinline__ void flush(Acc &a) const {
-        for (int k = 0; k < 3; ++k) {
-            a.f[k] += (double)f[k];
-            a.v[k] += (double)v[k];
-            a.m[k] += (double)m[k];
-        }
-        a.u += (double)u;
-        a.rf += (double)rf;
+template <int TI, typename R, bool MOLSITE, bool MULTI> struct Tile {
+    using C = TileCfg<TI, R, MOLSITE, MULTI>;
+    // CAP slots of the largest record set (site, molecule, orientation,
+    // head index and site count); each partner pass lays out only the records
+    // its partner type needs (PassTile), so a pass with smaller records holds
+    // more sites in the same bytes
+    static constexpr int SLOT =
+        (int)sizeof(Q4<R>) * (1 + C::MOL + C::ORI) + (C::MOL && TI != T_LJ ? 3 : 0);
+    alignas(32) unsigned char raw[C::CAP * SLOT];
+    unsigned short lst[C::LIST][64];  // per-lane hit lists (tile indices)
+    int j0[C::NB], pre[C::NB + 1];
+    double shift[C::NB][3];
+};
+
+// The records of one partner pass (partner type TJ) in a tile's slot bytes:
+// p site position (w = charge / moment, LJ table column, or |x|^2 in FP32
+// one-centre tiles), m molecule position (w = |m|^2 in FP32 tiles), e
+// orientation (dipole and quadrupole partners), h first-site (head) indices
+// and ns site counts at heads (charge partners, tested per molecule).
+template <int TI, int TJ, typename R, bool MOLSITE, bool MULTI> struct PassTile {
+    using C = TileCfg<TI, R, MOLSITE, MULTI>;
+    using TT = Tile<TI, R, MOLSITE, MULTI>;
+    static constexpr bool HEADS = C::MOL && TJ == T_C && TI != T_LJ;
+    static constexpr bool ORIJ = TI != T_LJ && TJ >= T_D;
+    static constexpr int REC = 1 + C::MOL + ORIJ;
+    static constexpr int CAP =
+        (C::CAP * TT::SLOT) / ((int)sizeof(Q4<R>) * REC + (HEADS ? 3 : 0));
+    static_assert(CAP >= C::CAP && CAP < 65536, "pass capacity");
+    Q4<R> *p, *m, *e;
+    unsigned short *h;
+    unsigned char *ns;
+    __device__ __forceinline__ explicit PassTile(TT &t) {
+        p = reinterpret_cast<Q4<R> *>(t.raw);
+        m = p + (C::MOL ? CAP : 0);
+        e = p + CAP * (1 + C::MOL);
+        h = reinterpret_cast<unsigned short *>(p + CAP * REC);
+        ns = reinterpret_cast<unsigned char *>(h + (HEADS ? CAP : 0));
     }
 };
 
-// LJ pair seen from site i, evaluated on every lane of the wave: a lane
-// whose entry is not accepted (ok false) runs the body at a huge r^2 (FP32:
-// +inf; FP64: 1e300, which keeps the Newton steps of 1/r^2 finite), where
-// force and virial come out exactly 0, and adds no energy; u = 6 U_LJ +
-// shift6 (_loopBodyLJ, VectorizedCellProcessor.cpp:171-224). FP64 form: into
-// acc; FP32 form: into the drain's FP32 partial sums pa.
-template <typename R, bool MOLSITE, bool MULTI>
-__device__ __forceinline__ void eval_lj(const PairArgs &a, const ISite<R> &I, const Q4<R> &pj,
-                                        const Q4<R> &mj, bool ok, R eps24, R sig2, R shift6,
-                                        Acc &acc, Part32 &pa) {
-    const V3<R> d = {I.pos.x - pj.x, I.pos.y - pj.y, I.pos.z - pj.z};
-    V3<R> dm = d;
-    if constexpr (!MOLSITE) dm = {I.mol.x - mj.x, I.mol.y - mj.y, I.mol.z - mj.z};
-    if constexpr (MULTI) {
-        // pj.w carries the partner's column offset (4 * its LJ id) as integer
-        // bits in the low word
-        if constexpr (sizeof(R) == 8) {
-            const double *t = a.pp.dpar + (unsigned)(I.ljrow + __double2loint(pj.w));
-            const double2 es = *reinterpret_cast<const double2 *>(t);
-            eps24 = es.x;
-            sig2 = es.y;
-            shift6 = t[2];
-        } else {
-            const float4 t =
-                *reinterpret_cast<const float4 *>(a.pp.fpar + (unsigned)(I.ljrow + __float_as_int(pj.w)));
-            eps24 = t.x;
-            sig2 = t.y;
-            shift6 = t.z;
-        }
-    }
-    const R far = sizeof(R) == 4 ? R(__builtin_inff()) : R(1e300);
-    const R r2inv = Math<R>::rcp(ok ? dot3(d, d) : far);
-    const R lj2 = sig2 * r2inv, lj6 = lj2 * lj2 * lj2, lj12 = lj6 * lj6;
-    const R lj12m6 = lj12 - lj6;
-    const R s = eps24 * r2inv * (lj12 + lj12m6);
-    const R fx = d.x * s, fy = d.y * s, fz = d.z * s;
-    const R u = ok ? eps24 * lj12m6 + shift6 : R(0);
-    if constexpr (sizeof(R) == 4) {
-        pa.f[0] += fx;
-        pa.f[1] += fy;
-        pa.f[2] += fz;
-        pa.v[0] += dm.x * fx;
-        pa.v[1] += dm.y * fy;
-        pa.v[2] += dm.z * fz;
-        pa.u += u;
-    } else {
-        acc.f[0] += fx;
-        acc.f[1] += fy;
-        acc.f[2] += fz;
-        acc.v[0] += dm.x * fx;
-        acc.v[1] += dm.y * fy;
-        acc.v[2] += dm.z * fz;
-        acc.u += u;
-    }
+template <typename R>
+__device__ __forceinline__ V3<R> tile_offset(const Geom &g, const double (*shift)[3], int k,
+                                             int nxs);
+template <>
+__device__ __forceinline__ V3<double> tile_offset<double>(const Geom &, const double (*shift)[3],
+                                                          int k, int) {
+    return {shift[k][0], shift[k][1], shift[k][2]};
 }
-
-// One electrostatic site pair seen from site i: force on i, virial
-// (m_i - m_j) * f_i, torque on i; roles swapped where the reference swaps.
-// pj, mj, ej: the partner's site, molecule and orientation records (the
-// caller reads them from its pass's tile records; ej only for dipole and
-// quadrupole partners).
-template <int TI, int TJ, typename R, bool MOLSITE, bool MULTI>
-__device__ __forceinline__ void eval_pair(const PairArgs &a, const ISite<R> &I,
-                                          const Q4<R> &eq, const Q4<R> &pj, const Q4<R> &mj,
-                                          R eps24, R sig2, R shift6, Acc &acc, Part32 &pa) {
-    V3<R> d = {I.pos.x - pj.x, I.pos.y - pj.y, I.pos.z - pj.z};
-    V3<R> dm = d;
-    if constexpr (!MOLSITE) dm = {I.mol.x - mj.x, I.mol.y - mj.y, I.mol.z - mj.z};
-    PO<R> o;
-    o.rf = R(0);
-    R sign = R(1);
-    V3<R> tq = {R(0), R(0), R(0)};
-    static_assert(TI != T_LJ, "LJ pairs go through eval_lj");
-    V3<R> ej = {R(0), R(0), R(0)};
-    if constexpr (TJ >= T_D) ej = v3(eq);
-    const R qj = pj.w;
-    if constexpr (TI == T_C && TJ == T_C) {
-        body_cc<R>(d, I.par, qj, o);
-    } else if constexpr (TI == T_C && TJ == T_D) {
-        body_cd<R>(d, I.par, ej, qj, o);
-    } else if constexpr (TI == T_C && TJ == T_Q) {
-        body_cq<R>(d, I.par, ej, qj, o);
-    } else if constexpr (TI == T_D && TJ == T_C) {
-        V3<R> nd = {-d.x, -d.y, -d.z};
-        body_cd<R>(nd, qj, I.e, I.par, o);
-        sign = R(-1);
-        tq = o.M2;
-    } else if constexpr (TI == T_D && TJ == T_D) {
-        body_dd<R>(d, I.e, I.par, ej, qj, (R)a.epsRFInvrc3, o);
-        tq = o.M1;
-    } else if constexpr (TI == T_D && TJ == T_Q) {
-        body_dq<R>(d, I.e, I.par, ej, qj, o);
-        tq = o.M1;
-    } else if constexpr (TI == T_Q && TJ == T_C) {
-        V3<R> nd = {-d.x, -d.y, -d.z};
-        body_cq<R>(nd, qj, I.e, I.par, o);
-        sign = R(-1);
-        tq = o.M2;
-    } else if constexpr (TI == T_Q && TJ == T_D) {
-        V3<R> nd = {-d.x, -d.y, -d.z};
-        body_dq<R>(nd, ej, qj, I.e, I.par, o);
-        sign = R(-1);
-        tq = o.M2;
-    } else if constexpr (TI == T_Q && TJ == T_Q) {
-        body_qq<R>(d, I.e, I.par, ej, qj, o);
-        tq = o.M1;
-    }
-    V3<R> f = {sign * o.f.x, sign * o.f.y, sign * o.f.z};
-    if constexpr (sizeof(R) == 4) {
-        pa.f[0] += f.x;
-        pa.f[1] += f.y;
-        pa.f[2] += f.z;
-        pa.v[0] += dm.x * f.x;
-        pa.v[1] += dm.y * f.y;
-        pa.v[2] += dm.z * f.z;
-        pa.u += o.u;
-        if constexpr (TI == T_D && TJ == T_D) pa.rf += o.rf;
-        if constexpr (TI >= T_D) {
-            pa.m[0] += tq.x;
-            pa.m[1] += tq.y;
-            pa.m[2] += tq.z;
-        }
-    } else {
-        acc.f[0] += f.x;
-        acc.f[1] += f.y;
-        acc.f[2] += f.z;
-        acc.v[0] += dm.x * f.x;
-        acc.v[1] += dm.y * f.y;
-        acc.v[2] += dm.z * f.z;
-        acc.u += o.u;
-        if constexpr (TI == T_D && TJ == T_D) acc.rf += o.rf;
-        if constexpr (TI >= T_D) {
-            acc.m[0] += tq.x;
-            acc.m[1] += tq.y;
-            acc.m[2] += tq.z;
-        }
-    }
+template <>
+__device__ __forceinline__ V3<float> tile_offset<float>(const Geom &g, const double (*)[3], int k,
+                                                        int nxs) {
+    return {(float)((k % nxs - 1) * g.cl[0]), (float)((k / nxs % 3 - 1) * g.cl[1]),
+            (float)((k / (3 * nxs) - 1) * g.cl[2])};
 }
 
 constexpr int kUnroll = 4;  // stage-A candidates in flight per lane
@@ -203,6 +145,12 @@ __device__ __forceinline__ void partner_pass(const PairArgs &a, const Geom &g, i
                                              Tile<TI, R, MOLSITE, MULTI> &T, Acc &acc, R eps24,
                                              R sig2, R shift6, unsigned long long &ntest) {
     using C = TileCfg<TI, R, MOLSITE, MULTI>;
+    constexpr int TAB = MULTI ? kTableGlobal : kTableNone;
+    const R *par;  // the interleaved LJ table
+    if constexpr (sizeof(R) == 8)
+        par = a.pp.dpar;
+    else
+        par = a.pp.fpar;
     const SiteArrays &J = a.s[TJ];
     const double rc2 = (TI == T_LJ) ? a.rclj2 : a.rc2;
     const R rc2r = (R)rc2;
@@ -277,7 +225,7 @@ __device__ __forceinline__ void partner_pass(const PairArgs &a, const Geom &g, i
             if (base + nst < total) {
                 const int idx = base + nst;
                 const int k = tile_k(T.pre, idx, nb);
-                next_head = J.nhead[T.j0[k] + (idx - T.pre[k])];
+                next_head = SiteView<R>::heads(J, T.j0[k] + (idx - T.pre[k]));
             }
         }
         int nh = nst;
@@ -296,19 +244,15 @@ __device__ __forceinline__ void partner_pass(const PairArgs &a, const Geom &g, i
             q.y = p.y + off.y;
             q.z = p.z + off.z;
             q.w = R(0);
-            if constexpr (C::LJID) {  // column offset of the interleaved table, as bits
-                if constexpr (sizeof(R) == 8)
-                    q.w = __hiloint2double(0, 4 * J.ljid[j]);
-                else
-                    q.w = __int_as_float(4 * J.ljid[j]);
-            }
+            // column offset of the interleaved table, as bits
+            if constexpr (C::LJID) q.w = column_bits<R>(SiteView<R>::column(J, j));
             if constexpr (TI != T_LJ) q.w = SiteView<R>::par(J, j);
             if constexpr (NORM && !C::MOL) q.w = q.x * q.x + q.y * q.y + q.z * q.z;
             V.p[s] = q;
             if constexpr (C::MOL) {
                 const V3<R> m = SiteView<R>::mol(J, j);
                 if constexpr (heads) {
-                    const int w = J.nhead[j];
+                    const int w = SiteView<R>::heads(J, j);
                     head = w != 0;
                     V.ns[s] = (unsigned char)w;
                 }
@@ -397,7 +341,8 @@ __device__ __forceinline__ void partner_pass(const PairArgs &a, const Geom &g, i
                         ok = ok && !b;
                     }
                     const Q4<R> pj = C::MOL ? V.p[sj] : qj;
-                    eval_lj<R, MOLSITE, MULTI>(a, I, pj, qj, ok, eps24, sig2, shift6, acc, pa);
+                    eval_lj<R, MOLSITE, TAB>((const Q4<R> *)nullptr, par, I, pj, qj, ok, eps24,
+                                                sig2, shift6, acc, pa);
                     if (COUNT) nhit += ok;
                 }
                 if constexpr (sizeof(R) == 4) {
@@ -409,7 +354,8 @@ __device__ __forceinline__ void partner_pass(const PairArgs &a, const Geom &g, i
                         const bool ok = has && recheck(sj);
                         const Q4<R> qj = C::MOL ? V.m[sj] : V.p[sj];
                         const Q4<R> pj = C::MOL ? V.p[sj] : qj;
-                        eval_lj<R, MOLSITE, MULTI>(a, I, pj, qj, ok, eps24, sig2, shift6, acc, pa);
+                        eval_lj<R, MOLSITE, TAB>((const Q4<R> *)nullptr, par, I, pj, qj, ok, eps24,
+                                                sig2, shift6, acc, pa);
                         if (COUNT) nhit += ok;
                     }
                 }
@@ -438,16 +384,14 @@ __device__ __forceinline__ void partner_pass(const PairArgs &a, const Geom &g, i
                             const int ns = (int)V.ns[sj];  // the molecule's sites sj .. sj + ns - 1
                             for (int t = 0; t < ns; ++t) {
                                 const Q4<R> pj = V.p[sj + t];
-                                eval_pair<TI, TJ, R, MOLSITE, MULTI>(a, I, Q4<R>{}, pj, qj,
-                                                                     eps24, sig2, shift6, acc, pa);
+                                eval_pair<TI, TJ, R, MOLSITE>((R)a.epsRFInvrc3, I, Q4<R>{}, pj, qj, acc, pa);
                             }
                             if (COUNT) nhit += ns;
                         } else {
                             const Q4<R> pj = C::MOL ? V.p[sj] : qj;
                             Q4<R> eq{};
                             if constexpr (PT::ORIJ) eq = V.e[sj];
-                            eval_pair<TI, TJ, R, MOLSITE, MULTI>(a, I, eq, pj, qj, eps24, sig2,
-                                                                 shift6, acc, pa);
+                            eval_pair<TI, TJ, R, MOLSITE>((R)a.epsRFInvrc3, I, eq, pj, qj, acc, pa);
                             if (COUNT) ++nhit;
                         }
                     }
@@ -599,13 +543,12 @@ __device__ __forceinline__ bool pair_cell(const PairArgs &a, Tile<TI, R, MOLSITE
             I.idx = i;
             if constexpr (TI >= T_D) I.e = SiteView<R>::ori(S, i);
             if constexpr (TI == T_LJ) {
-                I.ljid = S.ljid[i];
-                I.ljrow = 4 * a.pp.nlj * I.ljid;
+                I.ljrow = MULTI ? a.pp.nlj * SiteView<R>::column(S, i) : 0;
             } else
                 I.par = SiteView<R>::par(S, i);
             Acc acc;
             for (int k = 0; k < 3; ++k) acc.f[k] = acc.v[k] = acc.m[k] = 0.0;
-            acc.u = acc.vir = acc.rf = 0.0;
+            acc.u = acc.rf = 0.0;
             if constexpr (TI == T_LJ) {
                 partner_pass<T_LJ, T_LJ, R, MOLSITE, MULTI, COUNT>(a, g, cbase, I, valid, cx, cy, cz, nxs, ph, P,
                                                                    lane, T, acc, eps24, sig2,
@@ -718,6 +661,10 @@ __global__ __launch_bounds__(64) __attribute__((
         int last = -1, rep_prev = -1;
         for (int cell = c0; cell < c1;) {
             const int rep = cell_replica(a.R, cell);
+            if (a.others && a.R.geom[rep].small) {  // the block kernels'
+                ++cell;
+                continue;
+            }
             if (rep != rep_prev && last >= 0) {  // rows never mix replicas
                 flush_macro<TI>(a, wmac, last, lane);
                 last = -1;
@@ -765,11 +712,14 @@ __global__ void k_enum_pairs(Geom g, int ncell, int *out) {
     out[2 * t + 1] = b.ok ? e2 : -1;
 }
 
-// Host-side launcher table.
-template <int T, typename R, bool C>
-PairKernel pick(bool molsite, bool multi) {
-    if (molsite) return multi ? k_pairs<T, R, C, true, true> : k_pairs<T, R, C, true, false>;
-    return multi ? k_pairs<T, R, C, false, true> : k_pairs<T, R, C, false, false>;
+// Host-side launcher table (the molecule-centre and several-type variants are
+// LJ's only).
+template <int T, typename R, bool C> PairKernel pick(bool molsite, bool multi) {
+    if constexpr (T == T_LJ) {
+        if (molsite) return multi ? k_pairs<T, R, C, true, true> : k_pairs<T, R, C, true, false>;
+        if (multi) return k_pairs<T, R, C, false, true>;
+    }
+    return k_pairs<T, R, C, false, false>;
 }
 
 template <int T> PairKernel pick_t(bool fp32, bool count, bool molsite, bool multi) {
