@@ -15,16 +15,18 @@
 
 namespace mdx {
 __global__ void k_leapfrog_pre(MolArrays, const double *, const double *, const Component *, Reps,
-                               double, int);
+                               double, int, Bins);
+template <bool SITES>
+__global__ void k_leapfrog_post(MolArrays, double *, double *, double *, const Component *, int,
+                                Reps, double, int, const int *, const int *, double *, int, int,
+                                SiteArrays, SiteArrays, SiteArrays, SiteArrays, const double *);
+template <bool SITES>
 __global__ void k_leapfrog_post_pre(MolArrays, const double *, const double *, const Component *,
-                                    Reps, double, int, const int *, const int *, double *);
-__global__ void k_leapfrog_post(MolArrays, const double *, const double *, const Component *,
-                                double, int, const int *, const int *, double *, int, int);
-__global__ void k_seg_reduce(const double *, int, const int *, double *);
+                                    int, Reps, double, int, const int *, const int *, double *,
+                                    Bins, SiteArrays, SiteArrays, SiteArrays, SiteArrays);
 __global__ void k_reduce_partials(const double *, int, int, int, double *);
 __global__ void k_fill_int(int *, int, int);
-__global__ void k_fill_double(double *, int, double);
-__global__ void k_bin_count(MolArrays, Reps, int, int *, int *, int *, int *);
+__global__ void k_bin_count(MolArrays, Reps, int, Bins);
 __global__ void k_bin_scatter(int, const int *, const int *, const int *, int *);
 __global__ void k_bin_gather(int, MolArrays, MolArrays, const int *, const int *, const int *,
                              int *, const int *, int *, const Component *, int *, int *, int *,
@@ -34,10 +36,10 @@ __global__ void k_bin_gather_point(int, MolArrays, MolArrays, const int *, const
                                    float4 *, int *);
 __global__ void k_scan_block(ScanArgs);
 __global__ void k_scan_add(ScanArgs);
-__global__ void k_scan_total(ScanArgs);
-__global__ void k_cell_site_start(int, const int *, ScanArgs);
+__global__ void k_scan_one(ScanArgs);
 __global__ void k_build_sites(int, MolArrays, Reps, const int *, const Component *, int, int,
-                              int, SiteArrays, SiteArrays, SiteArrays, SiteArrays);
+                              int, int, const int *, SiteArrays, SiteArrays, SiteArrays,
+                              SiteArrays);
 __global__ void k_calc_fm(int, MolArrays, const Component *, int, SiteArrays, SiteArrays,
                           SiteArrays, SiteArrays, double *, double *, double *, Reps,
                           const double *);
@@ -45,10 +47,7 @@ __global__ void k_velocity_scale(MolArrays, double *, double *, const Component 
                                  const double *, int);
 __global__ void k_scatter_orig(int, const int *, const double *, double *, int, int);
 __global__ void k_normalize_q(int, MolArrays, long long);
-__global__ void k_finalize_macro(const double *, double *, double *, const int *, int,
-                                 const double *);
-__global__ void k_finalize_lf(const double *, double *, const int *, int, double *, int);
-__global__ void k_step_advance(int *);
+__global__ void k_step_end(StepEnd);
 __global__ void k_enum_pairs(Geom, int, int *);
 }  // namespace mdx
 
@@ -152,7 +151,6 @@ struct mdx_context {
     double *F = nullptr, *M = nullptr, *Vi = nullptr;
     int *cell = nullptr, *rank = nullptr, *count = nullptr, *start = nullptr, *perm = nullptr,
         *mcell = nullptr, *ls1id = nullptr, *mls1id = nullptr;
-    double *red_tmp = nullptr;  // first level of the two-level reductions
     double *dl_tmp = nullptr;   // download staging (4 n)
     double *adj_site = nullptr, *adj_cot = nullptr, *adj_part = nullptr, *adj_out = nullptr;
     double *scratch = nullptr;  // this device's copy of the library scratch array
@@ -167,7 +165,8 @@ struct mdx_context {
     std::vector<ScanLevel> scan_tmp;
     int site_forms = 0;  // site record forms built for the current re-bin (1 FP64, 2 FP32)
     double *macro_part = nullptr, *lf_part = nullptr, *red = nullptr, *step_out = nullptr;
-    int *step_idx = nullptr;
+    double *end_part = nullptr;  // k_step_end's block sums, tickets and step counts
+    int *end_ticket = nullptr, *step_idx = nullptr;
     int cap_steps = 0;
     unsigned long long *d_counters = nullptr;
     std::vector<uint64_t> ids;
@@ -604,7 +603,12 @@ int upload_reps(mdx_context *c) {
     const int R = c->nrep;
     TRY(dalloc(c, &c->d_geoms, R));
     TRY(dalloc(c, &c->d_cell_off, R + 1));
-    TRY(dalloc(c, &c->red, 12 * (size_t)R));
+    TRY(dalloc(c, &c->red, 8 * (size_t)R));
+    TRY(dalloc(c, &c->end_part, (size_t)R * kStepBlocks * 8));
+    TRY(dalloc(c, &c->end_ticket, R));
+    TRY(dalloc(c, &c->step_idx, R));
+    HIPCHK(c, hipMemset(c->end_ticket, 0, 4 * (size_t)R));
+    HIPCHK(c, hipMemset(c->step_idx, 0, 4 * (size_t)R));
     TRY(dalloc(c, &c->d_thermo, (size_t)kThermoW * R));
     HIPCHK(c, hipMemcpy(c->d_geoms, c->geoms.data(), sizeof(Geom) * R, hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->d_cell_off, c->cell_off.data(), 4 * (size_t)(R + 1),
@@ -705,28 +709,36 @@ int alloc_scan(mdx_context *c, int n) {
 }
 
 // Exclusive scans of na arrays of a.n ints each in one set of launches
-// (array t on blockIdx.y), out_t[n] = total of in_t, on the context stream.
+// (array t on blockIdx.y), out_t[n] = total of in_t, on the context stream: one
+// block each up to kScanOne ints, else blocks of 1024 ints that are added up
+// behind (the adding block sums the block sums before it while those are few,
+// else they are scanned first). 1 M molecules' site counts: two launches of 7 and
+// 6 us, which were four of 5 us each and their gaps.
+constexpr int kScanSelf = 4096;  // most block sums that the adding blocks sum themselves
 int scan_exclusive(mdx_context *c, const ScanArgs &a, int na, int level = 0) {
     const int n = a.n;
-    const int nb = std::max(1, (n + 1023) / 1024);
+    if (n <= kScanOne) {
+        hipLaunchKernelGGL(k_scan_one, dim3(1, na), dim3(1024), 0, c->stream, a);
+        return MDX_OK;
+    }
+    const int nb = (n + 1023) / 1024;
     if (level >= (int)c->scan_tmp.size()) return fail(c, MDX_ERR_CAPACITY, "scan depth");
     const mdx_context::ScanLevel &L = c->scan_tmp[level];
     ScanArgs blk = a, sub = a, add = a;
     sub.n = nb;
+    sub.clear = 0;
+    add.scanned = nb > kScanSelf;
     for (int t = 0; t < na; ++t) {
         int *bsum = L.p + (size_t)t * L.seg;
         int *bscan = bsum + ((nb + 1023) / 1024) * 1024;
         blk.aux[t] = bsum;
         sub.in[t] = bsum;
         sub.out[t] = bscan;
-        add.aux[t] = bscan;
+        add.aux[t] = add.scanned ? bscan : bsum;
     }
     hipLaunchKernelGGL(k_scan_block, dim3(nb, na), dim3(256), 0, c->stream, blk);
-    if (nb > 1) {
-        TRY(scan_exclusive(c, sub, na, level + 1));
-        hipLaunchKernelGGL(k_scan_add, dim3(nb, na), dim3(256), 0, c->stream, add);
-    }
-    if (level == 0) hipLaunchKernelGGL(k_scan_total, dim3(1, na), dim3(1), 0, c->stream, a);
+    if (add.scanned) TRY(scan_exclusive(c, sub, na, level + 1));
+    hipLaunchKernelGGL(k_scan_add, dim3(nb, na), dim3(256), 0, c->stream, add);
     return MDX_OK;
 }
 
@@ -749,21 +761,6 @@ int n_present(const mdx_context *c) {
     int k = 0;
     for (int t = 0; t < kTypes; ++t) k += c->nsites[t] > 0;
     return k;
-}
-
-// Sum of nb blocks x width partials into out[width], fixed order.
-void launch_reduce(mdx_context *c, const double *in, int nb, int width, double *out) {
-    const int g1 = 256;
-    if (nb <= 4 * g1) {
-        hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(256), 0, c->stream, in, nb, width, nb,
-                           out);
-        return;
-    }
-    const int per = (nb + g1 - 1) / g1;
-    hipLaunchKernelGGL(k_reduce_partials, dim3(g1), dim3(256), 0, c->stream, in, nb, width, per,
-                       c->red_tmp);
-    hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(256), 0, c->stream, c->red_tmp, g1, width,
-                       g1, out);
 }
 
 // The site arrays of type t as the kernels see them. For point_lj systems
@@ -797,20 +794,26 @@ int rebin_forms(const mdx_context *c) {
 
 // Re-bin (LinkedCells::update + exchangeMolecules' periodic wrap, which
 // leapfrog_pre already applied) and SoA cache build (setupSoACache).
-int launch_update(mdx_context *c) {
+// counted: the drift has binned the molecules already (bins()).
+Bins bins(const mdx_context *c) { return {c->cell, c->rank, c->count, c->ls1id}; }
+
+int launch_update(mdx_context *c, bool counted = false) {
     const int n = c->n;
     if (c->point_lj) ++c->q_renorm;
     MolArrays &src = c->mol[c->cur], &dst = c->mol[1 - c->cur];
-    hipLaunchKernelGGL(k_fill_int, dim3(nblk(c->ncell + 2)), dim3(kBlock), 0, c->stream, c->count,
-                       c->ncell + 2, 0);
-    hipLaunchKernelGGL(k_bin_count, dim3(nblk(n)), dim3(kBlock), 0, c->stream, src, reps(c), n,
-                       c->cell, c->rank, c->count, c->ls1id);
+    if (!counted) {
+        hipLaunchKernelGGL(k_fill_int, dim3(nblk(c->ncell + 2)), dim3(kBlock), 0, c->stream,
+                           c->count, c->ncell + 2, 0);
+        hipLaunchKernelGGL(k_bin_count, dim3(nblk(n)), dim3(kBlock), 0, c->stream, src, reps(c), n,
+                           bins(c));
+    }
     // the cells and the bin of deleted molecules behind them: start[ncell] is
     // the live count, start[ncell + 1] = n
     ScanArgs cells{};
     cells.in[0] = c->count;
     cells.out[0] = c->start;
     cells.n = c->ncell + 1;
+    cells.clear = 1;  // for the drift's binning
     TRY(scan_exclusive(c, cells, 1));
     hipLaunchKernelGGL(k_bin_scatter, dim3(nblk(n)), dim3(kBlock), 0, c->stream, n, c->cell,
                        c->rank, c->start, c->perm);
@@ -830,30 +833,24 @@ int launch_update(mdx_context *c) {
                        c->nsite_mol[1], c->nsite_mol[2], c->nsite_mol[3]);
     c->cur = 1 - c->cur;
     // per site type: molecule site starts (scan of the per-molecule site
-    // counts), then cell site starts, all present types in one launch each
-    ScanArgs ms{}, cs{};
+    // counts); the build below takes the cells' site starts from them
+    ScanArgs ms{};
     int na = 0;
     for (int t = 0; t < kTypes; ++t) {
         if (c->nsites[t] == 0) continue;
         ms.in[na] = c->nsite_mol[t];
         ms.out[na] = c->sites[t].mstart;
-        cs.in[na] = c->sites[t].mstart;
-        cs.out[na] = c->sites[t].cstart;
         ++na;
     }
     ms.n = n;
-    if (na > 0) {
-        TRY(scan_exclusive(c, ms, na));
-        hipLaunchKernelGGL(k_cell_site_start, dim3(nblk(c->ncell + 1), na), dim3(kBlock), 0,
-                           c->stream, c->ncell, c->start, cs);
-    }
+    if (na > 0) TRY(scan_exclusive(c, ms, na));
     // the site records of the current precision form only; another form is
     // added on demand (ensure_sites)
     const int nc = c->model.ncomp;
     const int forms = rebin_forms(c);
     hipLaunchKernelGGL(k_build_sites, dim3(nblk(n)), dim3(kBlock), nc * sizeof(Component),
                        c->stream, n, c->mol[c->cur], reps(c), c->mcell, c->d_comps, nc, forms,
-                       1, c->sites[0], c->sites[1], c->sites[2], c->sites[3]);
+                       1, c->ncell, c->start, c->sites[0], c->sites[1], c->sites[2], c->sites[3]);
     c->site_forms = forms;
     c->binned = true;
     HIPCHK(c, hipGetLastError());
@@ -876,16 +873,43 @@ int ensure_sites(mdx_context *c, int need) {
     const int nc = c->model.ncomp, n = c->n;
     hipLaunchKernelGGL(k_build_sites, dim3(nblk(n)), dim3(kBlock), nc * sizeof(Component),
                        c->stream, n, c->mol[c->cur], reps(c), c->mcell, c->d_comps, nc,
-                       need & ~c->site_forms, 0, c->sites[0], c->sites[1], c->sites[2],
-                       c->sites[3]);
+                       need & ~c->site_forms, 0, c->ncell, c->start, c->sites[0], c->sites[1],
+                       c->sites[2], c->sites[3]);
     c->site_forms |= need;
     HIPCHK(c, hipGetLastError());
     return MDX_OK;
 }
 
+// The step's sums (k_step_end) of what: macroscopic values, leapfrog sums, the
+// step count.
+void launch_step_end(mdx_context *c, int what) {
+    StepEnd e;
+    memset(&e, 0, sizeof(e));
+    e.macro_part = n_present(c) > 0 ? c->macro_part : nullptr;
+    e.lf_part = c->lf_part;
+    e.cell_off = c->d_cell_off;
+    e.lf_off = c->d_lf_off;
+    e.part = c->end_part;
+    e.ticket = c->end_ticket;
+    e.macro = c->red;
+    e.sums = c->red + 4 * (size_t)c->nrep;
+    e.step_out = c->step_out;
+    e.step_idx = c->step_idx;
+    e.lrc = c->lrc ? c->d_thermo : nullptr;
+    e.thermo = c->thermostat ? c->d_thermo : nullptr;
+    e.nrep = c->nrep;
+    e.heuristics = c->heuristics;
+    e.what = what;
+    int cells = 0;
+    for (int r = 0; r < c->nrep; ++r) cells = std::max(cells, c->cell_off[r + 1] - c->cell_off[r]);
+    const int nb = std::max(1, std::min(kStepBlocks, (cells + kStepRows - 1) / kStepRows));
+    hipLaunchKernelGGL(k_step_end, dim3(nb, c->nrep), dim3(256), 0, c->stream, e);
+}
+
 // kick != 0 (reduced-memory mode): the pair kernel adds kick * F to the
-// velocities instead of storing F and Vi.
-int launch_traverse(mdx_context *c, double kick = 0.0) {
+// velocities instead of storing F and Vi. in_step: the molecules' F, M and Vi
+// and the macroscopic values are left to the kernels that end the step.
+int launch_traverse(mdx_context *c, double kick = 0.0, bool in_step = false) {
     TRY(ensure_sites(c, rebin_forms(c)));
     PairArgs a;
     memset(&a, 0, sizeof(a));
@@ -953,14 +977,10 @@ int launch_traverse(mdx_context *c, double kick = 0.0) {
         for (int k = slot; k < kTypes; ++k) c->kev_order[k] = -1;
     }
     if (c->timing) HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
-    const int R = c->nrep;
-    if (slot == 0)
-        hipLaunchKernelGGL(k_fill_double, dim3(1), dim3(64), 0, c->stream, c->red, 4 * R, 0.0);
-    else if (R == 1)
-        launch_reduce(c, c->macro_part, c->ncell, 4, c->red);
-    else
-        hipLaunchKernelGGL(k_seg_reduce, dim3(R), dim3(256), 0, c->stream, c->macro_part, 4,
-                           c->d_cell_off, c->red);
+    if (in_step) {
+        HIPCHK(c, hipGetLastError());
+        return MDX_OK;
+    }
     // point_lj: the pair kernel wrote F and Vi; M stays 0 (no site offsets)
     if (!c->point_lj)
         hipLaunchKernelGGL(k_calc_fm, dim3(nblk(c->n)), dim3(kBlock),
@@ -968,9 +988,7 @@ int launch_traverse(mdx_context *c, double kick = 0.0) {
                            c->mol[c->cur], c->d_comps, c->model.ncomp, c->sites[0],
                            c->sites[1], c->sites[2], c->sites[3], c->F, c->M, c->Vi, reps(c),
                            c->lrc ? c->d_thermo : nullptr);
-    hipLaunchKernelGGL(k_finalize_macro, dim3((R + 63) / 64), dim3(64), 0, c->stream, c->red,
-                       c->red + 4 * R, c->step_out, c->step_idx, R,
-                       c->lrc ? c->d_thermo : nullptr);
+    launch_step_end(c, kEndMacro);
     HIPCHK(c, hipGetLastError());
     return MDX_OK;
 }
@@ -981,28 +999,30 @@ bool open_domain(const mdx_context *c) {
     return c->g.outflow[0] | c->g.outflow[1] | c->g.outflow[2];
 }
 
-int launch_lf_pre(mdx_context *c, double dt) {
+// count: also bin the moved molecules (the next re-bin is launch_update with
+// counted set).
+int launch_lf_pre(mdx_context *c, double dt, bool count = false) {
     // reduced-memory mode: PositionCellProcessorRMM, r += dt v only
     hipLaunchKernelGGL(k_leapfrog_pre, dim3(nblk(c->n)), dim3(kBlock), 0, c->stream,
                        c->mol[c->cur], c->rmm_dt != 0.0 ? nullptr : c->F, c->M, c->d_comps,
-                       reps(c), dt, c->n);
+                       reps(c), dt, c->n, count ? bins(c) : Bins{});
     HIPCHK(c, hipGetLastError());
     return MDX_OK;
 }
 
-int launch_lf_post(mdx_context *c, double dt) {
-    const int R = c->nrep, nb = c->lf_nchunk;
-    hipLaunchKernelGGL(k_leapfrog_post, dim3(nb), dim3(kBlock), 0, c->stream, c->mol[c->cur], c->F,
-                       c->M, c->d_comps, dt, c->n, c->d_lf_chunk, c->d_lf_chunk_end, c->lf_part,
-                       c->rmm_dt != 0.0 ? 1 : 0, open_domain(c) ? 1 : 0);
-    if (R == 1)
-        launch_reduce(c, c->lf_part, nb, 4, c->red + 8);
-    else
-        hipLaunchKernelGGL(k_seg_reduce, dim3(R), dim3(256), 0, c->stream, c->lf_part, 4,
-                           c->d_lf_off, c->red + 8 * R);
-    hipLaunchKernelGGL(k_finalize_lf, dim3((R + 63) / 64), dim3(64), 0, c->stream, c->red + 8 * R,
-                       c->step_out, c->step_idx, R, c->thermostat ? c->d_thermo : nullptr,
-                       c->heuristics);
+// in_step: behind a traversal of the same step, whose site forces (multi-site
+// systems) are summed here and whose macroscopic values end the step with the
+// leapfrog's sums.
+int launch_lf_post(mdx_context *c, double dt, bool in_step = false) {
+    const bool sites = in_step && !c->point_lj;
+    const int nc = c->model.ncomp;
+    hipLaunchKernelGGL(sites ? k_leapfrog_post<true> : k_leapfrog_post<false>, dim3(c->lf_nchunk),
+                       dim3(kBlock), sites ? nc * sizeof(Component) : 0, c->stream, c->mol[c->cur],
+                       c->F, c->M, c->Vi, c->d_comps, nc, reps(c), dt, c->n, c->d_lf_chunk,
+                       c->d_lf_chunk_end, c->lf_part, c->rmm_dt != 0.0 ? 1 : 0,
+                       open_domain(c) ? 1 : 0, c->sites[0], c->sites[1], c->sites[2], c->sites[3],
+                       c->lrc ? c->d_thermo : nullptr);
+    launch_step_end(c, kEndLeapfrog | (in_step ? kEndMacro | kEndAdvance : 0));
     if (c->thermostat)
         hipLaunchKernelGGL(k_velocity_scale, dim3(nblk(c->n)), dim3(kBlock), 0, c->stream,
                            c->mol[c->cur], c->F, c->M, c->d_comps, reps(c), c->d_thermo, c->n);
@@ -1010,20 +1030,17 @@ int launch_lf_post(mdx_context *c, double dt) {
     return MDX_OK;
 }
 
-// Step n's second half kick and step n + 1's first half kick and drift in
-// one pass (no thermostat acts between them).
+// Step n's second half kick and step n + 1's first half kick, drift and binning
+// in one pass (no thermostat acts between them).
 int launch_lf_post_pre(mdx_context *c, double dt) {
-    const int R = c->nrep, nb = c->lf_nchunk;
-    hipLaunchKernelGGL(k_leapfrog_post_pre, dim3(nb), dim3(kBlock), 0, c->stream, c->mol[c->cur],
-                       c->F, c->M, c->d_comps, reps(c), dt, c->n, c->d_lf_chunk,
-                       c->d_lf_chunk_end, c->lf_part);
-    if (R == 1)
-        launch_reduce(c, c->lf_part, nb, 4, c->red + 8);
-    else
-        hipLaunchKernelGGL(k_seg_reduce, dim3(R), dim3(256), 0, c->stream, c->lf_part, 4,
-                           c->d_lf_off, c->red + 8 * R);
-    hipLaunchKernelGGL(k_finalize_lf, dim3((R + 63) / 64), dim3(64), 0, c->stream, c->red + 8 * R,
-                       c->step_out, c->step_idx, R, nullptr, c->heuristics);
+    const bool sites = !c->point_lj;
+    const int nc = c->model.ncomp;
+    hipLaunchKernelGGL(sites ? k_leapfrog_post_pre<true> : k_leapfrog_post_pre<false>,
+                       dim3(c->lf_nchunk), dim3(kBlock), sites ? nc * sizeof(Component) : 0,
+                       c->stream, c->mol[c->cur], c->F, c->M, c->d_comps, nc, reps(c), dt, c->n,
+                       c->d_lf_chunk, c->d_lf_chunk_end, c->lf_part, bins(c), c->sites[0],
+                       c->sites[1], c->sites[2], c->sites[3]);
+    launch_step_end(c, kEndMacro | kEndLeapfrog | kEndAdvance);
     HIPCHK(c, hipGetLastError());
     return MDX_OK;
 }
@@ -1034,19 +1051,11 @@ int launch_lf_post_pre(mdx_context *c, double dt) {
 enum { kStepFull = 0, kStepFused = 1, kStepLast = 2 };
 
 int launch_step(mdx_context *c, double dt, int kind = kStepFull) {
-    if (kind == kStepFull) TRY(launch_lf_pre(c, dt));
-    TRY(launch_update(c));
-    if (c->rmm_dt != 0.0)  // LeapfrogRMM: one full kick dt/m inside the force kernel
-        TRY(launch_traverse(c, dt / c->model.comp[0].m));
-    else
-        TRY(launch_traverse(c));
-    if (kind == kStepFused)
-        TRY(launch_lf_post_pre(c, dt));
-    else
-        TRY(launch_lf_post(c, dt));
-    hipLaunchKernelGGL(k_step_advance, dim3(1), dim3(1), 0, c->stream, c->step_idx);
-    HIPCHK(c, hipGetLastError());
-    return MDX_OK;
+    if (kind == kStepFull) TRY(launch_lf_pre(c, dt, true));
+    TRY(launch_update(c, true));
+    // LeapfrogRMM: one full kick dt/m inside the force kernel
+    TRY(launch_traverse(c, c->rmm_dt != 0.0 ? dt / c->model.comp[0].m : 0.0, true));
+    return kind == kStepFused ? launch_lf_post_pre(c, dt) : launch_lf_post(c, dt, true);
 }
 
 int need(mdx_context *c, bool model, bool domain, bool state) {
@@ -1206,15 +1215,13 @@ int mdx_create(int device, mdx_context **out) {
     }
     for (auto &e : c->ev) (void)hipEventCreate(&e);
     for (auto &e : c->kev) (void)hipEventCreate(&e);
-    if (dalloc(c, &c->red_tmp, 256 * 8) || dalloc(c, &c->d_counters, 8 * kTypes) ||
-        dalloc(c, &c->step_idx, 1) ||
+    if (dalloc(c, &c->d_counters, 8 * kTypes) ||
         dalloc(c, &c->d_comps, kMaxComp) || ensure_steps(c, 1)) {
         g_create_error = c->err;
         free_list(c->allocs);
         delete c;
         return MDX_ERR_HIP;
     }
-    (void)hipMemset(c->step_idx, 0, sizeof(int));
     (void)hipMemset(c->d_counters, 0, 8 * kTypes * sizeof(unsigned long long));
     if (device < kMaxDevices) {
         // once per device, with that device current
@@ -1488,7 +1495,7 @@ int mdx_autotune(mdx_context *c, int reps, int32_t *chosen, double *best_ms) {
         for (size_t i = 0; i < cand.size(); ++i) {
             c->cpb = cand[i].first;
             c->blocks_per_xcd = cand[i].second;
-            HIPCHK(c, hipMemsetAsync(c->step_idx, 0, sizeof(int), c->stream));
+            HIPCHK(c, hipMemsetAsync(c->step_idx, 0, sizeof(int) * c->nrep, c->stream));
             TRY(launch_traverse(c));
             HIPCHK(c, hipStreamSynchronize(c->stream));
             float ms = 0;
@@ -1762,14 +1769,14 @@ int mdx_traverse(mdx_context *c, double *macro) {
     if (c->counting)
         HIPCHK(c, hipMemsetAsync(c->d_counters, 0, 8 * kTypes * sizeof(unsigned long long),
                                  c->stream));
-    HIPCHK(c, hipMemsetAsync(c->step_idx, 0, sizeof(int), c->stream));
+    HIPCHK(c, hipMemsetAsync(c->step_idx, 0, sizeof(int) * c->nrep, c->stream));
     if (c->timing) HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
     // in the reduced-memory mode the traversal is VCP1CLJRMM's: force + kick
     TRY(launch_traverse(c, c->rmm_dt != 0.0 ? c->rmm_dt / c->model.comp[0].m : 0.0));
     if (c->timing) HIPCHK(c, hipEventRecord(c->ev[3], c->stream));
     if (macro) {
         TRY(0);
-        HIPCHK(c, hipMemcpyAsync(macro, c->red + 4 * c->nrep, 4 * sizeof(double) * c->nrep,
+        HIPCHK(c, hipMemcpyAsync(macro, c->red, 4 * sizeof(double) * c->nrep,
                                  hipMemcpyDeviceToHost, c->stream));
     }
     HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -1800,10 +1807,10 @@ int mdx_leapfrog_post(mdx_context *c, double dt, double *sums) {
     if (!c) return MDX_ERR_ARG;
     TRY(need(c, true, true, true));
     HIPCHK(c, hipSetDevice(c->device));
-    HIPCHK(c, hipMemsetAsync(c->step_idx, 0, sizeof(int), c->stream));
+    HIPCHK(c, hipMemsetAsync(c->step_idx, 0, sizeof(int) * c->nrep, c->stream));
     TRY(launch_lf_post(c, dt));
     if (sums) {
-        HIPCHK(c, hipMemcpyAsync(sums, c->red + 8 * c->nrep, 4 * sizeof(double) * c->nrep,
+        HIPCHK(c, hipMemcpyAsync(sums, c->red + 4 * c->nrep, 4 * sizeof(double) * c->nrep,
                                  hipMemcpyDeviceToHost, c->stream));
     }
     HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -1818,7 +1825,7 @@ int mdx_step(mdx_context *c, int nsteps, double dt, double *per_step, int use_gr
     HIPCHK(c, hipSetDevice(c->device));
     TRY(ensure_steps(c, nsteps));
     const int64_t q_renorm0 = c->q_renorm;
-    HIPCHK(c, hipMemsetAsync(c->step_idx, 0, sizeof(int), c->stream));
+    HIPCHK(c, hipMemsetAsync(c->step_idx, 0, sizeof(int) * c->nrep, c->stream));
     if (c->timing) HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
     // Consecutive steps without a thermostat between them share one pass
     // over the molecules for step n's second and step n + 1's first half
@@ -1828,7 +1835,11 @@ int mdx_step(mdx_context *c, int nsteps, double dt, double *per_step, int use_gr
         if (!fuse) return (int)kStepFull;
         return s < nsteps - 1 ? (int)kStepFused : (int)kStepLast;
     };
-    if (fuse) TRY(launch_lf_pre(c, dt));
+    // the steps bin their molecules while they move them, from empty bins (each
+    // re-bin leaves them so)
+    hipLaunchKernelGGL(k_fill_int, dim3(nblk(c->ncell + 2)), dim3(kBlock), 0, c->stream, c->count,
+                       c->ncell + 2, 0);
+    if (fuse) TRY(launch_lf_pre(c, dt, true));
     if (use_graph && !c->counting && !c->timing) {
         if (c->graph_dt != dt) drop_graphs(c);
         for (int s = 0; s < nsteps; ++s) {

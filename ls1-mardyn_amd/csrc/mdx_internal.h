@@ -81,18 +81,27 @@ struct SiteArrays {
 };
 
 // Up to kTypes independent exclusive scans of n ints each, array t on
-// blockIdx.y = t; aux: the block sums (k_scan_block) or their exclusive scan
-// (k_scan_add).
+// blockIdx.y = t, out[n] = the total; aux: the block sums (k_scan_block, and
+// k_scan_add with scanned = 0) or their exclusive scan (k_scan_add); clear: in
+// is set to 0 behind the scan.
 struct ScanArgs {
     const int *in[kTypes];
     int *out[kTypes];
     int *aux[kTypes];
     int n;
+    int scanned, clear;
 };
+constexpr int kScanOne = 16384;  // longest scan of one block (k_scan_one)
 
 struct MolArrays {
     double *rx, *ry, *rz, *vx, *vy, *vz, *qw, *qx, *qy, *qz, *Lx, *Ly, *Lz;
     int *cid, *orig;
+};
+
+// The counting sort's bins: each molecule's cell, its arrival rank there, its
+// ls1 cell id, and the cells' counts (0 before a binning).
+struct Bins {
+    int *cell, *rank, *count, *ls1id;
 };
 
 struct PairParams {
@@ -135,6 +144,25 @@ enum {
     kThTarget = 0, kThUcorr = 1, kThWcorr = 2, kThVi = 3,
     kThT = 4, kThBetaT = 5, kThBetaR = 6, kThExplode = 7, kThermoW = 8
 };
+
+// The sums of a step (k_step_end): the pair kernels' cell rows and the leapfrog
+// chunks' rows of each replica.
+struct StepEnd {
+    const double *macro_part;      // [ncell][4], or null: no sites, sums 0
+    const double *lf_part;         // [chunks][4]
+    const int *cell_off, *lf_off;  // [nrep + 1] rows of each replica
+    double *part;                  // [nrep][kStepBlocks][8] block sums
+    int *ticket;                   // [nrep] finished blocks, 0 between launches
+    double *macro, *sums;          // [nrep][4] macroscopic values, leapfrog sums
+    double *step_out;              // [step][nrep][6] records
+    int *step_idx;                 // [nrep] the replica's current step
+    const double *lrc;             // thermo records if the long-range correction acts
+    double *thermo;                // thermo records if the thermostat acts, else null
+    int nrep, heuristics;
+    int what;                      // kEndMacro | kEndLeapfrog | kEndAdvance
+};
+enum { kEndMacro = 1, kEndLeapfrog = 2, kEndAdvance = 4 };
+constexpr int kStepRows = 4096, kStepBlocks = 64;  // rows per block, most blocks per replica
 
 struct PairArgs {
     Reps R;

@@ -121,8 +121,8 @@ __device__ __forceinline__ double wave_sum(double v) {
 // Point molecules skip it: their invI and torque are 0, so L is unchanged and
 // q only re-normalised (which k_build_sites does every step, as ls1's
 // setupSoACache does).
-__device__ __forceinline__ void rotate_pre(MolArrays &s, const double *__restrict__ M,
-                                           const Component &c, double dt, int n, int i) {
+__device__ __forceinline__ void rotate_pre(MolArrays &s, const double M[3], const Component &c,
+                                           double dt, int i) {
 #pragma clang fp contract(off)
     const double dt_halve = .5 * dt;
     double q[4] = {s.qw[i], s.qx[i], s.qy[i], s.qz[i]};
@@ -134,7 +134,7 @@ __device__ __forceinline__ void rotate_pre(MolArrays &s, const double *__restric
     for (int k = 0; k < 4; ++k) qh[k] = qh[k] * dt_halve + q[k];
     double qc = 1. / sqrt(qh[0] * qh[0] + qh[1] * qh[1] + qh[2] * qh[2] + qh[3] * qh[3]);
     for (int k = 0; k < 4; ++k) qh[k] *= qc;
-    for (int d = 0; d < 3; ++d) L[d] += dt_halve * M[d * n + i];
+    for (int d = 0; d < 3; ++d) L[d] += dt_halve * M[d];
     qrotinv(qh, L, w);
     for (int d = 0; d < 3; ++d) w[d] *= c.invI[d];
     qdiff(qh, w, qi);
@@ -147,15 +147,15 @@ __device__ __forceinline__ void rotate_pre(MolArrays &s, const double *__restric
 
 // FullMolecule::upd_preF (FullMolecule.cpp:331-361), then the periodic wrap of
 // DomainDecompBase::handleDomainLeavingParticles (DomainDecompBase.cpp:199-249),
-// for molecule i with its velocity v and force f in registers (f null:
-// PositionCellProcessorRMM, r += dt v only). Writes r and v.
-__device__ __forceinline__ void lf_pre_mol(MolArrays &s, const double *__restrict__ M,
-                                           const Component &c, const Geom &g, double dt, int n,
-                                           int i, double v[3], const double *f) {
+// for molecule i with its velocity v, force f (null: PositionCellProcessorRMM,
+// r += dt v only) and torque M in registers. Writes r (also to r[]) and v.
+__device__ __forceinline__ void lf_pre_mol(MolArrays &s, const double M[3], const Component &c,
+                                           const Geom &g, double dt, int i, double v[3],
+                                           const double *f, double r[3]) {
 #pragma clang fp contract(off)
     const double dt_halve = .5 * dt;
     const double dtInv2m = dt_halve / c.m;
-    double r[3] = {s.rx[i], s.ry[i], s.rz[i]};
+    r[0] = s.rx[i], r[1] = s.ry[i], r[2] = s.rz[i];
     if (r[0] != r[0]) return;  // deleted at an outflow wall: no longer moved
     if (f && (g.reflect[0] | g.reflect[1] | g.reflect[2] | g.outflow[0] | g.outflow[1] |
               g.outflow[2])) {
@@ -191,7 +191,7 @@ __device__ __forceinline__ void lf_pre_mol(MolArrays &s, const double *__restric
             }
         }
         if (dead) {
-            s.rx[i] = s.ry[i] = s.rz[i] = __builtin_nan("");
+            r[0] = s.rx[i] = s.ry[i] = s.rz[i] = __builtin_nan("");
             return;
         }
     }
@@ -199,7 +199,7 @@ __device__ __forceinline__ void lf_pre_mol(MolArrays &s, const double *__restric
         if (f) v[d] += dtInv2m * f[d];
         r[d] += dt * v[d];
     }
-    if (!c.point) rotate_pre(s, M, c, dt, n, i);
+    if (!c.point) rotate_pre(s, M, c, dt, i);
     for (int d = 0; d < 3; ++d) {
         if (!g.pdim[d]) continue;
         double x = r[d];
@@ -216,24 +216,76 @@ __device__ __forceinline__ void lf_pre_mol(MolArrays &s, const double *__restric
     s.vx[i] = v[0]; s.vy[i] = v[1]; s.vz[i] = v[2];
 }
 
+// Cell of molecule i at p (ls1 index -> inner index) and its arrival rank in
+// the cell, for every lane of the wave (in: the lane has a molecule; the lanes
+// that have one come first). Molecules are stored in cell order, so a wave's
+// lanes form a few runs of equal cells: the first lane of each run takes one
+// atomic for the whole run, and all runs' atomics go out in the same
+// instruction (one round trip per wave; a cell that shows up in two runs gets
+// two disjoint rank ranges).
+__device__ __forceinline__ void bin_mol(const double p[3], const Reps &R, int i, bool in,
+                                        const Bins &b) {
+    const int lane = threadIdx.x & 63;
+    int c = -1;
+    if (in) {
+        if (p[0] != p[0] && R.nrep == 1) {
+            // deleted at an outflow wall: the bin behind the last cell, which
+            // no traversal visits
+            c = R.cell_off[1];
+            b.ls1id[i] = -1;
+        } else {
+            const int rep = mol_replica(R, i);
+            const Geom &g = R.geom[rep];
+            int ci[3];
+            ls1_cell3(g, p, ci);
+            c = R.cell_off[rep] + inner_index(g, ci);
+            b.ls1id[i] = (ci[2] * g.cpd[1] + ci[1]) * g.cpd[0] + ci[0];
+        }
+        b.cell[i] = c;
+    }
+    const int cprev = __shfl_up(c, 1, 64);
+    const bool head = in && (lane == 0 || cprev != c);
+    const unsigned long long heads = __ballot(head);
+    const unsigned long long valid = __ballot(in);
+    // my run's head: the highest head at or below my lane
+    const unsigned long long upto = (2ull << lane) - 1ull;  // lanes 0..lane (all for 63)
+    const unsigned long long below = heads & upto;
+    const int h = in ? 63 - __clzll((long long)below) : 0;
+    int base = 0;
+    if (head) {
+        // the run ends at the next head or at the last valid lane
+        const unsigned long long after = heads & ~upto;
+        const int end = after ? __ffsll((long long)after) - 1 : 64 - __clzll((long long)valid);
+        base = atomicAdd(&b.count[c], end - lane);
+    }
+    base = __shfl(base, h, 64);
+    if (in) b.rank[i] = base + (lane - h);
+}
+
+// bins.count non-null: the moved molecules are also binned (the next re-bin's
+// k_bin_count, with r in registers).
 __global__ __launch_bounds__(256) void k_leapfrog_pre(MolArrays s, const double *__restrict__ F,
                                                       const double *__restrict__ M,
                                                       const Component *__restrict__ comps, Reps R,
-                                                      double dt, int n) {
+                                                      double dt, int n, Bins bins) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    double v[3] = {s.vx[i], s.vy[i], s.vz[i]};
-    double f[3] = {0., 0., 0.};
-    if (F) f[0] = F[i], f[1] = F[n + i], f[2] = F[2 * n + i];
-    lf_pre_mol(s, M, comps[s.cid[i]], R.geom[mol_replica(R, i)], dt, n, i, v, F ? f : nullptr);
+    double r[3] = {0., 0., 0.};
+    if (i < n) {
+        double v[3] = {s.vx[i], s.vy[i], s.vz[i]};
+        double f[3] = {0., 0., 0.}, m[3] = {0., 0., 0.};
+        const Component &c = comps[s.cid[i]];
+        if (F) f[0] = F[i], f[1] = F[n + i], f[2] = F[2 * n + i];
+        if (!c.point) m[0] = M[i], m[1] = M[n + i], m[2] = M[2 * n + i];
+        lf_pre_mol(s, m, c, R.geom[mol_replica(R, i)], dt, i, v, F ? f : nullptr, r);
+    }
+    if (bins.count) bin_mol(r, R, i, i < n, bins);
 }
 
 // FullMolecule::upd_postF (FullMolecule.cpp:363-387) for molecule i: v (in
 // registers) and L advanced, {m v^2, I w^2} added to the sums.
-__device__ __forceinline__ void lf_post_mol(MolArrays &s, const double *__restrict__ M,
-                                            const Component &c, double dt, int n, int i,
-                                            double v[3], const double f[3], double &mv2,
-                                            double &iw2) {
+__device__ __forceinline__ void lf_post_mol(MolArrays &s, const double M[3], const Component &c,
+                                            double dt, int i, double v[3], const double f[3],
+                                            double &mv2, double &iw2) {
 #pragma clang fp contract(off)
     const double dt_halve = 0.5 * dt;
     const double dtInv2m = dt_halve / c.m;
@@ -245,7 +297,7 @@ __device__ __forceinline__ void lf_post_mol(MolArrays &s, const double *__restri
     mv2 = c.m * v2;
     if (!c.point) {  // point molecules: L unchanged, I w^2 = 0
         double L[3] = {s.Lx[i], s.Ly[i], s.Lz[i]};
-        for (int d = 0; d < 3; ++d) L[d] += dt_halve * M[d * n + i];
+        for (int d = 0; d < 3; ++d) L[d] += dt_halve * M[d];
         double q[4] = {s.qw[i], s.qx[i], s.qy[i], s.qz[i]};
         double w[3];
         qrotinv(q, L, w);
@@ -275,66 +327,6 @@ __device__ __forceinline__ void lf_block_sums(double mv2, double iw2, double cnt
         for (int k = 0; k < (int)(blockDim.x >> 6); ++k) a += red[k][threadIdx.x];
         partial[blockIdx.x * 4 + threadIdx.x] = a;
     }
-}
-
-// The second half kick of every molecule with the step's sums. Block b
-// covers molecules [chunk[b], chunk[b] + 256) clipped to chunk_end[b]: chunks
-// never straddle two replicas.
-__global__ __launch_bounds__(256) void k_leapfrog_post(MolArrays s, const double *__restrict__ F,
-                                                       const double *__restrict__ M,
-                                                       const Component *__restrict__ comps,
-                                                       double dt, int n,
-                                                       const int *__restrict__ chunk,
-                                                       const int *__restrict__ chunk_end,
-                                                       double *partial, int rmm, int open) {
-    int i = chunk[blockIdx.x] + threadIdx.x;
-    double mv2 = 0, iw2 = 0, cnt = 0, rot = 0;
-    const bool deleted = open && i < chunk_end[blockIdx.x] && s.rx[i] != s.rx[i];
-    if (deleted) {
-        // deleted at an outflow wall: not moved, not counted
-    } else if (rmm && i < chunk_end[blockIdx.x]) {
-        // VelocityCellProcessorRMM (VelocityCellProcessorRMM.h:60-110): the
-        // kick happened in the force kernel; sum v^2 (no mass factor, as the
-        // reference's reduced-memory mode sums it) and N, no rotation
-        const double v[3] = {s.vx[i], s.vy[i], s.vz[i]};
-        mv2 = v[0] * v[0] + v[1] * v[1] + v[2] * v[2];
-        cnt = 1.0;
-    } else if (i < chunk_end[blockIdx.x]) {
-        const Component &c = comps[s.cid[i]];
-        double v[3] = {s.vx[i], s.vy[i], s.vz[i]};
-        const double f[3] = {F[i], F[n + i], F[2 * n + i]};
-        lf_post_mol(s, M, c, dt, n, i, v, f, mv2, iw2);
-        cnt = 1.0;
-        rot = c.rotdof;
-        s.vx[i] = v[0]; s.vy[i] = v[1]; s.vz[i] = v[2];
-    }
-    lf_block_sums(mv2, iw2, cnt, rot, partial);
-}
-
-// Step n's second half kick (with its sums) fused with step n + 1's first
-// half kick and drift, for consecutive steps without a thermostat between
-// them: the same operations in the same order as k_leapfrog_post followed by
-// k_leapfrog_pre, with v and F read once.
-__global__ __launch_bounds__(256) void k_leapfrog_post_pre(MolArrays s,
-                                                           const double *__restrict__ F,
-                                                           const double *__restrict__ M,
-                                                           const Component *__restrict__ comps,
-                                                           Reps R, double dt, int n,
-                                                           const int *__restrict__ chunk,
-                                                           const int *__restrict__ chunk_end,
-                                                           double *partial) {
-    int i = chunk[blockIdx.x] + threadIdx.x;
-    double mv2 = 0, iw2 = 0, cnt = 0, rot = 0;
-    if (i < chunk_end[blockIdx.x]) {
-        const Component &c = comps[s.cid[i]];
-        double v[3] = {s.vx[i], s.vy[i], s.vz[i]};
-        const double f[3] = {F[i], F[n + i], F[2 * n + i]};
-        lf_post_mol(s, M, c, dt, n, i, v, f, mv2, iw2);
-        cnt = 1.0;
-        rot = c.rotdof;
-        lf_pre_mol(s, M, c, R.geom[mol_replica(R, i)], dt, n, i, v, f);
-    }
-    lf_block_sums(mv2, iw2, cnt, rot, partial);
 }
 
 // Fixed-order reduction of per-block partials (width values per block):
@@ -368,57 +360,12 @@ __global__ void k_fill_int(int *a, int n, int v) {
     if (i < n) a[i] = v;
 }
 
-__global__ void k_fill_double(double *a, int n, double v) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) a[i] = v;
-}
-
-// Cell of every molecule (ls1 index -> inner index) and its arrival rank in
-// the cell. Molecules are stored in cell order, so a wave's lanes form a few
-// runs of equal cells: the first lane of each run takes one atomic for the
-// whole run, and all runs' atomics go out in the same instruction (one
-// round trip per wave; a cell that shows up in two runs gets two disjoint
-// rank ranges).
-__global__ __launch_bounds__(256) void k_bin_count(MolArrays s, Reps R, int n, int *cell,
-                                                   int *rank, int *count, int *ls1id) {
+__global__ __launch_bounds__(256) void k_bin_count(MolArrays s, Reps R, int n, Bins b) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int lane = threadIdx.x & 63;
     const bool in = i < n;
-    int c = -1;
-    if (in) {
-        double p[3] = {s.rx[i], s.ry[i], s.rz[i]};
-        if (p[0] != p[0] && R.nrep == 1) {
-            // deleted at an outflow wall: the bin behind the last cell, which
-            // no traversal visits
-            c = R.cell_off[1];
-            ls1id[i] = -1;
-        } else {
-            const int rep = mol_replica(R, i);
-            const Geom &g = R.geom[rep];
-            int ci[3];
-            ls1_cell3(g, p, ci);
-            c = R.cell_off[rep] + inner_index(g, ci);
-            ls1id[i] = (ci[2] * g.cpd[1] + ci[1]) * g.cpd[0] + ci[0];
-        }
-        cell[i] = c;
-    }
-    const int cprev = __shfl_up(c, 1, 64);
-    const bool head = in && (lane == 0 || cprev != c);
-    const unsigned long long heads = __ballot(head);
-    const unsigned long long valid = __ballot(in);
-    // my run's head: the highest head at or below my lane
-    const unsigned long long upto = (2ull << lane) - 1ull;  // lanes 0..lane (all for 63)
-    const unsigned long long below = heads & upto;
-    const int h = in ? 63 - __clzll((long long)below) : 0;
-    int base = 0;
-    if (head) {
-        // the run ends at the next head or at the last valid lane
-        const unsigned long long after = heads & ~upto;
-        const int end = after ? __ffsll((long long)after) - 1 : 64 - __clzll((long long)valid);
-        base = atomicAdd(&count[c], end - lane);
-    }
-    base = __shfl(base, h, 64);
-    if (in) rank[i] = base + (lane - h);
+    double p[3] = {0., 0., 0.};
+    if (in) p[0] = s.rx[i], p[1] = s.ry[i], p[2] = s.rz[i];
+    bin_mol(p, R, i, in, b);
 }
 
 __global__ __launch_bounds__(256) void k_bin_scatter(int n, const int *__restrict__ cell,
@@ -565,10 +512,54 @@ __global__ __launch_bounds__(256) void k_normalize_q(int n, MolArrays s, long lo
 
 // ------------------------------------------------------------- scan (int)
 
+// Inclusive scan over the wave.
+__device__ __forceinline__ int wave_incl(int x, int lane) {
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(x, o, 64);
+        if (lane >= o) x += y;
+    }
+    return x;
+}
+
+// Exclusive scan of up to kScanOne ints by one block of 1024 threads: four
+// tiles of 4096, all loaded at once, the 64 wave sums (tile-major) scanned by
+// every wave for itself. One launch of 4.7 us where block scan, scan of the block
+// sums, addition and total were four of about 4 us each (2744 cells).
+__global__ __launch_bounds__(1024) void k_scan_one(ScanArgs a) {
+    __shared__ int ws[64];
+    const int *in = a.in[blockIdx.y];
+    int *out = a.out[blockIdx.y];
+    const int n = a.n, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    int v[4][4], incl[4];
+    for (int t = 0; t < 4; ++t) {
+        const int base = t * 4096 + threadIdx.x * 4;
+        for (int k = 0; k < 4; ++k) v[t][k] = base + k < n ? in[base + k] : 0;
+    }
+    for (int t = 0; t < 4; ++t) {
+        incl[t] = wave_incl(v[t][0] + v[t][1] + v[t][2] + v[t][3], lane);
+        if (lane == 63) ws[t * 16 + wv] = incl[t];
+    }
+    __syncthreads();
+    const int w = ws[lane], wi = wave_incl(w, lane);
+    for (int t = 0; t < 4; ++t) {
+        const int base = t * 4096 + threadIdx.x * 4;
+        const int woff = __shfl(wi - w, t * 16 + wv, 64);
+        int excl = woff + incl[t] - (v[t][0] + v[t][1] + v[t][2] + v[t][3]);
+        for (int k = 0; k < 4; ++k) {
+            if (base + k < n) {
+                out[base + k] = excl;
+                if (a.clear) const_cast<int *>(in)[base + k] = 0;
+            }
+            excl += v[t][k];
+        }
+    }
+    if (threadIdx.x == 63) out[n] = wi;
+}
+
 // Exclusive scan of blocks of 1024 ints (256 threads x 4); block totals out.
 __global__ __launch_bounds__(256) void k_scan_block(ScanArgs a) {
     __shared__ int ws[4];
-    const int *__restrict__ in = a.in[blockIdx.y];
+    const int *in = a.in[blockIdx.y];
     int *out = a.out[blockIdx.y];
     const int n = a.n;
     int base = blockIdx.x * 1024 + threadIdx.x * 4;
@@ -579,48 +570,48 @@ __global__ __launch_bounds__(256) void k_scan_block(ScanArgs a) {
     }
     // inclusive scan of t across the block
     int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    int x = t;
-    for (int o = 1; o < 64; o <<= 1) {
-        int y = __shfl_up(x, o, 64);
-        if (lane >= o) x += y;
-    }
+    const int x = wave_incl(t, lane);
     if (lane == 63) ws[wv] = x;
     __syncthreads();
     int woff = 0;
     for (int k = 0; k < wv; ++k) woff += ws[k];
     int excl = woff + x - t;
     for (int k = 0; k < 4; ++k) {
-        if (base + k < n) out[base + k] = excl;
+        if (base + k < n) {
+            out[base + k] = excl;
+            if (a.clear) const_cast<int *>(in)[base + k] = 0;
+        }
         excl += v[k];
     }
     if (threadIdx.x == 255) a.aux[blockIdx.y][blockIdx.x] = woff + x;
 }
 
+// Adds what the blocks before sum to: aux holds their scan (scanned), or their
+// sums, which the block then adds up itself (a few thousand at most: cheaper
+// than a launch of their own). The last block writes the total.
 __global__ __launch_bounds__(256) void k_scan_add(ScanArgs a) {
+    __shared__ int ws[4];
+    const int *aux = a.aux[blockIdx.y];
     int *out = a.out[blockIdx.y];
-    const int n = a.n;
-    int i = blockIdx.x * 1024 + threadIdx.x;
-    int off = a.aux[blockIdx.y][blockIdx.x];
+    const int n = a.n, nb = gridDim.x, b = blockIdx.x;
+    int off = 0, own = 0;
+    if (a.scanned) {
+        off = aux[b];
+        own = aux[b + 1] - off;
+    } else {
+        for (int k = threadIdx.x; k < b; k += 256) off += aux[k];
+        off = wave_incl(off, threadIdx.x & 63);
+        if ((threadIdx.x & 63) == 63) ws[threadIdx.x >> 6] = off;
+        __syncthreads();
+        off = ws[0] + ws[1] + ws[2] + ws[3];
+        own = aux[b];
+    }
+    int i = b * 1024 + threadIdx.x;
     for (int k = 0; k < 4; ++k) {
         int j = i + k * 256;
         if (j < n) out[j] += off;
     }
-}
-
-// out[n] = the total of array blockIdx.y (out holds n + 1 ints).
-__global__ void k_scan_total(ScanArgs a) {
-    const int *in = a.in[blockIdx.y];
-    int *out = a.out[blockIdx.y];
-    const int n = a.n;
-    if (threadIdx.x == 0 && blockIdx.x == 0) out[n] = (n > 0) ? out[n - 1] + in[n - 1] : 0;
-}
-
-// For array t = blockIdx.y: cstart_t[c] = mstart_t[start[c]] for c in
-// [0, ncell] (start[ncell] = n), with mstart_t = a.in[t], cstart_t = a.out[t].
-__global__ void k_cell_site_start(int ncell, const int *__restrict__ start, ScanArgs a) {
-    int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c > ncell) return;
-    a.out[blockIdx.y][c] = a.in[blockIdx.y][start[c]];
+    if (b == nb - 1 && threadIdx.x == 0) out[n] = off + own;
 }
 
 // --------------------------------------------------- SoA site cache build
@@ -647,17 +638,29 @@ __device__ __forceinline__ const Component *stage_comps(const Component *__restr
 // forms: bit 0 the FP64 site records (positions, molecule positions,
 // orientations, parameters) the FP64 pair kernels and the adjoint read, bit 1
 // the FP32 ones of the FP32-pair form. first: the re-bin's build, which also
-// normalises q and writes what both forms read (molecule index of each site,
-// LJ ids, charge head counts); a later call with first = 0 adds a form the
+// normalises q and writes what both forms read (per-cell site starts, molecule
+// index of each site, LJ ids, charge head counts); a later call with first = 0 adds a form the
 // re-bin did not build, from the same (normalised) q.
 __global__ __launch_bounds__(256) void k_build_sites(int n, MolArrays s, Reps R,
                                                      const int *__restrict__ mcell,
                                                      const Component *__restrict__ gcomps,
                                                      int ncomp, int forms, int first,
+                                                     int ncell, const int *__restrict__ start,
                                                      SiteArrays s0, SiteArrays s1,
                                                      SiteArrays s2, SiteArrays s3) {
     const Component *comps = stage_comps(gcomps, ncomp);
     int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (first) {
+        // cstart[c] = mstart[start[c]] for c in [0, ncell] (start[ncell]: the
+        // live count), for the types that are present
+        for (int c = i; c <= ncell; c += gridDim.x * blockDim.x) {
+            const int m = start[c];
+            if (s0.Fx) s0.cstart[c] = s0.mstart[m];
+            if (s1.Fx) s1.cstart[c] = s1.mstart[m];
+            if (s2.Fx) s2.cstart[c] = s2.mstart[m];
+            if (s3.Fx) s3.cstart[c] = s3.mstart[m];
+        }
+    }
     if (i >= n) return;
     double q[4] = {s.qw[i], s.qx[i], s.qy[i], s.qz[i]};
     if (first) {
@@ -715,25 +718,21 @@ __global__ __launch_bounds__(256) void k_build_sites(int n, MolArrays s, Reps R,
 }
 
 // FullMolecule::calcFM (FullMolecule.cpp:548-631): F = sum F_site,
-// M = sum d_site x F_site + sum M_site(D, Q), Vi = 0.5 sum V_site.
-__global__ __launch_bounds__(256) void k_calc_fm(int n, MolArrays s,
-                                                 const Component *__restrict__ gcomps,
-                                                 int ncomp, SiteArrays s0, SiteArrays s1,
-                                                 SiteArrays s2, SiteArrays s3, double *F,
-                                                 double *M, double *Vi, Reps R,
-                                                 const double *__restrict__ thermo) {
-    const Component *comps = stage_comps(gcomps, ncomp);
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const Component &c = comps[s.cid[i]];
+// M = sum d_site x F_site + sum M_site(D, Q), Vi = 0.5 sum V_site (tv: the sum),
+// of molecule i.
+__device__ __forceinline__ void calc_fm_mol(const MolArrays &s, const Component &c,
+                                            const SiteArrays &s0, const SiteArrays &s1,
+                                            const SiteArrays &s2, const SiteArrays &s3, int i,
+                                            bool virial, double f[3], double M[3], double tv[3]) {
     // point molecules: every site offset is 0, so no d x F term needs q
     double q[4] = {1, 0, 0, 0};
     if (!c.point) q[0] = s.qw[i], q[1] = s.qx[i], q[2] = s.qy[i], q[3] = s.qz[i];
-    double f[3] = {0, 0, 0}, m[3] = {0, 0, 0}, tm[3] = {0, 0, 0}, tv[3] = {0, 0, 0};
-    SiteArrays *S[4] = {&s0, &s1, &s2, &s3};
+    double m[3] = {0, 0, 0}, tm[3] = {0, 0, 0};
+    for (int d = 0; d < 3; ++d) f[d] = tv[d] = 0;
+    const SiteArrays *S[4] = {&s0, &s1, &s2, &s3};
 #pragma unroll
     for (int t = 0; t < kTypes; ++t) {
-        SiteArrays &A = *S[t];
+        const SiteArrays &A = *S[t];
         int base = A.mstart[i];
         for (int k = 0; k < c.n[t]; ++k) {
             int j = base + k;
@@ -744,21 +743,135 @@ __global__ __launch_bounds__(256) void k_calc_fm(int n, MolArrays s,
             m[0] += d[1] * fs[2] - d[2] * fs[1];
             m[1] += d[2] * fs[0] - d[0] * fs[2];
             m[2] += d[0] * fs[1] - d[1] * fs[0];
-            tv[0] += A.Vx[j]; tv[1] += A.Vy[j]; tv[2] += A.Vz[j];
+            if (virial) tv[0] += A.Vx[j], tv[1] += A.Vy[j], tv[2] += A.Vz[j];
             if (t >= T_D) {
                 tm[0] += A.Mx[j]; tm[1] += A.My[j]; tm[2] += A.Mz[j];
             }
         }
     }
+    for (int d = 0; d < 3; ++d) M[d] = m[d] + tm[d];
+}
+
+// Molecule i's F, M and Vi into the arrays.
+__device__ __forceinline__ void put_fm(const double f[3], const double M[3], const double tv[3],
+                                       const Reps &R, const double *__restrict__ lrc, int n, int i,
+                                       double *F, double *Mo, double *Vi) {
     for (int d = 0; d < 3; ++d) {
         F[d * n + i] = f[d];
-        M[d * n + i] = m[d] + tm[d];
+        Mo[d * n + i] = M[d];
         // Homogeneous::calculateLongRange adds VirialCorr / (3N) to every
         // molecule before calcFM adds its sites (Homogeneous.cpp:139-145)
         Vi[d * n + i] =
-            thermo ? __dadd_rn(__dmul_rn(0.5, tv[d]), thermo[kThermoW * mol_replica(R, i) + kThVi])
-                   : 0.5 * tv[d];
+            lrc ? __dadd_rn(__dmul_rn(0.5, tv[d]), lrc[kThermoW * mol_replica(R, i) + kThVi])
+                : 0.5 * tv[d];
     }
+}
+
+__global__ __launch_bounds__(256) void k_calc_fm(int n, MolArrays s,
+                                                 const Component *__restrict__ gcomps,
+                                                 int ncomp, SiteArrays s0, SiteArrays s1,
+                                                 SiteArrays s2, SiteArrays s3, double *F,
+                                                 double *M, double *Vi, Reps R,
+                                                 const double *__restrict__ lrc) {
+    const Component *comps = stage_comps(gcomps, ncomp);
+    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    double f[3], m[3], tv[3];
+    calc_fm_mol(s, comps[s.cid[i]], s0, s1, s2, s3, i, true, f, m, tv);
+    put_fm(f, m, tv, R, lrc, n, i, F, M, Vi);
+}
+
+// The second half kick of every molecule with the step's sums. Block b
+// covers molecules [chunk[b], chunk[b] + 256) clipped to chunk_end[b]: chunks
+// never straddle two replicas. sites: F, M and Vi are first summed from the
+// site arrays and stored (k_calc_fm), with no pass of its own.
+template <bool SITES>
+__global__ __launch_bounds__(256) void k_leapfrog_post(MolArrays s, double *F, double *M,
+                                                       double *Vi,
+                                                       const Component *__restrict__ gcomps,
+                                                       int ncomp, Reps R, double dt, int n,
+                                                       const int *__restrict__ chunk,
+                                                       const int *__restrict__ chunk_end,
+                                                       double *partial, int rmm, int open,
+                                                       SiteArrays s0, SiteArrays s1,
+                                                       SiteArrays s2, SiteArrays s3,
+                                                       const double *__restrict__ lrc) {
+    const Component *comps = gcomps;
+    if constexpr (SITES) comps = stage_comps(gcomps, ncomp);
+    int i = chunk[blockIdx.x] + threadIdx.x;
+    const bool in = i < chunk_end[blockIdx.x];
+    double mv2 = 0, iw2 = 0, cnt = 0, rot = 0;
+    double f[3] = {0., 0., 0.}, m[3] = {0., 0., 0.};
+    if constexpr (SITES) {
+        if (in) {
+            double tv[3];
+            calc_fm_mol(s, comps[s.cid[i]], s0, s1, s2, s3, i, true, f, m, tv);
+            put_fm(f, m, tv, R, lrc, n, i, F, M, Vi);
+        }
+    }
+    const bool deleted = open && in && s.rx[i] != s.rx[i];
+    if (deleted) {
+        // deleted at an outflow wall: not moved, not counted
+    } else if (rmm && in) {
+        // VelocityCellProcessorRMM (VelocityCellProcessorRMM.h:60-110): the
+        // kick happened in the force kernel; sum v^2 (no mass factor, as the
+        // reference's reduced-memory mode sums it) and N, no rotation
+        const double v[3] = {s.vx[i], s.vy[i], s.vz[i]};
+        mv2 = v[0] * v[0] + v[1] * v[1] + v[2] * v[2];
+        cnt = 1.0;
+    } else if (in) {
+        const Component &c = comps[s.cid[i]];
+        double v[3] = {s.vx[i], s.vy[i], s.vz[i]};
+        if constexpr (!SITES) {
+            f[0] = F[i], f[1] = F[n + i], f[2] = F[2 * n + i];
+            if (!c.point) m[0] = M[i], m[1] = M[n + i], m[2] = M[2 * n + i];
+        }
+        lf_post_mol(s, m, c, dt, i, v, f, mv2, iw2);
+        cnt = 1.0;
+        rot = c.rotdof;
+        s.vx[i] = v[0]; s.vy[i] = v[1]; s.vz[i] = v[2];
+    }
+    lf_block_sums(mv2, iw2, cnt, rot, partial);
+}
+
+// Step n's second half kick (with its sums) fused with step n + 1's first
+// half kick, drift and binning, for consecutive steps without a thermostat
+// between them: the same operations in the same order as k_leapfrog_post
+// followed by k_leapfrog_pre, with v and F read once. SITES: F and M come from
+// the site arrays and stay in registers (nothing reads such a step's F, M and
+// Vi). Bound by memory: 1 M molecules of the 2CLJQ + water mixture, calc_fm 76 +
+// this 68 + binning 19 us before, 110 with the sites' virials and the molecules'
+// F, M and Vi neither read nor written; 1 M one-centre molecules 30 + 20 -> 46.
+template <bool SITES>
+__global__ __launch_bounds__(256) void k_leapfrog_post_pre(
+    MolArrays s, const double *__restrict__ F, const double *__restrict__ M,
+    const Component *__restrict__ gcomps, int ncomp, Reps R, double dt, int n,
+    const int *__restrict__ chunk, const int *__restrict__ chunk_end, double *partial, Bins bins,
+    SiteArrays s0, SiteArrays s1, SiteArrays s2, SiteArrays s3) {
+    const Component *comps = gcomps;
+    if constexpr (SITES) comps = stage_comps(gcomps, ncomp);
+    int i = chunk[blockIdx.x] + threadIdx.x;
+    const bool in = i < chunk_end[blockIdx.x];
+    double mv2 = 0, iw2 = 0, cnt = 0, rot = 0;
+    double r[3] = {0., 0., 0.};
+    if (in) {
+        const Component &c = comps[s.cid[i]];
+        double v[3] = {s.vx[i], s.vy[i], s.vz[i]};
+        double f[3], m[3] = {0., 0., 0.};
+        if constexpr (SITES) {
+            double tv[3];
+            calc_fm_mol(s, c, s0, s1, s2, s3, i, false, f, m, tv);
+        } else {
+            f[0] = F[i], f[1] = F[n + i], f[2] = F[2 * n + i];
+            if (!c.point) m[0] = M[i], m[1] = M[n + i], m[2] = M[2 * n + i];
+        }
+        lf_post_mol(s, m, c, dt, i, v, f, mv2, iw2);
+        cnt = 1.0;
+        rot = c.rotdof;
+        lf_pre_mol(s, m, c, R.geom[mol_replica(R, i)], dt, i, v, f, r);
+    }
+    bin_mol(r, R, i, in, bins);
+    lf_block_sums(mv2, iw2, cnt, rot, partial);
 }
 
 // Macroscopic sums of one traversal (VectorizedCellProcessor::endTraversal,
@@ -766,47 +879,35 @@ __global__ __launch_bounds__(256) void k_calc_fm(int n, MolArrays s,
 // sides of every pair {u6, uXpoles, virial, rf}; halved here. myRF carries
 // the reference's negative sign (VectorizedCellProcessor.cpp:2727).
 // Step record: Upot, virial, summv2, sumIw2, Upot_LJ, Upot_rest.
-// One thread per replica; raw, macro are [nrep][4], the step record is
-// [step][nrep][6].
-__global__ void k_finalize_macro(const double *raw, double *macro, double *step_out,
-                                 const int *step_idx, int nrep,
-                                 const double *__restrict__ thermo) {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nrep) return;
-    raw += 4 * r;
-    macro += 4 * r;
+__device__ __forceinline__ void finalize_macro(const double raw[4], double *macro, double *rec,
+                                               const double *thermo) {
     double u6 = 0.5 * raw[0], ux = 0.5 * raw[1], vir = 0.5 * raw[2], rf = -0.5 * raw[3];
     macro[0] = u6;
     macro[1] = ux;
     macro[2] = vir;
     macro[3] = rf;
-    double *rec = step_out + 6 * ((size_t)step_idx[0] * nrep + r);
     rec[0] = u6 / 6.0 + ux + rf;
     rec[1] = vir + 3.0 * rf;
     if (thermo) {  // Domain::calculateGlobalValues (Domain.cpp:187-188)
-        rec[0] = rec[0] + thermo[kThermoW * r + kThUcorr];
-        rec[1] = rec[1] + thermo[kThermoW * r + kThWcorr];
+        rec[0] = rec[0] + thermo[kThUcorr];
+        rec[1] = rec[1] + thermo[kThWcorr];
     }
     rec[4] = u6 / 6.0;
     rec[5] = ux + rf;
 }
 
-__global__ void k_finalize_lf(const double *sums, double *step_out, const int *step_idx,
-                              int nrep, double *thermo, int heuristics) {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nrep) return;
-    double *rec = step_out + 6 * ((size_t)step_idx[0] * nrep + r);
-    rec[2] = sums[4 * r];
-    rec[3] = sums[4 * r + 1];
-    if (!thermo) return;
+__device__ __forceinline__ void finalize_lf(const double sums[4], double *rec, double *th,
+                                            int heuristics) {
+    rec[2] = sums[0];
+    rec[3] = sums[1];
+    if (!th) return;
     // Domain::calculateGlobalValues, global thermostat, Tfactor 1
     // (Domain.cpp:219-313): temperature and scaling factors; the explosion
     // heuristic replaces them when one is below MIN_BETA = 0.9 (its error
     // counter never rises above 0 in the reference, so it stays armed)
-    double *th = thermo + kThermoW * r;
     const double Ti = th[kThTarget];
-    const double summv2 = sums[4 * r], N = sums[4 * r + 2], rot = sums[4 * r + 3];
-    const double sumIw2 = rot > 0 ? sums[4 * r + 1] : 0.0;
+    const double summv2 = sums[0], N = sums[2], rot = sums[3];
+    const double sumIw2 = rot > 0 ? sums[1] : 0.0;
     th[kThT] = N > 0 ? (summv2 + sumIw2) / (3 * N + rot) : Ti;
     double bt = 1.0, br = 1.0;
     if (Ti > 0.0 && N > 0) {
@@ -883,29 +984,101 @@ __global__ __launch_bounds__(256) void k_velocity_scale(MolArrays s, double *F, 
     }
 }
 
-// Segmented fixed-order sum: block r adds rows [off[r], off[r+1]) of a
-// [rows][width] array into out[r][width] (one block per replica).
-__global__ __launch_bounds__(256) void k_seg_reduce(const double *__restrict__ in, int width,
-                                                    const int *__restrict__ off, double *out) {
-    __shared__ double red[256];
-    const int b0 = off[blockIdx.x], b1 = off[blockIdx.x + 1];
-    for (int w = 0; w < width; ++w) {
-        double a = 0;
-        for (int b = b0 + threadIdx.x; b < b1; b += blockDim.x) a += in[(size_t)b * width + w];
-        red[threadIdx.x] = a;
-        __syncthreads();
-        for (int o = blockDim.x / 2; o > 0; o >>= 1) {
-            if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-            __syncthreads();
+// What a step ends with, in one launch: per replica the fixed-order sums of the
+// pair kernels' cell rows and of the leapfrog chunks' rows, the step record, the
+// thermostat's factors and the step count (before: two reductions of one or two
+// launches, two final kernels and the count, 4 to 5 us each; a batch's two
+// segmented sums 17 us each; now 4 us for 64 cells, 6 for 2744, 10 for a batch of
+// 64 boxes, 15 for 1 M molecules). Replica r's rows go to min(rows / kStepRows,
+// kStepBlocks) blocks (its own rows alone decide, so a replica's sums do not
+// depend on the batch); a replica of several blocks is finished by the block
+// that takes its last ticket, from the block sums in block order. Thread t of a
+// block adds rows t, t + 256, ..., the threads' sums go through one tree.
+__global__ __launch_bounds__(256) void k_step_end(StepEnd a) {
+    const int r = blockIdx.y, t = threadIdx.x;
+    const int m0 = a.cell_off[r], m1 = a.cell_off[r + 1];
+    const int nb = max(1, min(kStepBlocks, (m1 - m0 + kStepRows - 1) / kStepRows));
+    const int b = blockIdx.x;
+    if (b >= nb) return;
+    double v[8];
+    for (int k = 0; k < 8; ++k) v[k] = 0.0;
+    auto rows = [&](const double *in, int b0, int b1, double *x) {
+        const int per = (b1 - b0 + nb - 1) / nb;
+        const int k0 = b0 + b * per, k1 = min(k0 + per, b1);
+        for (int k = k0 + t; k < k1; k += 256) {
+            const double2 *p = reinterpret_cast<const double2 *>(in) + 2 * (size_t)k;
+            const double2 lo = p[0], hi = p[1];
+            x[0] += lo.x;
+            x[1] += lo.y;
+            x[2] += hi.x;
+            x[3] += hi.y;
         }
-        if (threadIdx.x == 0) out[(size_t)blockIdx.x * width + w] = red[0];
-        __syncthreads();
+    };
+    if ((a.what & kEndMacro) && a.macro_part) rows(a.macro_part, m0, m1, v);
+    if (a.what & kEndLeapfrog) rows(a.lf_part, a.lf_off[r], a.lf_off[r + 1], v + 4);
+    __shared__ double red[8][192];
+    if (t >= 64)
+        for (int k = 0; k < 8; ++k) red[k][t - 64] = v[k];
+    __syncthreads();
+    if (t >= 64) return;
+    for (int k = 0; k < 8; ++k) v[k] = (v[k] + red[k][t + 64]) + (red[k][t] + red[k][t + 128]);
+    auto tree = [&]() {
+        for (int k = 0; k < 8; ++k)
+            for (int o = 32; o > 0; o >>= 1) v[k] += __shfl_down(v[k], o, 64);
+    };
+    tree();
+    if (nb > 1) {
+        double *part = a.part + (size_t)r * kStepBlocks * 8;
+        int last = 0;
+        if (t == 0) {
+            for (int k = 0; k < 8; ++k)
+                __hip_atomic_store(&part[b * 8 + k], v[k], __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+            last = __hip_atomic_fetch_add(&a.ticket[r], 1, __ATOMIC_ACQ_REL,
+                                          __HIP_MEMORY_SCOPE_AGENT) == nb - 1;
+        }
+        if (!__shfl(last, 0, 64)) return;
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        for (int k = 0; k < 8; ++k)
+            v[k] = t < nb ? __hip_atomic_load(&part[t * 8 + k], __ATOMIC_RELAXED,
+                                              __HIP_MEMORY_SCOPE_AGENT)
+                          : 0.0;
+        tree();
     }
+    if (t > 0) return;
+    if (nb > 1) a.ticket[r] = 0;  // (for the next launch: no block is left to take one)
+    const int step = a.step_idx[r];
+    double *rec = a.step_out + 6 * ((size_t)step * a.nrep + r);
+    if (a.what & kEndMacro)
+        finalize_macro(v, a.macro + 4 * r, rec, a.lrc ? a.lrc + kThermoW * r : nullptr);
+    if (a.what & kEndLeapfrog) {
+        for (int k = 0; k < 4; ++k) a.sums[4 * r + k] = v[4 + k];
+        finalize_lf(v + 4, rec, a.thermo ? a.thermo + kThermoW * r : nullptr, a.heuristics);
+    }
+    if (a.what & kEndAdvance) a.step_idx[r] = step + 1;
 }
 
-__global__ void k_step_advance(int *step_idx) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) step_idx[0] += 1;
-}
+// (the host code lies in another file)
+template __global__ void k_leapfrog_post<false>(MolArrays, double *, double *, double *,
+                                                const Component *, int, Reps, double, int,
+                                                const int *, const int *, double *, int, int,
+                                                SiteArrays, SiteArrays, SiteArrays, SiteArrays,
+                                                const double *);
+template __global__ void k_leapfrog_post<true>(MolArrays, double *, double *, double *,
+                                               const Component *, int, Reps, double, int,
+                                               const int *, const int *, double *, int, int,
+                                               SiteArrays, SiteArrays, SiteArrays, SiteArrays,
+                                               const double *);
+template __global__ void k_leapfrog_post_pre<false>(MolArrays, const double *, const double *,
+                                                    const Component *, int, Reps, double, int,
+                                                    const int *, const int *, double *, Bins,
+                                                    SiteArrays, SiteArrays, SiteArrays,
+                                                    SiteArrays);
+template __global__ void k_leapfrog_post_pre<true>(MolArrays, const double *, const double *,
+                                                   const Component *, int, Reps, double, int,
+                                                   const int *, const int *, double *, Bins,
+                                                   SiteArrays, SiteArrays, SiteArrays,
+                                                   SiteArrays);
 
 // Download helper: scatter a current-order array back to upload order.
 __global__ void k_scatter_orig(int n, const int *__restrict__ orig, const double *__restrict__ a,
