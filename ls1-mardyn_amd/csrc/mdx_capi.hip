@@ -12,6 +12,7 @@
 #include "../../include/ls1amd.h"
 #include "mdx_adjoint.h"
 #include "mdx_internal.h"
+#include "mdx_transfer.h"
 
 namespace mdx {
 __global__ void k_leapfrog_pre(MolArrays, const double *, const double *, const Component *, Reps,
@@ -48,6 +49,9 @@ __global__ void k_velocity_scale(MolArrays, double *, double *, const Component 
 __global__ void k_scatter_orig(int, const int *, const double *, double *, int, int);
 __global__ void k_normalize_q(int, MolArrays, long long);
 __global__ void k_step_end(StepEnd);
+__global__ void k_pack(PackArgs);
+__global__ void k_unpack(UnpackArgs);
+__global__ void k_iota(int *, int);
 __global__ void k_enum_pairs(Geom, int, int *);
 }  // namespace mdx
 
@@ -151,7 +155,10 @@ struct mdx_context {
     double *F = nullptr, *M = nullptr, *Vi = nullptr;
     int *cell = nullptr, *rank = nullptr, *count = nullptr, *start = nullptr, *perm = nullptr,
         *mcell = nullptr, *ls1id = nullptr, *mls1id = nullptr;
-    double *dl_tmp = nullptr;   // download staging (4 n)
+    double *dl_tmp = nullptr;   // transfer staging, dl_cap doubles (>= 4 n)
+    size_t dl_cap = 0;
+    PinnedRing ring;
+    std::vector<long> state_sig;  // what the state's allocations were sized for
     double *adj_site = nullptr, *adj_cot = nullptr, *adj_part = nullptr, *adj_out = nullptr;
     double *scratch = nullptr;  // this device's copy of the library scratch array
     int *nsite_mol[kTypes] = {nullptr, nullptr, nullptr, nullptr};
@@ -1076,36 +1083,13 @@ int ensure_steps(mdx_context *c, int nsteps) {
     return MDX_OK;
 }
 
-int state_setup(mdx_context *c, int64_t n64, const int32_t *cid_host) {
-    if (n64 <= 0 || n64 > (1 << 27)) return fail(c, MDX_ERR_ARG, "molecule count out of range");
-    if (c->nrep > 1) {
-        int64_t tot = 0;
-        for (int64_t k : c->rep_n) tot += k;
-        if (tot != n64) return fail(c, MDX_ERR_ARG, "n differs from the sum of replica counts");
-    }
-    const int n = (int)n64;
-    drop_graphs(c);
-    c->rmm_dt = 0.0;  // a new state starts with full-step velocities
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    free_list(c->state_allocs);
-    c->n = n;
-    for (int t = 0; t < kTypes; ++t) c->nsites[t] = 0;
-    for (int i = 0; i < n; ++i) {
-        int k = cid_host[i];
-        if (k < 0 || k >= c->model.ncomp) return fail(c, MDX_ERR_ARG, "component id out of range");
-        for (int t = 0; t < kTypes; ++t) c->nsites[t] += c->model.comp[k].n[t];
-    }
-    for (int t = 0; t < kTypes; ++t)
-        if (c->nsites[t] >= (1 << 27)) return fail(c, MDX_ERR_CAPACITY, "too many sites");
-    c->binned = false;
+// The state's arrays for n molecules.
+int state_alloc(mdx_context *c, int n) {
     TRY(alloc_mol(c, c->mol[0], n));
     TRY(alloc_mol(c, c->mol[1], n, c->point_lj ? &c->mol[0] : nullptr));
-    c->q_renorm = 0;
     TRY(dalloc(c, &c->F, 3 * (size_t)n, true));
     TRY(dalloc(c, &c->M, 3 * (size_t)n, true));
     TRY(dalloc(c, &c->Vi, 3 * (size_t)n, true));
-    int *ip[] = {nullptr};
-    (void)ip;
     TRY(dalloc(c, &c->cell, n, true));
     TRY(dalloc(c, &c->rank, n, true));
     TRY(dalloc(c, &c->perm, n, true));
@@ -1122,10 +1106,8 @@ int state_setup(mdx_context *c, int64_t n64, const int32_t *cid_host) {
         TRY(alloc_sites(c, c->sites[t], c->nsites[t], c->ncell, n, t));
     }
     if (c->point_lj) {
-        std::vector<int> id((size_t)n + 1);
-        for (int i = 0; i <= n; ++i) id[i] = i;
         TRY(dalloc(c, &c->ident, (size_t)n + 1, true));
-        HIPCHK(c, hipMemcpy(c->ident, id.data(), 4 * id.size(), hipMemcpyHostToDevice));
+        hipLaunchKernelGGL(k_iota, dim3(nblk(n + 1)), dim3(kBlock), 0, c->stream, c->ident, n + 1);
     }
     TRY(alloc_scan(c, std::max(n, c->ncell) + 1));
     TRY(dalloc(c, &c->macro_part, (size_t)c->ncell * 4, true));
@@ -1166,8 +1148,51 @@ int state_setup(mdx_context *c, int64_t n64, const int32_t *cid_host) {
         TRY(dalloc(c, &c->d_mol_rep, n, true));
         HIPCHK(c, hipMemcpy(c->d_mol_rep, mr.data(), 4 * mr.size(), hipMemcpyHostToDevice));
     }
-    TRY(dalloc(c, &c->dl_tmp, (size_t)n * 4, true));
+    // one array of four columns, or all of a download where that is little
+    c->dl_cap = std::max((size_t)n * 4, std::min((size_t)n * 22, (size_t)1 << 18));
+    TRY(dalloc(c, &c->dl_tmp, c->dl_cap, true));
     c->adj_site = c->adj_cot = c->adj_part = c->adj_out = nullptr;  // made on first use
+    return MDX_OK;
+}
+
+int state_setup(mdx_context *c, int64_t n64, const int32_t *cid_host) {
+    if (n64 <= 0 || n64 > (1 << 27)) return fail(c, MDX_ERR_ARG, "molecule count out of range");
+    if (c->nrep > 1) {
+        int64_t tot = 0;
+        for (int64_t k : c->rep_n) tot += k;
+        if (tot != n64) return fail(c, MDX_ERR_ARG, "n differs from the sum of replica counts");
+    }
+    const int n = (int)n64;
+    long nsites[kTypes] = {0, 0, 0, 0};
+    for (int i = 0; i < n; ++i) {
+        int k = cid_host[i];
+        if (k < 0 || k >= c->model.ncomp) return fail(c, MDX_ERR_ARG, "component id out of range");
+        for (int t = 0; t < kTypes; ++t) nsites[t] += c->model.comp[k].n[t];
+    }
+    for (int t = 0; t < kTypes; ++t)
+        if (nsites[t] >= (1 << 27)) return fail(c, MDX_ERR_CAPACITY, "too many sites");
+    drop_graphs(c);
+    c->rmm_dt = 0.0;  // a new state starts with full-step velocities
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    c->n = n;
+    for (int t = 0; t < kTypes; ++t) c->nsites[t] = (int)nsites[t];
+    c->binned = false;
+    c->site_forms = 0;
+    c->q_renorm = 0;
+    // A state of the same shape takes the arrays of the one before it (a fit
+    // uploads new positions on every call: some 60 allocations and frees, 0.36
+    // ms of a 500-molecule upload).
+    std::vector<long> sig = {n, c->ncell, c->nrep, c->point_lj};
+    for (int t = 0; t < kTypes; ++t) sig.push_back(c->nsites[t]);
+    if (c->nrep > 1) sig.insert(sig.end(), c->rep_n.begin(), c->rep_n.end());
+    if (sig != c->state_sig) {
+        c->state_sig.clear();
+        c->have_state = false;
+        free_list(c->state_allocs);
+        TRY(state_alloc(c, n));
+        c->state_sig = sig;
+    }
+    if (c->ring.open(22 * sizeof(double) * (size_t)n) != hipSuccess) (void)hipGetLastError();  // copies then are pageable
     HIPCHK(c, hipMemsetAsync(c->F, 0, 3 * (size_t)n * 8, c->stream));
     HIPCHK(c, hipMemsetAsync(c->M, 0, 3 * (size_t)n * 8, c->stream));
     HIPCHK(c, hipMemsetAsync(c->Vi, 0, 3 * (size_t)n * 8, c->stream));
@@ -1245,6 +1270,7 @@ int mdx_destroy(mdx_context *c) {
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
     drop_graphs(c);
+    c->ring.close();
     free_list(c->state_allocs);
     free_list(c->allocs);
     for (auto &e : c->ev)
@@ -1551,30 +1577,40 @@ int mdx_upload(mdx_context *c, int64_t n, const double *r, const double *v, cons
     HIPCHK(c, hipSetDevice(c->device));
     TRY(state_setup(c, n, cid));
     const int nn = (int)n;
-    std::vector<double> buf((size_t)nn);
     MolArrays &m = c->mol[0];
-    auto put = [&](const double *src, int stride, int k, double dflt, double *dst) -> int {
-        for (int i = 0; i < nn; ++i) buf[i] = src ? src[(size_t)i * stride + k] : dflt;
-        HIPCHK(c, hipMemcpy(dst, buf.data(), (size_t)nn * 8, hipMemcpyHostToDevice));
-        return MDX_OK;
-    };
-    TRY(put(r, 3, 0, 0., m.rx));
-    TRY(put(r, 3, 1, 0., m.ry));
-    TRY(put(r, 3, 2, 0., m.rz));
-    TRY(put(v, 3, 0, 0., m.vx));
-    TRY(put(v, 3, 1, 0., m.vy));
-    TRY(put(v, 3, 2, 0., m.vz));
-    TRY(put(q, 4, 0, 1., m.qw));
-    TRY(put(q, 4, 1, 0., m.qx));
-    TRY(put(q, 4, 2, 0., m.qy));
-    TRY(put(q, 4, 3, 0., m.qz));
-    TRY(put(L, 3, 0, 0., m.Lx));
-    TRY(put(L, 3, 1, 0., m.Ly));
-    TRY(put(L, 3, 2, 0., m.Lz));
-    HIPCHK(c, hipMemcpy(m.cid, cid, (size_t)nn * 4, hipMemcpyHostToDevice));
-    std::vector<int> orig((size_t)nn);
-    for (int i = 0; i < nn; ++i) orig[i] = i;
-    HIPCHK(c, hipMemcpy(m.orig, orig.data(), (size_t)nn * 4, hipMemcpyHostToDevice));
+    const double *src[4] = {r, v, q, L};
+    const int width[4] = {3, 3, 4, 3};
+    const UnpackPart part[4] = {{{m.rx, m.ry, m.rz, nullptr}, -1, 3, 0.},
+                                {{m.vx, m.vy, m.vz, nullptr}, -1, 3, 0.},
+                                {{m.qw, m.qx, m.qy, m.qz}, -1, 4, 1.},
+                                {{m.Lx, m.Ly, m.Lz, nullptr}, -1, 3, 0.}};
+    {
+        HostTransfer tr(c->ring, c->stream, c->device, 13 * sizeof(double) * (size_t)nn);
+        for (int k0 = 0; k0 < 4;) {  // as many arrays at a time as the staging takes
+            UnpackArgs a;
+            memset(&a, 0, sizeof(a));
+            std::vector<HostPiece> pieces;
+            size_t used = 0;
+            int k = k0;
+            for (; k < 4 && (k == k0 || used + (size_t)nn * width[k] <= c->dl_cap); ++k) {
+                a.p[k - k0] = part[k];
+                if (!src[k]) continue;
+                a.p[k - k0].off = (long long)used;
+                pieces.push_back({(char *)src[k], sizeof(double) * (size_t)nn * width[k]});
+                used += (size_t)nn * width[k];
+            }
+            tr.to_device((char *)c->dl_tmp, pieces);
+            tr.wait();
+            a.in = c->dl_tmp;
+            a.orig = k0 == 0 ? m.orig : nullptr;
+            a.n = nn;
+            hipLaunchKernelGGL(k_unpack, dim3(nblk(nn), k - k0), dim3(kBlock), 0, c->stream, a);
+            k0 = k;
+        }
+        HIPCHK(c, tr.finish());
+    }
+    HIPCHK(c, hipMemcpyAsync(m.cid, cid, (size_t)nn * 4, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
     c->ids.assign((size_t)nn, 0);
     for (int i = 0; i < nn; ++i) c->ids[i] = ids ? ids[i] : (uint64_t)(i + 1);
     c->have_state = true;
@@ -1600,9 +1636,8 @@ int mdx_upload_device(mdx_context *c, int64_t n, const double *r, const double *
         HIPCHK(c, hipMemcpyAsync(dst[k], srcs[k], (size_t)nn * 8, hipMemcpyDeviceToDevice,
                                  c->stream));
     HIPCHK(c, hipMemcpyAsync(m.cid, cid, (size_t)nn * 4, hipMemcpyDeviceToDevice, c->stream));
-    std::vector<int> orig((size_t)nn);
-    for (int i = 0; i < nn; ++i) orig[i] = i;
-    HIPCHK(c, hipMemcpy(m.orig, orig.data(), (size_t)nn * 4, hipMemcpyHostToDevice));
+    hipLaunchKernelGGL(k_iota, dim3(nblk(nn)), dim3(kBlock), 0, c->stream, m.orig, nn);
+    HIPCHK(c, hipStreamSynchronize(c->stream));
     c->ids.assign((size_t)nn, 0);
     for (int i = 0; i < nn; ++i) c->ids[i] = (uint64_t)(i + 1);
     c->have_state = true;
@@ -1613,67 +1648,85 @@ int mdx_upload_device(mdx_context *c, int64_t n, const double *r, const double *
 
 namespace {
 
+// Downloads of at most this many bytes are packed straight into pinned memory:
+// one launch and one wait (500 molecules: 370 -> 40 us).
+constexpr size_t kDirectBytes = PinnedRing::kSmall;
+
 // Every uploaded molecule (live or deleted) in upload order.
 int download_all(mdx_context *c, double *r, double *v, double *q, double *L, double *F,
                  double *M, double *Vi, uint64_t *ids) {
     HIPCHK(c, hipSetDevice(c->device));
     const int nn = c->n;
     MolArrays &m = c->mol[c->cur];
-    double *tmp = c->dl_tmp;
     if (c->point_lj && c->q_renorm > 0) {  // the pending normalisations of q
         hipLaunchKernelGGL(k_normalize_q, dim3(nblk(nn)), dim3(kBlock), 0, c->stream, nn, m,
                            (long long)c->q_renorm);
         HIPCHK(c, hipGetLastError());
         c->q_renorm = 0;
     }
-    // upload-order arrays (point_lj: q, L) are copied as they are
-    auto get_plain = [&](const double *a, double *out) -> int {
-        HIPCHK(c, hipMemcpyAsync(out, a, (size_t)nn * 8, hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
-        return MDX_OK;
+    // upload-order arrays (point_lj: q, L) are taken as they are
+    const size_t N = (size_t)nn;
+    const int kept = c->point_lj;
+    struct Part {
+        double *dst;
+        PackPart p;
     };
-    auto get = [&](const double *a, int width, int stride_in, double *out) -> int {
-        if (!out) return MDX_OK;
-        hipLaunchKernelGGL(k_scatter_orig, dim3(nblk(nn)), dim3(kBlock), 0, c->stream, nn, m.orig,
-                           a, tmp, stride_in, width);
-        HIPCHK(c, hipMemcpyAsync(out, tmp, (size_t)nn * width * 8, hipMemcpyDeviceToHost,
-                                 c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
-        return MDX_OK;
+    std::vector<Part> parts;
+    auto add = [&](double *dst, const double *x, const double *y, const double *z,
+                   const double *w, int plain) {
+        if (dst) parts.push_back({dst, {{x, y, z, w}, 0, w ? 4 : 3, plain}});
     };
-    // the molecule arrays are separate allocations; gather them pairwise
-    auto get3 = [&](double *x, double *y, double *z, int width, double *out) -> int {
-        if (!out) return MDX_OK;
-        double *parts[4] = {x, y, z, nullptr};
-        std::vector<double> col((size_t)nn);
-        for (int w = 0; w < width; ++w) {
-            TRY(get(parts[w], 1, nn, col.data()));
-            for (int i = 0; i < nn; ++i) out[(size_t)i * width + w] = col[i];
+    add(r, m.rx, m.ry, m.rz, nullptr, 0);
+    add(v, m.vx, m.vy, m.vz, nullptr, 0);
+    add(q, m.qw, m.qx, m.qy, m.qz, kept);
+    add(L, m.Lx, m.Ly, m.Lz, nullptr, kept);
+    add(F, c->F, c->F + N, c->F + 2 * N, nullptr, 0);
+    add(M, c->M, c->M + N, c->M + 2 * N, nullptr, 0);
+    add(Vi, c->Vi, c->Vi + N, c->Vi + 2 * N, nullptr, 0);
+    size_t total = 0;
+    for (const Part &p : parts) total += N * p.p.width;
+    auto pack = [&](size_t k0, size_t k1, double *out) {
+        PackArgs a;
+        memset(&a, 0, sizeof(a));
+        size_t off = 0;
+        for (size_t k = k0; k < k1; ++k) {
+            a.p[k - k0] = parts[k].p;
+            a.p[k - k0].off = off;
+            off += N * parts[k].p.width;
         }
-        return MDX_OK;
+        a.orig = m.orig;
+        a.out = out;
+        a.n = nn;
+        hipLaunchKernelGGL(k_pack, dim3(nblk(nn), (unsigned)(k1 - k0)), dim3(kBlock), 0, c->stream,
+                           a);
     };
-    TRY(get3(m.rx, m.ry, m.rz, 3, r));
-    TRY(get3(m.vx, m.vy, m.vz, 3, v));
-    auto get_rot = [&](double *const *parts, int width, double *out) -> int {
-        if (!out) return MDX_OK;
-        std::vector<double> col((size_t)nn);
-        for (int w = 0; w < width; ++w) {
-            if (c->point_lj)
-                TRY(get_plain(parts[w], col.data()));
-            else
-                TRY(get(parts[w], 1, nn, col.data()));
-            for (int i = 0; i < nn; ++i) out[(size_t)i * width + w] = col[i];
+    if (total > 0 && total * 8 <= kDirectBytes && c->ring.mem) {
+        pack(0, parts.size(), (double *)c->ring.dev);
+        HIPCHK(c, hipGetLastError());
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        const double *src = (const double *)c->ring.mem;
+        for (const Part &p : parts) {
+            memcpy(p.dst, src, 8 * N * p.p.width);
+            src += N * p.p.width;
         }
+        if (ids) memcpy(ids, c->ids.data(), 8 * N);
         return MDX_OK;
-    };
-    double *const lparts[3] = {m.Lx, m.Ly, m.Lz}, *const qparts[4] = {m.qw, m.qx, m.qy, m.qz};
-    TRY(get_rot(lparts, 3, L));
-    TRY(get_rot(qparts, 4, q));
-    TRY(get(c->F, 3, nn, F));
-    TRY(get(c->M, 3, nn, M));
-    TRY(get(c->Vi, 3, nn, Vi));
-    if (ids)
-        for (int i = 0; i < nn; ++i) ids[i] = c->ids[i];
+    }
+    HostTransfer tr(c->ring, c->stream, c->device, 8 * (total + (ids ? N : 0)));
+    if (ids) tr.host_copy(ids, c->ids.data(), 8 * N);
+    for (size_t k0 = 0; k0 < parts.size();) {  // as many arrays as the staging takes
+        std::vector<HostPiece> pieces;
+        size_t k = k0, used = 0;
+        for (; k < parts.size() && (k == k0 || used + N * parts[k].p.width <= c->dl_cap); ++k) {
+            pieces.push_back({(char *)parts[k].dst, 8 * N * parts[k].p.width});
+            used += N * parts[k].p.width;
+        }
+        pack(k0, k, c->dl_tmp);
+        tr.to_host((const char *)c->dl_tmp, pieces);
+        k0 = k;
+    }
+    HIPCHK(c, tr.finish());
+    HIPCHK(c, hipGetLastError());
     return MDX_OK;
 }
 
@@ -2052,8 +2105,9 @@ int adjoint_run(mdx_context *c, const double *cot, double *dU_deps, double *dU_d
     const int nsl = c->nsites[T_LJ], nsc = c->nsites[T_C];
     MolArrays &m = c->mol[c->cur];
     if (cot) {
-        HIPCHK(c, hipMemcpyAsync(c->dl_tmp, cot, (size_t)nn * 3 * 8, hipMemcpyHostToDevice,
-                                 c->stream));
+        HostTransfer tr(c->ring, c->stream, c->device, (size_t)nn * 3 * 8);
+        tr.to_device((char *)c->dl_tmp, {{(char *)cot, (size_t)nn * 3 * 8}});
+        HIPCHK(c, tr.finish());
         hipLaunchKernelGGL(gather_orig3_kernel(), dim3(nblk(nn)), dim3(kBlock), 0, c->stream, nn,
                            m.orig, c->dl_tmp, b.cot);
     }
@@ -2120,9 +2174,11 @@ int adjoint_run(mdx_context *c, const double *cot, double *dU_deps, double *dU_d
                            c->dl_tmp, b.cot, nn, 3);
     }
     if (c->timing) HIPCHK(c, hipEventRecord(c->ev[3], c->stream));
-    if (vjp)
-        HIPCHK(c, hipMemcpyAsync(vjp, b.cot, (size_t)nn * 3 * 8, hipMemcpyDeviceToHost,
-                                 c->stream));
+    if (vjp) {
+        HostTransfer tr(c->ring, c->stream, c->device, (size_t)nn * 3 * 8);
+        tr.to_host((const char *)b.cot, {{(char *)vjp, (size_t)nn * 3 * 8}});
+        HIPCHK(c, tr.finish());
+    }
     HIPCHK(c, hipStreamSynchronize(c->stream));
     if (c->timing) {
         // kernel time: the derivative passes with their reductions, and up to

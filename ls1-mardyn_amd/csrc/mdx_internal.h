@@ -145,6 +145,34 @@ enum {
     kThT = 4, kThBetaT = 5, kThBetaR = 6, kThExplode = 7, kThermoW = 8
 };
 
+// Arrays of a download: part p's columns a[0 .. width), in current order (plain:
+// upload order), become rows of `width` in upload order at out + off.
+struct PackPart {
+    const double *a[4];
+    size_t off;
+    int width, plain;
+};
+struct PackArgs {
+    PackPart p[7];
+    const int *orig;
+    double *out;
+    int n;
+};
+// Arrays of an upload, the other way round, current order = upload order; a part
+// with off < 0 takes its default (first, 0, 0, 0).
+struct UnpackPart {
+    double *a[4];
+    long long off;
+    int width;
+    double first;
+};
+struct UnpackArgs {
+    UnpackPart p[4];
+    const double *in;
+    int *orig;  // set to 0 .. n - 1, or null
+    int n;
+};
+
 // The sums of a step (k_step_end): the pair kernels' cell rows and the leapfrog
 // chunks' rows of each replica.
 struct StepEnd {

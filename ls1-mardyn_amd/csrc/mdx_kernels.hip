@@ -1089,4 +1089,31 @@ __global__ void k_scatter_orig(int n, const int *__restrict__ orig, const double
     for (int w = 0; w < width; ++w) out[o * width + w] = a[w * stride_in + i];
 }
 
+// A download's arrays (one per blockIdx.y) as the caller's rows, so the host
+// only moves bytes: it transposed 16 columns before (1 M molecules: a third of
+// 24.7 ms).
+__global__ __launch_bounds__(256) void k_pack(PackArgs a) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= a.n) return;
+    const PackPart &p = a.p[blockIdx.y];
+    const size_t o = p.plain ? i : a.orig[i];
+    double *out = a.out + p.off + o * p.width;
+    for (int w = 0; w < p.width; ++w) out[w] = p.a[w][i];
+}
+
+// An upload's rows into columns.
+__global__ __launch_bounds__(256) void k_unpack(UnpackArgs a) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= a.n) return;
+    const UnpackPart &p = a.p[blockIdx.y];
+    for (int w = 0; w < p.width; ++w)
+        p.a[w][i] = p.off >= 0 ? a.in[p.off + (size_t)i * p.width + w] : w == 0 ? p.first : 0.;
+    if (blockIdx.y == 0 && a.orig) a.orig[i] = i;
+}
+
+__global__ void k_iota(int *a, int n) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) a[i] = i;
+}
+
 }  // namespace mdx

@@ -233,7 +233,6 @@ class Context:
 
     def upload(self, r, v, q, L, cid, ids=None):
         n = len(r)
-        self.n = n
         f = lambda a, w: np.ascontiguousarray(np.asarray(a, np.float64).reshape(n, w))
         idp = None
         if ids is not None:
@@ -241,6 +240,7 @@ class Context:
             idp = _ptr(self._ids)
         self._chk(self.L.mdx_upload(self.h, n, f(r, 3), f(v, 3), f(q, 4), f(L, 3),
                                     np.ascontiguousarray(cid, np.int32), idp), "mdx_upload")
+        self.n = n
 
     def molecule_count(self):
         """Live molecules: the uploaded count less those deleted at outflow walls."""
@@ -248,15 +248,15 @@ class Context:
         self._chk(self.L.mdx_molecule_count(self.h, C.byref(k)), "mdx_molecule_count")
         return k.value
 
-    def download(self):
+    def download(self, keys=None):
         """State in upload order (with outflow walls: the surviving molecules,
-        ids tell which)."""
+        ids tell which). keys: the arrays wanted (all of r, v, q, L, F, M, Vi,
+        ids by default)."""
         n = self.molecule_count() if self.open else self.n
-        out = dict(r=np.zeros((n, 3)), v=np.zeros((n, 3)), q=np.zeros((n, 4)), L=np.zeros((n, 3)),
-                   F=np.zeros((n, 3)), M=np.zeros((n, 3)), Vi=np.zeros((n, 3)),
-                   ids=np.zeros(n, np.uint64))
-        self._chk(self.L.mdx_download(self.h, n, *(_ptr(out[k]) for k in
-                                                   ("r", "v", "q", "L", "F", "M", "Vi", "ids"))),
+        names = ("r", "v", "q", "L", "F", "M", "Vi", "ids")
+        out = {k: np.empty(n, np.uint64) if k == "ids" else np.empty((n, 4 if k == "q" else 3))
+               for k in (names if keys is None else keys)}
+        self._chk(self.L.mdx_download(self.h, n, *(_ptr(out.get(k)) for k in names)),
                   "mdx_download")
         return out
 
@@ -367,7 +367,7 @@ class Context:
         c = None
         if cot is not None:
             c = np.ascontiguousarray(cot, np.float64).reshape(n, 3)
-            out["vjp"] = np.zeros((n, 3))
+            out["vjp"] = np.empty((n, 3))
         fn, name = ((self.L.mdx_adjoint_noalloc, "mdx_adjoint_noalloc") if noalloc
                     else (self.L.mdx_adjoint, "mdx_adjoint"))
         self._chk(fn(self.h, n, _ptr(c), *(_ptr(out[k]) for k in (

@@ -87,7 +87,7 @@ class ForceFieldEngine:
         self.ctx.upload(r, s.v, s.q, s.L, s.cid)
         self.ctx.update_container()
         self._macro = self.ctx.traverse()
-        self._F = self.ctx.download()["F"]
+        self._F = self.ctx.download(("F",))["F"]
         self._loaded = key
 
     def evaluate(self, eps, sig, q, r):
