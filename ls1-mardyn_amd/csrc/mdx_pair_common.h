@@ -284,6 +284,50 @@ __device__ __forceinline__ Nbr neighbour(const Geom &g, int cx, int cy, int cz, 
     return b;
 }
 
+// x of the lane that the DPP control names; 0 where there is none and in rows
+// of 16 lanes outside the row mask
+template <int CTRL, int ROWS> __device__ __forceinline__ int dpp(int x) {
+    return __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xf, false);
+}
+template <int CTRL, int ROWS> __device__ __forceinline__ double dpp(double x) {
+    return __hiloint2double(dpp<CTRL, ROWS>(__double2hiint(x)), dpp<CTRL, ROWS>(__double2loint(x)));
+}
+// inclusive prefix sums over the wave (row shifts by 1, 2, 4, 8, then the row
+// ends broadcast into the next rows), without LDS round trips
+template <typename X> __device__ __forceinline__ X wave_scan(X x) {
+    x += dpp<0x111, 0xf>(x);
+    x += dpp<0x112, 0xf>(x);
+    x += dpp<0x114, 0xf>(x);
+    x += dpp<0x118, 0xf>(x);
+    x += dpp<0x142, 0xa>(x);
+    x += dpp<0x143, 0xc>(x);
+    return x;
+}
+// the same for the maximum of values >= 0
+__device__ __forceinline__ int wave_max_scan(int x) {
+    x = max(x, dpp<0x111, 0xf>(x));
+    x = max(x, dpp<0x112, 0xf>(x));
+    x = max(x, dpp<0x114, 0xf>(x));
+    x = max(x, dpp<0x118, 0xf>(x));
+    x = max(x, dpp<0x142, 0xa>(x));
+    x = max(x, dpp<0x143, 0xc>(x));
+    return x;
+}
+
+// LDS by 32-bit address.
+__device__ __forceinline__ unsigned lds_address(const void *p) {
+    return (unsigned)(uintptr_t)(const __attribute__((address_space(3))) void *)p;
+}
+
+template <typename T> __device__ __forceinline__ T lds_value(unsigned a) {
+    return *(const __attribute__((address_space(3))) T *)a;
+}
+template <typename R> __device__ __forceinline__ Q4<R> lds_q4(unsigned a) {
+    typedef R Vec __attribute__((ext_vector_type(4)));
+    const Vec q = lds_value<Vec>(a);
+    return {q.x, q.y, q.z, q.w};
+}
+
 // Neighbour index of tile entry idx (concatenated neighbour order): the
 // largest k < nb with pre[k] <= idx.
 __device__ __forceinline__ int tile_k(const int *pre, int idx, int nb = 27) {

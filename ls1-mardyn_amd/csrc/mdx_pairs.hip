@@ -30,6 +30,19 @@
 
 namespace mdx {
 
+// What the staged sites of a neighbour take: the offset of their positions (FP64:
+// the image shift; FP32: between the cells' corners), and the site of tile entry
+// e, e + dj.
+template <typename R> struct NbrRec;
+template <> struct NbrRec<double> {
+    double x, y, z;
+    int dj, pad;
+};
+template <> struct alignas(16) NbrRec<float> {
+    float x, y, z;
+    int dj;
+};
+
 // LDS tile: the j sites of the 27 neighbour images of one cell, positions
 // already moved into the i cell's frame (FP64: + image shift, exactly the
 // reference's halo copy r + L; FP32: + offset of the neighbour's corner).
@@ -71,7 +84,7 @@ template <int TI, typename R, bool MOLSITE, bool MULTI> struct TileCfg {
     // tiles at fewer waves: FP32 quadrupole kernel -6 %; FP64 LJ -3 %,
     // charge -4 %, quadrupole -9 %.
     static constexpr int WAVES =
-        (TI == T_Q && sizeof(R) == 4) || (TI == T_C && sizeof(R) == 8) ? 4 : 1;
+        (TI == T_Q && sizeof(R) == 4) || TI == T_C ? 4 : 1;
 };
 
 template <int TI, typename R, bool MOLSITE, bool MULTI> struct Tile {
@@ -83,15 +96,15 @@ template <int TI, typename R, bool MOLSITE, bool MULTI> struct Tile {
     static constexpr int SLOT =
         (int)sizeof(Q4<R>) * (1 + C::MOL + C::ORI) + (C::MOL && TI != T_LJ ? 3 : 0);
     alignas(32) unsigned char raw[C::CAP * SLOT];
-    unsigned short lst[C::LIST][64];  // per-lane hit lists (tile indices)
-    int j0[C::NB], pre[C::NB + 1];
-    double shift[C::NB][3];
+    unsigned short lst[C::LIST][64];  // per-lane hit lists (LDS addresses of site records)
+    int pre[C::NB + 1];               // first tile entry of each neighbour
+    NbrRec<R> nbr[C::NB];
 };
 
 // The records of one partner pass (partner type TJ) in a tile's slot bytes:
 // p site position (w = charge / moment, LJ table column, or |x|^2 in FP32
 // one-centre tiles), m molecule position (w = |m|^2 in FP32 tiles), e
-// orientation (dipole and quadrupole partners), h first-site (head) indices
+// orientation (dipole and quadrupole partners), h addresses of the first sites
 // and ns site counts at heads (charge partners, tested per molecule).
 template <int TI, int TJ, typename R, bool MOLSITE, bool MULTI> struct PassTile {
     using C = TileCfg<TI, R, MOLSITE, MULTI>;
@@ -115,18 +128,14 @@ template <int TI, int TJ, typename R, bool MOLSITE, bool MULTI> struct PassTile 
 };
 
 template <typename R>
-__device__ __forceinline__ V3<R> tile_offset(const Geom &g, const double (*shift)[3], int k,
-                                             int nxs);
+__device__ __forceinline__ NbrRec<R> nbr_rec(const Geom &g, const Nbr &b, int dj);
 template <>
-__device__ __forceinline__ V3<double> tile_offset<double>(const Geom &, const double (*shift)[3],
-                                                          int k, int) {
-    return {shift[k][0], shift[k][1], shift[k][2]};
+__device__ __forceinline__ NbrRec<double> nbr_rec<double>(const Geom &, const Nbr &b, int dj) {
+    return {b.s[0], b.s[1], b.s[2], dj, 0};
 }
 template <>
-__device__ __forceinline__ V3<float> tile_offset<float>(const Geom &g, const double (*)[3], int k,
-                                                        int nxs) {
-    return {(float)((k % nxs - 1) * g.cl[0]), (float)((k / nxs % 3 - 1) * g.cl[1]),
-            (float)((k / (3 * nxs) - 1) * g.cl[2])};
+__device__ __forceinline__ NbrRec<float> nbr_rec<float>(const Geom &g, const Nbr &b, int dj) {
+    return {(float)(b.dd[0] * g.cl[0]), (float)(b.dd[1] * g.cl[1]), (float)(b.dd[2] * g.cl[2]), dj};
 }
 
 constexpr int kUnroll = 4;  // stage-A candidates in flight per lane
@@ -178,28 +187,20 @@ __device__ __forceinline__ void partner_pass(const PairArgs &a, const Geom &g, i
         cut = (R)(rc2 * (1.0 + band));
     }
     unsigned long long nhit = 0;
-    int nk = 0;
+    int nk = 0, j0 = 0;
     const int nb = 9 * nxs;  // neighbour ranges: 27, or 36 for two cells
+    Nbr nbr = neighbour(g, cx, cy, cz, lane, nxs);
+    if (lane < nb && nbr.ok) {
+        j0 = J.cstart[cbase + nbr.cell];
+        nk = J.cstart[cbase + nbr.cell + 1] - j0;
+    }
+    const int incl = wave_scan(nk), pre = incl - nk;
     if (lane < nb) {
-        Nbr b = neighbour(g, cx, cy, cz, lane, nxs);
-        int j0 = 0;
-        if (b.ok) {
-            j0 = J.cstart[cbase + b.cell];
-            nk = J.cstart[cbase + b.cell + 1] - j0;
-        }
-        T.j0[lane] = j0;
-        T.shift[lane][0] = b.s[0];
-        T.shift[lane][1] = b.s[1];
-        T.shift[lane][2] = b.s[2];
+        T.pre[lane + 1] = incl;
+        T.nbr[lane] = nbr_rec<R>(g, nbr, j0 - pre);
     }
-    int incl = nk;
-    for (int o = 1; o < (C::NB > 32 ? 64 : 32); o <<= 1) {
-        int y = __shfl_up(incl, o, 64);
-        if (lane >= o) incl += y;
-    }
-    if (lane < nb) T.pre[lane + 1] = incl;
     if (lane == 0) T.pre[0] = 0;
-    const int total = __shfl(incl, nb - 1, 64);
+    const int total = __builtin_amdgcn_readlane(incl, 63);
     __syncthreads();
     // Charge partners are tested once per molecule (neutral molecules carry
     // two or more charges): the tile keeps a molecule's sites contiguous, the
@@ -225,19 +226,35 @@ __device__ __forceinline__ void partner_pass(const PairArgs &a, const Geom &g, i
             if (base + nst < total) {
                 const int idx = base + nst;
                 const int k = tile_k(T.pre, idx, nb);
-                next_head = SiteView<R>::heads(J, T.j0[k] + (idx - T.pre[k]));
+                next_head = SiteView<R>::heads(J, T.nbr[k].dj + idx);
             }
         }
         int nh = nst;
         int hb = 0, last_head = 0;
+        // The neighbour of each tile entry: the neighbours of the chunk leave
+        // their number + 1 at their first entry (in the hit lists' bytes, not in
+        // use here), and a maximum scan over 64 entries at a time carries it to
+        // the others: 6 operations without an LDS round trip, where a binary
+        // search of the prefix takes five dependent reads of 7 each. With the
+        // neighbours' offsets in one LDS record each, and list lengths and prefix
+        // by DPP: 1 M-molecule slab FP32 397 -> 355 us, FP64 496 -> 440; 1 M
+        // mixture, LJ 842 -> 800, charges 973 -> 936, quadrupoles 706 -> 653.
+        unsigned char *mark = reinterpret_cast<unsigned char *>(T.lst);
+        static_assert(PT::CAP <= sizeof(T.lst), "marks");
+        for (int z = 4 * lane; z < nst; z += 256) *reinterpret_cast<unsigned *>(mark + z) = 0u;
+        __syncthreads();
+        if (nk > 0 && pre < base + nst && incl > base)
+            mark[max(pre - base, 0)] = (unsigned char)(lane + 1);
+        __syncthreads();
+        int carry = 0;
         for (int s0 = 0; s0 < nst; s0 += 64) {
             const int s = s0 + lane;
             bool head = false;
+            const int k1 = max(wave_max_scan(s < nst ? mark[s] : 0), carry);
+            carry = __builtin_amdgcn_readlane(k1, 63);
             if (s < nst) {
-            const int idx = base + s;
-            const int k = tile_k(T.pre, idx, nb);
-            const int j = T.j0[k] + (idx - T.pre[k]);
-            const V3<R> off = tile_offset<R>(g, T.shift, k, nxs);
+            const NbrRec<R> off = T.nbr[k1 - 1];
+            const int j = off.dj + base + s;
             const V3<R> p = SiteView<R>::pos(J, j);
             Q4<R> q;
             q.x = p.x + off.x;
@@ -267,7 +284,9 @@ __device__ __forceinline__ void partner_pass(const PairArgs &a, const Geom &g, i
             }
             if constexpr (heads) {  // compact the heads in tile order
                 const unsigned long long hm = __ballot(head);
-                if (head) V.h[hb + __popcll(hm & ((1ull << lane) - 1ull))] = (unsigned short)s;
+                if (head)  // the address of the head's record
+                    V.h[hb + __popcll(hm & ((1ull << lane) - 1ull))] =
+                        (unsigned short)(lds_address(V.p) + s * (unsigned)sizeof(Q4<R>));
                 hb += __popcll(hm);
                 if (hm) last_head = s0 + 63 - __clzll((long long)hm);
             }
@@ -284,7 +303,15 @@ __device__ __forceinline__ void partner_pass(const PairArgs &a, const Geom &g, i
             }
         }
         __syncthreads();
-        int cnt = 0;
+        // A listed candidate is the LDS address of its site record; its test
+        // record (the molecule's, where that differs) and orientation lie MO
+        // and EO bytes behind. la: the end of the lane's list.
+        constexpr unsigned REC = sizeof(Q4<R>);
+        constexpr unsigned MO = C::MOL ? PT::CAP * REC : 0, EO = PT::CAP * REC * (1 + C::MOL);
+        const unsigned pb = lds_address(V.p), l0 = lds_address(&T.lst[0][lane]);
+        constexpr unsigned ROW = sizeof(T.lst[0]);  // an entry is a row of the lists
+        unsigned la = l0;
+        auto index = [&](unsigned at) -> int { return (int)((at - pb) / REC); };
         // Stage B. A listed candidate is final unless its molecule distance
         // is 0 (the molecule itself, SingleCellPolicy_) or, in FP32, lies in
         // the band [lo, hi] around rc^2, where the decision is re-made in FP64
@@ -292,105 +319,116 @@ __device__ __forceinline__ void partner_pass(const PairArgs &a, const Geom &g, i
         auto recheck = [&](int s) -> bool {  // the FP64 decision for tile entry s
             const int idx = base + s;
             const int k = tile_k(T.pre, idx, nb);
-            const int j = T.j0[k] + (idx - T.pre[k]);
+            const NbrRec<R> rec = T.nbr[k];
+            const int j = rec.dj + idx;
+            V3<double> sh;  // the image shift
+            if constexpr (sizeof(R) == 8) {
+                sh = {rec.x, rec.y, rec.z};
+            } else {
+                const Nbr b = neighbour(g, cx, cy, cz, k, nxs);
+                sh = {b.s[0], b.s[1], b.s[2]};
+            }
             // molecule positions through the sites' molecule indices (the
             // FP32 form builds no FP64 per-site copies)
             const int mi = a.s[TI].mol[I.idx], mj = J.mol[j];
-            const double ex = a.mrx[mi] - (a.mrx[mj] + T.shift[k][0]);
-            const double ey = a.mry[mi] - (a.mry[mj] + T.shift[k][1]);
-            const double ez = a.mrz[mi] - (a.mrz[mj] + T.shift[k][2]);
+            const double ex = a.mrx[mi] - (a.mrx[mj] + sh.x);
+            const double ey = a.mry[mi] - (a.mry[mj] + sh.y);
+            const double ez = a.mrz[mi] - (a.mrz[mj] + sh.z);
             const double r2d = ex * ex + ey * ey + ez * ez;
             return r2d < rc2 && r2d != 0.0;
         };
-        auto accept = [&](int s, const Q4<R> &q) -> bool {
+        auto accept = [&](unsigned at, const Q4<R> &q) -> bool {
             const V3<R> mi = C::MOL ? I.mol : I.pos;
             const R dx = mi.x - q.x, dy = mi.y - q.y, dz = mi.z - q.z;
             const R r2 = dx * dx + dy * dy + dz * dz;
             if (r2 == R(0)) return false;
             if constexpr (sizeof(R) == 4) {
-                if (r2 >= lo) return recheck(s);
+                if (r2 >= lo) return recheck(index(at));
             }
             return true;
         };
         auto drain = [&]() {
             Part32 pa;
             pa.clear();
+            // the longest list: a scalar trip count
+            const int emax = __builtin_amdgcn_readlane(wave_max_scan((int)((la - l0) / ROW)), 63);
             if constexpr (TI == T_LJ) {
                 // LJ: every lane runs every entry up to the longest list
-                // (exhausted lanes on entry 0 with the pair masked off), so
-                // the loop has no branch. FP32: entries in the re-check band
-                // around rc^2 are masked off here and marked in band (bit e),
-                // and re-decided in FP64 after the loop (rare)
-                unsigned band = 0u;
-                // the longest list, as a wave-uniform (scalar) trip count
-                int emax = cnt;
-                for (int o = 32; o > 0; o >>= 1) emax = max(emax, __shfl_xor(emax, o, 64));
-                emax = __builtin_amdgcn_readfirstlane(emax);
-                for (int e = 0; e < emax; ++e) {
-                    const bool act = e < cnt;
-                    const int raw = (int)T.lst[e][lane];  // e < LIST: in bounds
-                    const int sj = act ? raw : 0;
-                    const Q4<R> qj = C::MOL ? V.m[sj] : V.p[sj];
+                // (exhausted lanes on the tile's first record with the pair
+                // masked off), so the loop has no branch. FP32: entries in the
+                // re-check band around rc^2 are masked off here, and re-decided
+                // in FP64 in a second walk (rare: some 2e-5 of the entries)
+                unsigned long long near = 0;
+                unsigned lp = l0;
+                for (int e = 0; e < emax; ++e, lp += ROW) {
+                    const bool act = lp < la;
+                    unsigned raw = lds_value<unsigned short>(lp);  // e < LIST: in bounds
+                    asm("" : "+v"(raw));  // (read by all lanes: no branch around it)
+                    const unsigned at = act ? raw : pb;
+                    const Q4<R> qj = lds_q4<R>(at + MO);
                     const V3<R> mi = C::MOL ? I.mol : I.pos;
                     const R dx = mi.x - qj.x, dy = mi.y - qj.y, dz = mi.z - qj.z;
                     const R r2 = dx * dx + dy * dy + dz * dz;
                     bool ok = act && r2 != R(0);
                     if constexpr (sizeof(R) == 4) {
-                        const bool b = ok && r2 >= lo;
-                        band |= b ? (1u << e) : 0u;
-                        ok = ok && !b;
+                        const bool inner = r2 < lo;
+                        near |= __ballot(ok && !inner);
+                        ok = ok && inner;
                     }
-                    const Q4<R> pj = C::MOL ? V.p[sj] : qj;
+                    const Q4<R> pj = C::MOL ? lds_q4<R>(at) : qj;
                     eval_lj<R, MOLSITE, TAB>((const Q4<R> *)nullptr, par, I, pj, qj, ok, eps24,
                                                 sig2, shift6, acc, pa);
                     if (COUNT) nhit += ok;
                 }
                 if constexpr (sizeof(R) == 4) {
-                    while (__any(band != 0u)) {
-                        const bool has = band != 0u;
-                        const int e = has ? __builtin_ctz(band) : 0;
-                        band &= has ? band - 1u : 0u;
-                        const int sj = has ? (int)T.lst[e][lane] : 0;
-                        const bool ok = has && recheck(sj);
-                        const Q4<R> qj = C::MOL ? V.m[sj] : V.p[sj];
-                        const Q4<R> pj = C::MOL ? V.p[sj] : qj;
-                        eval_lj<R, MOLSITE, TAB>((const Q4<R> *)nullptr, par, I, pj, qj, ok, eps24,
-                                                sig2, shift6, acc, pa);
-                        if (COUNT) nhit += ok;
+                    if (near) {
+                        lp = l0;
+                        for (int e = 0; e < emax; ++e, lp += ROW) {
+                            const unsigned at = lp < la ? lds_value<unsigned short>(lp) : pb;
+                            const Q4<R> qj = lds_q4<R>(at + MO);
+                            const V3<R> mi = C::MOL ? I.mol : I.pos;
+                            const R dx = mi.x - qj.x, dy = mi.y - qj.y, dz = mi.z - qj.z;
+                            const R r2 = dx * dx + dy * dy + dz * dz;
+                            const bool b = lp < la && r2 != R(0) && !(r2 < lo);
+                            if (!__any(b)) continue;
+                            const bool ok = b && recheck(index(at));
+                            const Q4<R> pj = C::MOL ? lds_q4<R>(at) : qj;
+                            eval_lj<R, MOLSITE, TAB>((const Q4<R> *)nullptr, par, I, pj, qj, ok,
+                                                        eps24, sig2, shift6, acc, pa);
+                            if (COUNT) nhit += ok;
+                        }
                     }
                 }
             } else {
-                // the next entry's index and cutoff record are read one
+                // the next entry's address and cutoff record are read one
                 // iteration ahead, so their LDS latency overlaps the current body
-                int sn = 0;
+                unsigned an = pb, lp = l0;
                 Q4<R> qn{};
-                if (cnt > 0) {
-                    sn = (int)T.lst[0][lane];
-                    qn = C::MOL ? V.m[sn] : V.p[sn];
+                if (lp < la) {
+                    an = lds_value<unsigned short>(lp);
+                    qn = lds_q4<R>(an + MO);
                 }
-                int emax = cnt;  // the longest list: a scalar trip count
-                for (int o = 32; o > 0; o >>= 1) emax = max(emax, __shfl_xor(emax, o, 64));
-                emax = __builtin_amdgcn_readfirstlane(emax);
                 for (int e = 0; e < emax; ++e) {
-                    const bool act = e < cnt;
-                    const int sj = sn;
+                    const bool act = lp < la;
+                    const unsigned at = an;
                     const Q4<R> qj = qn;
-                    if (e + 1 < cnt) {
-                        sn = (int)T.lst[e + 1][lane];
-                        qn = C::MOL ? V.m[sn] : V.p[sn];
+                    lp += ROW;
+                    if (lp < la) {
+                        an = lds_value<unsigned short>(lp);
+                        qn = lds_q4<R>(an + MO);
                     }
-                    if (act && accept(sj, qj)) {
+                    if (act && accept(at, qj)) {
                         if constexpr (heads) {
-                            const int ns = (int)V.ns[sj];  // the molecule's sites sj .. sj + ns - 1
+                            const int ns = (int)V.ns[index(at)];  // the molecule's sites from `at` on
                             for (int t = 0; t < ns; ++t) {
-                                const Q4<R> pj = V.p[sj + t];
+                                const Q4<R> pj = lds_q4<R>(at + t * REC);
                                 eval_pair<TI, TJ, R, MOLSITE>((R)a.epsRFInvrc3, I, Q4<R>{}, pj, qj, acc, pa);
                             }
                             if (COUNT) nhit += ns;
                         } else {
-                            const Q4<R> pj = C::MOL ? V.p[sj] : qj;
+                            const Q4<R> pj = C::MOL ? lds_q4<R>(at) : qj;
                             Q4<R> eq{};
-                            if constexpr (PT::ORIJ) eq = V.e[sj];
+                            if constexpr (PT::ORIJ) eq = lds_q4<R>(at + EO);
                             eval_pair<TI, TJ, R, MOLSITE>((R)a.epsRFInvrc3, I, eq, pj, qj, acc, pa);
                             if (COUNT) ++nhit;
                         }
@@ -398,79 +436,74 @@ __device__ __forceinline__ void partner_pass(const PairArgs &a, const Geom &g, i
                 }
             }
             if constexpr (sizeof(R) == 4) pa.flush(acc);
-            cnt = 0;
+            la = l0;
         };
         // Stage A: keep candidates below the cutoff (FP32: up to the top of
         // the re-check band). Row m holds candidates m * P + ph; rows below
         // full are inside [0, nst) for every phase and need no bounds test,
         // and idle lanes carry a far-away position, so the bulk loop is a
-        // read, a distance and a compare per candidate.
+        // read, a distance, a compare and a list write per candidate. Its VALU
+        // count bounds these kernels (80 to 90 % of the issue slots): lists of
+        // addresses instead of indices, a running list address instead of a
+        // count and |i|^2 taken from the bound leave 31 operations of 37 per
+        // four candidates (1 M mixture, FP32: LJ 800 -> 751 us, charges 936 ->
+        // 859, quadrupoles 653 -> 618; 64 replicas 328 -> 316).
         // wave-uniform trip counts (scalar loop control; nh and P are
         // wave-uniform, so the division runs on the scalar unit)
         const int nhs = __builtin_amdgcn_readfirstlane(nh), Ps = __builtin_amdgcn_readfirstlane(P);
         const int per = (nhs + Ps - 1) / Ps, full = per - 1;
-        const Q4<R> *rec = (C::MOL ? V.m : V.p) + ph;
-        // candidate c of the stage-A sequence -> tile index
-        auto cand = [&](int c) -> int {
-            if constexpr (heads) return (int)V.h[c];
-            else return c;
+        // candidate c of the stage-A sequence -> its record's address
+        auto cand = [&](int c) -> unsigned {
+            if constexpr (heads) return V.h[c];
+            else return pb + (unsigned)c * REC;
         };
         const V3<R> mi = C::MOL ? Imol : Ipos;
-        // NORM: -2 i and |i|^2 per lane (idle lanes: far away, never a hit)
-        R mi2 = R(0), nx = R(0), ny = R(0), nz = R(0);
+        // NORM: -2 i, and |i|^2 taken from the bound (idle lanes: far away,
+        // never a hit)
+        R nx = R(0), ny = R(0), nz = R(0), bound = cut;
         if constexpr (NORM) {
-            mi2 = mi.x * mi.x + mi.y * mi.y + mi.z * mi.z;
+            bound = cut - (mi.x * mi.x + mi.y * mi.y + mi.z * mi.z);
             nx = R(-2) * mi.x;
             ny = R(-2) * mi.y;
             nz = R(-2) * mi.z;
         }
-        auto dist2 = [&](const Q4<R> &q) -> R {
+        auto hit = [&](const Q4<R> &q) -> bool {
             if constexpr (NORM) {
-                return __builtin_fmaf(nx, q.x, __builtin_fmaf(ny, q.y, __builtin_fmaf(nz, q.z, mi2 + q.w)));
+                return __builtin_fmaf(nx, q.x, __builtin_fmaf(ny, q.y, __builtin_fmaf(nz, q.z, q.w))) <= bound;
             } else {
                 const R dx = mi.x - q.x, dy = mi.y - q.y, dz = mi.z - q.z;
-                return dx * dx + dy * dy + dz * dz;
+                const R r2 = dx * dx + dy * dy + dz * dz;
+                return sizeof(R) == 4 ? r2 <= bound : r2 < bound;
             }
         };
-        auto test = [&](R r2) { return sizeof(R) == 4 ? r2 <= cut : r2 < cut; };
+        // every candidate is written at the end of the list and kept only on a
+        // hit (no branch; the drain test keeps the write within the list)
+        auto list = [&](unsigned at, bool h) {
+            *(__attribute__((address_space(3))) unsigned short *)la = (unsigned short)at;
+            la += h ? ROW : 0u;
+        };
         int m0 = 0;
         for (; m0 + kUnroll <= full; m0 += kUnroll) {
             // drain when some lane's list could overflow in this group
-            if (__any(cnt > C::LIST - kUnroll)) drain();
-            R r2v[kUnroll];
-            int sv[kUnroll];
+            if (__any(la > l0 + (C::LIST - kUnroll) * ROW)) drain();
+            unsigned at[kUnroll];
+            Q4<R> q[kUnroll];
 #pragma unroll
             for (int u = 0; u < kUnroll; ++u) {
-                Q4<R> q;
-                if constexpr (heads) {
-                    sv[u] = cand(ph + (m0 + u) * P);
-                    q = V.m[sv[u]];
-                } else {
-                    sv[u] = ph + (m0 + u) * P;
-                    q = rec[(m0 + u) * P];
-                }
-                r2v[u] = dist2(q);
+                at[u] = cand(ph + (m0 + u) * P);
+                q[u] = lds_q4<R>(at[u] + MO);
             }
             if (COUNT && valid) ntest += kUnroll;
-            // every candidate is written at the end of the list and kept only
-            // on a hit (no branch; the drain test above keeps cnt + kUnroll
-            // within the list)
 #pragma unroll
-            for (int u = 0; u < kUnroll; ++u) {
-                T.lst[cnt][lane] = (unsigned short)sv[u];
-                cnt += test(r2v[u]) ? 1 : 0;
-            }
+            for (int u = 0; u < kUnroll; ++u) list(at[u], hit(q[u]));
         }
         for (; m0 < per; ++m0) {  // the last rows, bounds-tested
-            if (__any(cnt > C::LIST - 1)) drain();
+            if (__any(la > l0 + (C::LIST - 1) * ROW)) drain();
             const int c = ph + m0 * P;
-            const int sidx = cand(min(c, nh - 1));
-            const Q4<R> q = C::MOL ? V.m[sidx] : V.p[sidx];
-            const R r2 = dist2(q);
+            const unsigned at = cand(min(c, nh - 1));
             const bool in = valid && c < nh;
             if (COUNT && in) ++ntest;
-            T.lst[cnt][lane] = (unsigned short)sidx;
-            cnt += (in && test(r2)) ? 1 : 0;
+            list(at, in && hit(lds_q4<R>(at + MO)));
         }
         drain();
         __syncthreads();

@@ -102,34 +102,6 @@ template <typename T> __device__ __forceinline__ const T &constant(const T *p, i
     return constant(p + __builtin_amdgcn_readfirstlane(i));
 }
 
-// x of the lane that the DPP control names; 0 where there is none and in rows
-// of 16 lanes outside the row mask
-template <int CTRL, int ROWS> __device__ __forceinline__ int dpp(int x) {
-    return __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xf, false);
-}
-template <int CTRL, int ROWS> __device__ __forceinline__ double dpp(double x) {
-    return __hiloint2double(dpp<CTRL, ROWS>(__double2hiint(x)), dpp<CTRL, ROWS>(__double2loint(x)));
-}
-// inclusive prefix sums over the wave (row shifts by 1, 2, 4, 8, then the row
-// ends broadcast into the next rows), without LDS round trips
-template <typename X> __device__ __forceinline__ X wave_scan(X x) {
-    x += dpp<0x111, 0xf>(x);
-    x += dpp<0x112, 0xf>(x);
-    x += dpp<0x114, 0xf>(x);
-    x += dpp<0x118, 0xf>(x);
-    x += dpp<0x142, 0xa>(x);
-    x += dpp<0x143, 0xc>(x);
-    return x;
-}
-
-__device__ __forceinline__ unsigned lds_address(const void *p) {
-    return (unsigned)(uintptr_t)(const __attribute__((address_space(3))) void *)p;
-}
-
-template <typename T> __device__ __forceinline__ T lds_value(unsigned a) {
-    return *(const __attribute__((address_space(3))) T *)a;
-}
-
 __device__ __forceinline__ float lane_value(float v, int l) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
@@ -350,9 +322,7 @@ __device__ __forceinline__ void partner_pass(const Cell &G, const Pass<R> &S,
             unsigned at = lds_address(L) + 2 * S.ph;
             auto entry = [&](unsigned a) { return (int)lds_value<unsigned short>(min(a, last)); };
             auto site = [&](int s4) {
-                typedef R Vec __attribute__((ext_vector_type(4)));
-                const Vec q = lds_value<Vec>(lds_address(V.p) + s4 * (int)sizeof(R));
-                return Q4<R>{q.x, q.y, q.z, q.w};
+                return lds_q4<R>(lds_address(V.p) + s4 * (int)sizeof(R));
             };
             auto mol = [&](int s4, const Q4<R> &pj) {
                 if constexpr (C::MOL) {
