@@ -47,8 +47,12 @@ template <bool MS, int CAP> struct AdjTile {
     Q4<double> m[MS ? 1 : CAP];  // molecule position, i cell frame (MS: = p)
     Q4<double> c[CAP];  // cotangent on the partner molecule's force
     unsigned short lst[kAdjList][64];
-    int j0[27], pre[28];
-    double shift[27][3];
+    // what the staged sites of a neighbour take: the image shift, and the site of
+    // tile entry e, e + dj
+    struct Nb {
+        double x, y, z;
+        int dj, pad;
+    } nbr[27];
 };
 
 // NLR > 0: the LJ parameter sums of a lane (partner LJ ids < NLR) stay in
@@ -124,27 +128,15 @@ __global__ __launch_bounds__(64) void k_adjoint(AdjArgs a) {
         const int cx = cell % a.g.n[0], cy = (cell / a.g.n[0]) % a.g.n[1],
                   cz = cell / (a.g.n[0] * a.g.n[1]);
         // the 27 neighbour ranges and their prefix (same for every chunk)
-        int nk = 0;
-        if (lane < 27) {
-            Nbr b = neighbour(a.g, cx, cy, cz, lane);
-            int j0 = 0;
-            if (b.ok) {
-                j0 = S.cstart[b.cell];
-                nk = S.cstart[b.cell + 1] - j0;
-            }
-            T.j0[lane] = j0;
-            T.shift[lane][0] = b.s[0];
-            T.shift[lane][1] = b.s[1];
-            T.shift[lane][2] = b.s[2];
+        int nk = 0, j0 = 0;
+        const Nbr b = neighbour(a.g, cx, cy, cz, lane);
+        if (lane < 27 && b.ok) {
+            j0 = S.cstart[b.cell];
+            nk = S.cstart[b.cell + 1] - j0;
         }
-        int incl = nk;
-        for (int o = 1; o < 32; o <<= 1) {
-            int y = __shfl_up(incl, o, 64);
-            if (lane >= o) incl += y;
-        }
-        if (lane < 27) T.pre[lane + 1] = incl;
-        if (lane == 0) T.pre[0] = 0;
-        const int total = __shfl(incl, 26, 64);
+        const int incl = wave_scan(nk), pre = incl - nk;
+        if (lane < 27) T.nbr[lane] = {b.s[0], b.s[1], b.s[2], j0 - pre, 0};
+        const int total = __builtin_amdgcn_readlane(incl, 63);
         __syncthreads();
         for (int chunk = i_begin; chunk < i_end; chunk += 64) {
             const int nI = min(64, i_end - chunk);
@@ -176,11 +168,27 @@ __global__ __launch_bounds__(64) void k_adjoint(AdjArgs a) {
             for (int w = 0; w < NR; ++w) racc[w] = 0.0;
             for (int base = 0; base < total; base += CAP) {
                 const int nst = min(CAP, total - base);
-                for (int t = lane; t < nst; t += 64) {
-                    const int idx = base + t;
-                    const int k = tile_k(T.pre, idx);
-                    const int j = T.j0[k] + (idx - T.pre[k]);
-                    const double sx = T.shift[k][0], sy = T.shift[k][1], sz = T.shift[k][2];
+                // the neighbour of each entry: marks at the neighbours' first
+                // entries (in the lists' bytes) and a maximum scan, as the cell
+                // pair kernels do; with the lists of addresses below 405 -> 370 us
+                // for 500 k one-centre molecules (two LJ ids, VJP)
+                unsigned char *mark = reinterpret_cast<unsigned char *>(T.lst);
+                static_assert(CAP + 3 <= sizeof(T.lst), "marks");
+                for (int z = 4 * lane; z < nst; z += 256)
+                    *reinterpret_cast<unsigned *>(mark + z) = 0u;
+                __syncthreads();
+                if (nk > 0 && pre < base + nst && incl > base)
+                    mark[max(pre - base, 0)] = (unsigned char)(lane + 1);
+                __syncthreads();
+                int carry = 0;
+                for (int t0 = 0; t0 < nst; t0 += 64) {
+                    const int t = t0 + lane;
+                    const int k1 = max(wave_max_scan(t < nst ? mark[t] : 0), carry);
+                    carry = __builtin_amdgcn_readlane(k1, 63);
+                    if (t >= nst) continue;
+                    const typename Tile::Nb nb = T.nbr[k1 - 1];
+                    const int j = nb.dj + base + t;
+                    const double sx = nb.x, sy = nb.y, sz = nb.z;
                     const double w = TI == T_LJ ? (double)S.ljid[j] : S.p[j];
                     T.p[t] = Q4<double>{S.x[j] + sx, S.y[j] + sy, S.z[j] + sz, w};
                     if constexpr (!MS)
@@ -191,24 +199,31 @@ __global__ __launch_bounds__(64) void k_adjoint(AdjArgs a) {
                     }
                 }
                 __syncthreads();
-                int cnt = 0;
+                // lists of LDS addresses of site records; la: the list's end
+                constexpr unsigned MO = MS ? 0 : offsetof(Tile, m) - offsetof(Tile, p),
+                                   CO = offsetof(Tile, c) - offsetof(Tile, p);
+                const unsigned pb = lds_address(T.p), l0 = lds_address(&T.lst[0][lane]);
+                constexpr unsigned ROW = sizeof(T.lst[0]);
+                unsigned la = l0;
                 // stage B: the derivative terms of the listed partners
                 auto drain = [&]() {
-                    int emax = cnt;  // the longest list: a scalar trip count
-                    for (int o = 32; o > 0; o >>= 1) emax = max(emax, __shfl_xor(emax, o, 64));
-                    emax = __builtin_amdgcn_readfirstlane(emax);
-                    for (int e = 0; e < emax; ++e) {
-                        if (e >= cnt) continue;
-                        const int t = T.lst[e][lane];
-                        const Q4<double> pj = T.p[t];
+                    // the longest list: a scalar trip count
+                    const int emax =
+                        __builtin_amdgcn_readlane(wave_max_scan((int)((la - l0) / ROW)), 63);
+                    unsigned lp = l0;
+                    for (int e = 0; e < emax; ++e, lp += ROW) {
+                        if (lp >= la) continue;
+                        const unsigned at = lds_value<unsigned short>(lp);
+                        const Q4<double> pj = lds_q4<double>(at);
                         const double dx = px - pj.x, dy = py - pj.y, dz = pz - pj.z;
                         const double r2 = dx * dx + dy * dy + dz * dz;
+                        if (MS && r2 == 0.0) continue;  // the molecule itself (SingleCellPolicy_)
                         const double r2i = Math<double>::rcp(r2);
                         // (m_i - m_j) . d: r^2 itself where sites are their
                         // molecules' centres
                         double dmd = r2;
                         if constexpr (!MS) {
-                            const Q4<double> mj4 = T.m[t];
+                            const Q4<double> mj4 = lds_q4<double>(at + MO);
                             dmd = (mx - mj4.x) * dx + (my - mj4.y) * dy + (mz - mj4.z) * dz;
                         }
                         double sc, sp;  // the force-derivative factors (VJP only)
@@ -253,7 +268,7 @@ __global__ __launch_bounds__(64) void k_adjoint(AdjArgs a) {
                             sp = -1.5 * qi * qj * r3i * r2i;
                         }
                         if (vjp) {  // wave-uniform: the parameter-only call skips it
-                            const Q4<double> cj = T.c[t];
+                            const Q4<double> cj = lds_q4<double>(at + CO);
                             const double dc[3] = {ci[0] - cj.x, ci[1] - cj.y, ci[2] - cj.z};
                             const double ddc = dx * dc[0] + dy * dc[1] + dz * dc[2];
                             g[0] += sc * dc[0] + 2.0 * sp * dx * ddc;
@@ -261,42 +276,47 @@ __global__ __launch_bounds__(64) void k_adjoint(AdjArgs a) {
                             g[2] += sc * dc[2] + 2.0 * sp * dz * ddc;
                         }
                     }
-                    cnt = 0;
+                    la = l0;
                 };
                 // stage A: molecule-centre cutoff, strictly less; the molecule
-                // itself (distance 0) is skipped (SingleCellPolicy_). Row r
-                // holds candidates ph + r P; rows below full lie inside
+                // itself (distance 0) is skipped (SingleCellPolicy_; MS: in stage
+                // B). Row r holds candidates ph + r P; rows below full lie inside
                 // [0, nst) for every phase, so they run without bounds tests,
                 // kAdjUnroll rows per drain check; every candidate is written
                 // at the end of the list and kept only on a hit
-                auto hit = [&](int m) -> bool {
-                    const Q4<double> q = MS ? T.p[m] : T.m[m];
+                auto hit = [&](unsigned at) -> bool {
+                    const Q4<double> q = lds_q4<double>(at + MO);
                     const double ex = mx - q.x, ey = my - q.y, ez = mz - q.z;
                     const double r2m = ex * ex + ey * ey + ez * ez;
-                    return r2m < rc2 && r2m != 0.0;
+                    return r2m < rc2 && (MS || r2m != 0.0);
                 };
+                auto list = [&](unsigned at, bool h) {
+                    *(__attribute__((address_space(3))) unsigned short *)la = (unsigned short)at;
+                    la += h ? ROW : 0u;
+                };
+                constexpr unsigned REC = sizeof(Q4<double>);
                 const int nsts = __builtin_amdgcn_readfirstlane(nst);
                 const int Ps = __builtin_amdgcn_readfirstlane(P);
                 const int per = (nsts + Ps - 1) / Ps, full = per - 1;
                 int row = 0;
                 for (; row + kAdjUnroll <= full; row += kAdjUnroll) {
-                    if (__any(cnt > kAdjList - kAdjUnroll)) drain();
+                    if (__any(la > l0 + (kAdjList - kAdjUnroll) * ROW)) drain();
+                    unsigned at[kAdjUnroll];
                     bool h[kAdjUnroll];
 #pragma unroll
-                    for (int u = 0; u < kAdjUnroll; ++u) h[u] = hit(ph + (row + u) * P);
-#pragma unroll
                     for (int u = 0; u < kAdjUnroll; ++u) {
-                        T.lst[cnt][lane] = (unsigned short)(ph + (row + u) * P);
-                        cnt += h[u] ? 1 : 0;
+                        at[u] = pb + (unsigned)(ph + (row + u) * P) * REC;
+                        h[u] = hit(at[u]);
                     }
+#pragma unroll
+                    for (int u = 0; u < kAdjUnroll; ++u) list(at[u], h[u]);
                 }
                 for (; row < per; ++row) {  // the last rows, bounds-tested
-                    if (__any(cnt > kAdjList - 1)) drain();
+                    if (__any(la > l0 + (kAdjList - 1) * ROW)) drain();
                     const int m = ph + row * P;
-                    const int mc = min(m, nst - 1);
-                    const bool h = hit(mc) && m < nst;
-                    T.lst[cnt][lane] = (unsigned short)mc;
-                    cnt += h ? 1 : 0;
+                    const unsigned at = pb + (unsigned)min(m, nst - 1) * REC;
+                    const bool h = hit(at) && m < nst;
+                    list(at, h);
                 }
                 drain();
                 __syncthreads();

@@ -25,7 +25,7 @@ template <bool SITES>
 __global__ void k_leapfrog_post_pre(MolArrays, const double *, const double *, const Component *,
                                     int, Reps, double, int, const int *, const int *, double *,
                                     Bins, SiteArrays, SiteArrays, SiteArrays, SiteArrays);
-__global__ void k_reduce_partials(const double *, int, int, int, double *);
+__global__ void k_reduce_partials(const double *, int, double *);
 __global__ void k_fill_int(int *, int, int);
 __global__ void k_bin_count(MolArrays, Reps, int, Bins);
 __global__ void k_bin_scatter(int, const int *, const int *, const int *, int *);
@@ -2092,6 +2092,11 @@ size_t adjoint_table_width(const mdx_context *c) {
     return std::max(nl * 4 * nl, (size_t)c->model.ncomp * kMaxSite * 2);
 }
 
+// The adjoint's one array each way goes with helping threads from 8 MB on (no
+// conversion of the caller's follows that would take their CPUs): 500 k molecules
+// 1700 -> 1280 us for a call.
+constexpr size_t kAdjMany = 8u << 20;
+
 // The adjoint on the given buffers (no allocation): the LJ and charge
 // passes, the per-molecule VJP, the copies back and the symmetric sums.
 int adjoint_run(mdx_context *c, const double *cot, double *dU_deps, double *dU_dsig,
@@ -2105,7 +2110,7 @@ int adjoint_run(mdx_context *c, const double *cot, double *dU_deps, double *dU_d
     const int nsl = c->nsites[T_LJ], nsc = c->nsites[T_C];
     MolArrays &m = c->mol[c->cur];
     if (cot) {
-        HostTransfer tr(c->ring, c->stream, c->device, (size_t)nn * 3 * 8);
+        HostTransfer tr(c->ring, c->stream, c->device, (size_t)nn * 3 * 8, kAdjMany);
         tr.to_device((char *)c->dl_tmp, {{(char *)cot, (size_t)nn * 3 * 8}});
         HIPCHK(c, tr.finish());
         hipLaunchKernelGGL(gather_orig3_kernel(), dim3(nblk(nn)), dim3(kBlock), 0, c->stream, nn,
@@ -2151,8 +2156,8 @@ int adjoint_run(mdx_context *c, const double *cot, double *dU_deps, double *dU_d
                            (t == T_LJ ? (size_t)nl * nl * kAdjPar * 8 : 0);
         hipLaunchKernelGGL(adjoint_kernel(t, nl, t == T_LJ && c->lj_at_origin), dim3(grid), dim3(64), lds, c->stream, a);
         const int width = a.K * a.W;
-        hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(256), 0, c->stream, b.part, grid,
-                           width, grid, t == T_LJ ? out_lj : out_q);
+        hipLaunchKernelGGL(k_reduce_partials, dim3(width), dim3(256), 0, c->stream, b.part, grid,
+                           t == T_LJ ? out_lj : out_q);
     }
     HIPCHK(c, hipGetLastError());
     if (c->timing) HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
@@ -2175,7 +2180,7 @@ int adjoint_run(mdx_context *c, const double *cot, double *dU_deps, double *dU_d
     }
     if (c->timing) HIPCHK(c, hipEventRecord(c->ev[3], c->stream));
     if (vjp) {
-        HostTransfer tr(c->ring, c->stream, c->device, (size_t)nn * 3 * 8);
+        HostTransfer tr(c->ring, c->stream, c->device, (size_t)nn * 3 * 8, kAdjMany);
         tr.to_host((const char *)b.cot, {{(char *)vjp, (size_t)nn * 3 * 8}});
         HIPCHK(c, tr.finish());
     }

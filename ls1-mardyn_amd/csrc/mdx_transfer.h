@@ -79,9 +79,18 @@ struct HostPiece {
 
 class HostTransfer {
   public:
-    HostTransfer(PinnedRing &ring, hipStream_t stream, int device, size_t total)
+    // Two threads from 32 MB on. 150 k molecules (34 MB): 2.4 ms alone, 1.5 with
+    // two, 0.9 with four; 1 M: 6.7 (15.8 into fresh memory), 6.2, 5.6. Below, one
+    // thread is as fast (100 k molecules: 0.73 ms, 0.71 with two) and more of them
+    // lose their CPUs to a caller's own spinning thread pool (a pass with a tensor
+    // conversion behind it: 1.4 ms alone, 2.1 with two, 3.8 with four, 4.8 with
+    // eight).
+    static constexpr size_t kWorkers = 2, kManyBytes = 32u << 20;
+
+    HostTransfer(PinnedRing &ring, hipStream_t stream, int device, size_t total,
+                 size_t many = kManyBytes)
         : ring_(ring), stream_(stream) {
-        const size_t want = ring.mem && total >= kManyBytes ? kWorkers : 0;
+        const size_t want = ring.mem && total >= many ? kWorkers : 0;
         const unsigned hw = std::thread::hardware_concurrency();
         const size_t most = hw > 1 ? hw - 1 : 0;
         try {
@@ -158,13 +167,6 @@ class HostTransfer {
     }
 
   private:
-    // Two threads from 32 MB on. 150 k molecules (34 MB): 2.4 ms alone, 1.5 with
-    // two, 0.9 with four; 1 M: 6.7 (15.8 into fresh memory), 6.2, 5.6. Below, one
-    // thread is as fast (100 k molecules: 0.73 ms, 0.71 with two) and more of them
-    // lose their CPUs to a caller's own spinning thread pool (a pass with a tensor
-    // conversion behind it: 1.4 ms alone, 2.1 with two, 3.8 with four, 4.8 with
-    // eight).
-    static constexpr size_t kWorkers = 2, kManyBytes = 32u << 20;
     // without a ring (no pinned memory left): pageable copies
     void direct(char *dev, const std::vector<HostPiece> &pieces, hipMemcpyKind kind) {
         for (const HostPiece &p : pieces) {
