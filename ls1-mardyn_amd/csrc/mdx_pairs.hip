@@ -52,17 +52,23 @@ template <int TI, typename R, bool MOLSITE, bool MULTI> struct TileCfg {
     static constexpr bool LJID = TI == T_LJ && MULTI;  // several LJ centre types
     // Per-lane hit list entries (LIST) and sites per LDS chunk (CAP). The
     // kernels are bound by VALU issue, so the tile is sized for occupancy
-    // first (160 KB of LDS per CU shared by the wavefronts of its 4 SIMDs,
-    // next to the register limit of each instantiation) and chunk count
-    // second; values measured best on the 4 M-molecule LJ slab (one-centre)
-    // and the 1 M-molecule multi-site mixture (2CLJQ + water). The FP64
-    // tiles that carry molecule positions or orientations keep 16-entry
-    // lists for their larger records.
+    // first (160 KB of LDS per CU in steps of 1280 bytes, shared by the
+    // wavefronts of its 4 SIMDs, next to the register limit of each
+    // instantiation) and chunk count second: each chunk ends with a drain of
+    // half-empty lists. Values measured best on the 1 M-molecule LJ slab and 64
+    // replicas (FP32 one-centre: 414 sites fill the 10240 bytes of 16 blocks per
+    // CU, 316 -> 307 us for the replicas against 352) and on the 1 M-molecule
+    // mixture (2CLJQ + water). The FP32 quadrupole kernel takes the 12800 bytes
+    // of 12 blocks: its 36-cell neighbourhood of charges goes in three chunks
+    // instead of five, 618 -> 576 us (114 sites: 618, 160: 682, 184: 618).
+    // Chunks of equal length cost more than they level (2234 -> 2288 us for all
+    // three). The FP64 tiles that carry molecule positions or orientations keep
+    // 16-entry lists for their larger records.
     static constexpr int LIST = (sizeof(R) == 8 && !(TI == T_LJ && MOLSITE)) ? 16 : 24;
     static constexpr int CAP =
-        TI == T_LJ ? (MOLSITE ? (sizeof(R) == 4 ? 352 : 192) : (sizeof(R) == 4 ? 192 : 112))
+        TI == T_LJ ? (MOLSITE ? (sizeof(R) == 4 ? 414 : 192) : (sizeof(R) == 4 ? 192 : 112))
         : TI == T_C ? (sizeof(R) == 4 ? 112 : 72)
-        : TI == T_Q ? (sizeof(R) == 4 ? 114 : 104)
+        : TI == T_Q ? (sizeof(R) == 4 ? 176 : 104)
                     : (sizeof(R) == 4 ? 192 : 160);
     // Quadrupole i sites are few per cell (one per 2CLJQ molecule) against
     // a neighbourhood of many partner sites, so the kernel takes two cells
@@ -75,14 +81,13 @@ template <int TI, typename R, bool MOLSITE, bool MULTI> struct TileCfg {
     // Minimum waves per SIMD the kernel's registers are allocated for (1: no
     // bound, the compiler's choice). Tiles of at most 10 KB of LDS (lists
     // included) let 16 blocks share a CU, 4 waves per SIMD, when the
-    // registers fit 128: the FP32 quadrupole kernel (114-site tile) and the
-    // FP64 charge kernel (72 sites) get the bound, which makes the compiler
-    // fit them with a few spilled values outside the pair loops; the FP64
-    // multi-site LJ kernel (112 sites) fits without it, and the FP64
-    // quadrupole kernel's 104-site tile (13 KB) reaches 3 waves per SIMD
-    // with its 166 registers. Measured on the mixture against the larger
-    // tiles at fewer waves: FP32 quadrupole kernel -6 %; FP64 LJ -3 %,
-    // charge -4 %, quadrupole -9 %.
+    // registers fit 128: the charge kernels (112 and 72 sites) get the bound,
+    // which makes the compiler fit them with a few spilled values outside the
+    // pair loops (FP32: 129 registers and 1090 us without, 936 with); so does
+    // the FP32 quadrupole kernel, whose larger tile runs 3 waves, for 575 us
+    // against 588 without. The FP64 multi-site LJ kernel (112 sites) fits
+    // without it, and the FP64 quadrupole kernel's 104-site tile (13 KB) reaches
+    // 3 waves per SIMD with its 160 registers.
     static constexpr int WAVES =
         (TI == T_Q && sizeof(R) == 4) || TI == T_C ? 4 : 1;
 };
