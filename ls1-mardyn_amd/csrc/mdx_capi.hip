@@ -893,6 +893,9 @@ void launch_step_end(mdx_context *c, int what) {
     StepEnd e;
     memset(&e, 0, sizeof(e));
     e.macro_part = n_present(c) > 0 ? c->macro_part : nullptr;
+    e.geom = c->d_geoms;
+    e.ncell = c->ncell;
+    for (int t = 0; t < kTypes; ++t) e.present[t] = c->nsites[t] > 0;
     e.lf_part = c->lf_part;
     e.cell_off = c->d_cell_off;
     e.lf_off = c->d_lf_off;
@@ -953,9 +956,11 @@ int launch_traverse(mdx_context *c, double kick = 0.0, bool in_step = false) {
     a.nsmall = c->nsmall;
     a.others = c->nsmall > 0;
     if (c->timing) HIPCHK(c, hipEventRecord(c->ev[0], c->stream));
-    // one [ncell][4] partial array: the first i-site type writes each cell's
+    // the cell kernels' partial array: the first i-site type writes each cell's
     // row, later types add to it (the launches are ordered on the stream)
-    int slot = 0;
+    int slot = 0, nes = 0, last_type = -1;
+    for (int t = 0; t < kTypes; ++t)
+        if (c->nsites[t] > 0) last_type = t;
     for (int t = 0; t < kTypes; ++t) {
         if (c->nsites[t] == 0) continue;
         a.macro_part = c->macro_part;
@@ -972,10 +977,17 @@ int launch_traverse(mdx_context *c, double kick = 0.0, bool in_step = false) {
             PairKernel k = pair_kernel(t, fp32, c->counting, centre, c->model.nlj > 1);
             hipLaunchKernelGGL(k, dim3(grid), dim3(64), 0, c->stream, a);
         }
-        if (c->nsmall > 0) {
+        // the electrostatic types' block kernel: all in one launch, or (timed)
+        // one by one
+        const bool last = t == last_type;
+        if (t != T_LJ) a.es[nes++] = t;
+        if (c->nsmall > 0 && (t == T_LJ || c->timing || last)) {
             const int grid = item_grid(c, c->nsmall, 1, &a.items_per_xcd);
-            PairKernel k = block_kernel(t, fp32, c->counting, centre, c->model.nlj);
-            hipLaunchKernelGGL(k, dim3(grid), dim3(kPairBlock), 0, c->stream, a);
+            PairKernel k = t == T_LJ ? block_kernel_lj(fp32, c->counting, centre, c->model.nlj)
+                                     : block_kernel_es(fp32, c->counting);
+            a.counters = c->d_counters;
+            hipLaunchKernelGGL(k, dim3(grid, std::max(nes, 1)), dim3(kPairBlock), 0, c->stream, a);
+            nes = 0;
         }
         ++slot;
     }
@@ -1110,7 +1122,8 @@ int state_alloc(mdx_context *c, int n) {
         hipLaunchKernelGGL(k_iota, dim3(nblk(n + 1)), dim3(kBlock), 0, c->stream, c->ident, n + 1);
     }
     TRY(alloc_scan(c, std::max(n, c->ncell) + 1));
-    TRY(dalloc(c, &c->macro_part, (size_t)c->ncell * 4, true));
+    // a plane per type where boxes are small (the block kernels)
+    TRY(dalloc(c, &c->macro_part, (size_t)c->ncell * 4 * (c->nsmall > 0 ? kTypes : 1), true));
     // molecule chunks of <= kBlock that never straddle two replicas
     {
         std::vector<int> ch, che, off(1, 0);
@@ -1182,7 +1195,7 @@ int state_setup(mdx_context *c, int64_t n64, const int32_t *cid_host) {
     // A state of the same shape takes the arrays of the one before it (a fit
     // uploads new positions on every call: some 60 allocations and frees, 0.36
     // ms of a 500-molecule upload).
-    std::vector<long> sig = {n, c->ncell, c->nrep, c->point_lj};
+    std::vector<long> sig = {n, c->ncell, c->nrep, c->point_lj, c->nsmall};
     for (int t = 0; t < kTypes; ++t) sig.push_back(c->nsites[t]);
     if (c->nrep > 1) sig.insert(sig.end(), c->rep_n.begin(), c->rep_n.end());
     if (sig != c->state_sig) {

@@ -176,7 +176,10 @@ struct UnpackArgs {
 // The sums of a step (k_step_end): the pair kernels' cell rows and the leapfrog
 // chunks' rows of each replica.
 struct StepEnd {
-    const double *macro_part;      // [ncell][4], or null: no sites, sums 0
+    const double *macro_part;      // [kTypes][ncell][4], or null: no sites, sums 0
+    const Geom *geom;              // [nrep]
+    int ncell;
+    int present[kTypes];           // planes of the small boxes
     const double *lf_part;         // [chunks][4]
     const int *cell_off, *lf_off;  // [nrep + 1] rows of each replica
     double *part;                  // [nrep][kStepBlocks][8] block sums
@@ -200,12 +203,14 @@ struct PairArgs {
     int nsmall;         // cells of small boxes (block kernels: one per work item)
     int items_per_xcd;  // work items of each XCD's contiguous range
     int present[kTypes];
+    int es[kTypes - 1];  // electrostatic block kernel: the i-site type per blockIdx.y
     int ncell;          // global cells
     int cpb;            // cells per work item of the cell kernels
     int others;         // some boxes are small: the cell kernels skip them
-    double *macro_part; // [ncell][4] sums {u6 (LJ), uXpoles, virial, rf}: a work item of
-                        // the cell kernels stores its cells' sums in the row of its last
-                        // non-empty cell (per replica), the block kernels each cell's
+    double *macro_part; // [kTypes][ncell][4] sums {u6 (LJ), uXpoles, virial, rf}. Cell
+                        // kernels: plane 0, a work item's sums in the row of its last
+                        // non-empty cell (per replica). Block kernels: each cell's sums
+                        // in the plane of the i-site type
     int accumulate;     // add to macro_part rows (a later i-site type) instead of writing
     double vscale;      // factor on the written site virial: 1, or 0.5 where the site
                         // arrays are the molecule arrays (calcFM's Vi = 0.5 sum V_site)
@@ -220,6 +225,8 @@ struct PairArgs {
 constexpr int kPairBlock = 256;  // threads per block of the block kernels
 typedef void (*PairKernel)(PairArgs);
 PairKernel pair_kernel(int ti, bool fp32, bool count, bool molsite, bool multi);
-PairKernel block_kernel(int ti, bool fp32, bool count, bool molsite, int nlj);
+// LJ i sites, and the electrostatic types of es[] (one per blockIdx.y)
+PairKernel block_kernel_lj(bool fp32, bool count, bool molsite, int nlj);
+PairKernel block_kernel_es(bool fp32, bool count);
 
 }  // namespace mdx

@@ -1008,7 +1008,14 @@ __global__ __launch_bounds__(256) void k_step_end(StepEnd a) {
             x[3] += hi.y;
         }
     };
-    if ((a.what & kEndMacro) && a.macro_part) rows(a.macro_part, m0, m1, v);
+    if ((a.what & kEndMacro) && a.macro_part) {
+        if (a.geom[r].small) {
+            for (int p = 0; p < kTypes; ++p)
+                if (a.present[p]) rows(a.macro_part + 4 * (size_t)p * a.ncell, m0, m1, v);
+        } else {
+            rows(a.macro_part, m0, m1, v);
+        }
+    }
     if (a.what & kEndLeapfrog) rows(a.lf_part, a.lf_off[r], a.lf_off[r + 1], v + 4);
     __shared__ double red[8][192];
     if (t >= 64)

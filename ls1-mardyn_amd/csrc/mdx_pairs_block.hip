@@ -532,7 +532,7 @@ __device__ __forceinline__ void partner_pass(const Cell &G, const Pass<R> &S,
     if (COUNT) {
         const PairArgs &b = args();
         for (int o = 32; o > 0; o >>= 1) nhit += __shfl_xor(nhit, o, 64);
-        if (lane == 0) atomicAdd(&b.counters[1 + Kind<TI, TJ>::k], nhit);
+        if (lane == 0) atomicAdd(&b.counters[8 * TI + 1 + Kind<TI, TJ>::k], nhit);
     }
 }
 
@@ -716,10 +716,11 @@ __device__ __forceinline__ void pair_cell(BlockShared<TI, R, MOLSITE, MULTI> &T,
     }
     if (wv == 0 && lane == 0) {
         const PairArgs &a = args();
-        double *o = a.macro_part + 4 * (size_t)cell;
-        const double v[4] = {(TI == T_LJ) ? wmac[0] : 0.0, (TI == T_LJ) ? 0.0 : wmac[0], wmac[1],
-                             wmac[2]};
-        for (int k = 0; k < 4; ++k) o[k] = a.accumulate ? o[k] + v[k] : v[k];
+        double *o = a.macro_part + 4 * ((size_t)TI * a.ncell + cell);
+        o[0] = (TI == T_LJ) ? wmac[0] : 0.0;
+        o[1] = (TI == T_LJ) ? 0.0 : wmac[0];
+        o[2] = wmac[1];
+        o[3] = wmac[2];
     }
 }
 
@@ -729,9 +730,8 @@ __device__ __forceinline__ void pair_cell(BlockShared<TI, R, MOLSITE, MULTI> &T,
 // items_per_xcd makes the blocks persistent: each walks its XCD's cells with
 // stride gridDim.x / 8, and every block leaves after its last cell.
 template <int TI, typename R, bool COUNT, bool MOLSITE, int MULTI>
-__global__ __launch_bounds__(64 * kPairWaves) __attribute__((
-    amdgpu_waves_per_eu(BlockCfg<TI, R, MOLSITE, MULTI>::WAVES))) void k_block(PairArgs a) {
-    __shared__ BlockShared<TI, R, MOLSITE, MULTI> T;
+__device__ __forceinline__ void block_cells(const PairArgs &a,
+                                            BlockShared<TI, R, MOLSITE, MULTI> &T) {
     if constexpr (MULTI == kTableLds) {  // (read behind the first staging's barrier)
         const Q4<R> *par;
         if constexpr (sizeof(R) == 8)
@@ -752,33 +752,52 @@ __global__ __launch_bounds__(64 * kPairWaves) __attribute__((
         const int cell = a.R.small_cell ? constant(a.R.small_cell, k) : k;
         pair_cell<TI, R, COUNT, MOLSITE, MULTI>(T, cell, lane, wv, ntest);
     }
-    if (COUNT && lane == 0) atomicAdd(&a.counters[0], ntest);
+    if (COUNT && lane == 0) atomicAdd(&a.counters[8 * TI], ntest);
 }
 
-template <int T, typename R, bool C> PairKernel pick(bool molsite, int nlj) {
-    if constexpr (T == T_LJ) {
-        if (nlj > kTableIds)
-            return molsite ? k_block<T, R, C, true, kTableGlobal> : k_block<T, R, C, false, kTableGlobal>;
-        if (nlj > 1)
-            return molsite ? k_block<T, R, C, true, kTableLds> : k_block<T, R, C, false, kTableLds>;
-        if (molsite) return k_block<T, R, C, true, kTableNone>;
-    }
-    return k_block<T, R, C, false, kTableNone>;
+template <typename R, bool COUNT, bool MOLSITE, int MULTI>
+__global__ __launch_bounds__(64 * kPairWaves) __attribute__((amdgpu_waves_per_eu(
+    BlockCfg<T_LJ, R, MOLSITE, MULTI>::WAVES))) void k_block_lj(PairArgs a) {
+    __shared__ BlockShared<T_LJ, R, MOLSITE, MULTI> T;
+    block_cells<T_LJ, R, COUNT, MOLSITE, MULTI>(a, T);
 }
 
-template <int T> PairKernel pick_t(bool fp32, bool count, bool molsite, int nlj) {
-    if (fp32) return count ? pick<T, float, true>(molsite, nlj) : pick<T, float, false>(molsite, nlj);
-    return count ? pick<T, double, true>(molsite, nlj) : pick<T, double, false>(molsite, nlj);
+// The electrostatic i-site types in one launch, one per blockIdx.y: each alone
+// leaves a chip of 256 CUs with one or two blocks per CU that wait for loads and
+// barriers; together they overlap (9001 mixture molecules FP32, charges and
+// quadrupoles: 24 + 24 -> 30 us; 3001 of all site types FP64, three types: 62 ->
+// 42).
+template <typename R, bool COUNT>
+__global__ __launch_bounds__(64 * kPairWaves) __attribute__((amdgpu_waves_per_eu(
+    BlockCfg<T_C, R, false, kTableNone>::WAVES))) void k_block_es(PairArgs a) {
+    typedef BlockShared<T_C, R, false, kTableNone> TC;
+    typedef BlockShared<T_D, R, false, kTableNone> TD;
+    typedef BlockShared<T_Q, R, false, kTableNone> TQ;
+    static_assert(sizeof(TC) == sizeof(TD) && sizeof(TC) == sizeof(TQ), "one LDS buffer");
+    __shared__ alignas(alignof(TC)) unsigned char buf[sizeof(TC)];
+    const int t = a.es[blockIdx.y];
+    if (t == T_C)
+        block_cells<T_C, R, COUNT, false, kTableNone>(a, *reinterpret_cast<TC *>(buf));
+    else if (t == T_D)
+        block_cells<T_D, R, COUNT, false, kTableNone>(a, *reinterpret_cast<TD *>(buf));
+    else
+        block_cells<T_Q, R, COUNT, false, kTableNone>(a, *reinterpret_cast<TQ *>(buf));
 }
 
-PairKernel block_kernel(int ti, bool fp32, bool count, bool molsite, int nlj) {
-    switch (ti) {
-    case T_LJ: return pick_t<T_LJ>(fp32, count, molsite, nlj);
-    case T_C: return pick_t<T_C>(fp32, count, false, 0);
-    case T_D: return pick_t<T_D>(fp32, count, false, 0);
-    case T_Q: return pick_t<T_Q>(fp32, count, false, 0);
-    }
-    return nullptr;
+template <typename R, bool C> PairKernel pick_lj(bool molsite, int nlj) {
+    if (nlj > kTableIds)
+        return molsite ? k_block_lj<R, C, true, kTableGlobal> : k_block_lj<R, C, false, kTableGlobal>;
+    if (nlj > 1) return molsite ? k_block_lj<R, C, true, kTableLds> : k_block_lj<R, C, false, kTableLds>;
+    return molsite ? k_block_lj<R, C, true, kTableNone> : k_block_lj<R, C, false, kTableNone>;
+}
+
+PairKernel block_kernel_lj(bool fp32, bool count, bool molsite, int nlj) {
+    if (fp32) return count ? pick_lj<float, true>(molsite, nlj) : pick_lj<float, false>(molsite, nlj);
+    return count ? pick_lj<double, true>(molsite, nlj) : pick_lj<double, false>(molsite, nlj);
+}
+PairKernel block_kernel_es(bool fp32, bool count) {
+    if (fp32) return count ? k_block_es<float, true> : k_block_es<float, false>;
+    return count ? k_block_es<double, true> : k_block_es<double, false>;
 }
 
 }  // namespace mdx
