@@ -2074,6 +2074,7 @@ struct AdjBufs {
     double *cot;   // 3 n: the cotangent in the current molecule order
     double *part;  // grid x (largest K * W): per-block parameter tables
     double *out;   // kAdjMaxLJ^2 * 4 + kMaxComp * kMaxSite * 2: reduced tables
+    PinnedRing &ring;
 };
 
 constexpr size_t kAdjOutDoubles = (size_t)kAdjMaxLJ * kAdjMaxLJ * 4 + kMaxComp * kMaxSite * 2;
@@ -2123,7 +2124,7 @@ int adjoint_run(mdx_context *c, const double *cot, double *dU_deps, double *dU_d
     const int nsl = c->nsites[T_LJ], nsc = c->nsites[T_C];
     MolArrays &m = c->mol[c->cur];
     if (cot) {
-        HostTransfer tr(c->ring, c->stream, c->device, (size_t)nn * 3 * 8, kAdjMany);
+        HostTransfer tr(b.ring, c->stream, c->device, (size_t)nn * 3 * 8, kAdjMany);
         tr.to_device((char *)c->dl_tmp, {{(char *)cot, (size_t)nn * 3 * 8}});
         HIPCHK(c, tr.finish());
         hipLaunchKernelGGL(gather_orig3_kernel(), dim3(nblk(nn)), dim3(kBlock), 0, c->stream, nn,
@@ -2193,7 +2194,7 @@ int adjoint_run(mdx_context *c, const double *cot, double *dU_deps, double *dU_d
     }
     if (c->timing) HIPCHK(c, hipEventRecord(c->ev[3], c->stream));
     if (vjp) {
-        HostTransfer tr(c->ring, c->stream, c->device, (size_t)nn * 3 * 8, kAdjMany);
+        HostTransfer tr(b.ring, c->stream, c->device, (size_t)nn * 3 * 8, kAdjMany);
         tr.to_host((const char *)b.cot, {{(char *)vjp, (size_t)nn * 3 * 8}});
         HIPCHK(c, tr.finish());
     }
@@ -2242,7 +2243,7 @@ int mdx_adjoint(mdx_context *c, int64_t n, const double *cot, double *dU_deps, d
         TRY(dalloc(c, &c->adj_out, kAdjOutDoubles, true));
     }
     return adjoint_run(c, cot, dU_deps, dU_dsig, dW_deps, dW_dsig, dU_dq, dW_dq, vjp,
-                       AdjBufs{c->adj_site, c->adj_cot, c->adj_part, c->adj_out});
+                       AdjBufs{c->adj_site, c->adj_cot, c->adj_part, c->adj_out, c->ring});
 }
 
 int mdx_adjoint_noalloc(mdx_context *c, int64_t n, const double *cot, double *dU_deps,
@@ -2264,8 +2265,9 @@ int mdx_adjoint_noalloc(mdx_context *c, int64_t n, const double *cot, double *dU
                         " bytes of scratch, more than the " + std::to_string(kScratchDoubles * 8) +
                         " bytes the library holds per device (use mdx_adjoint)");
     double *s = c->scratch;
+    PinnedRing none;  // plain copies: no events and no threads beside a capture
     return adjoint_run(c, cot, dU_deps, dU_dsig, dW_deps, dW_dsig, dU_dq, dW_dq, vjp,
-                       AdjBufs{s + o_site, s + o_cot, s + o_part, s});
+                       AdjBufs{s + o_site, s + o_cot, s + o_part, s, none});
 }
 
 int mdx_set_counting(mdx_context *c, int enable) {
