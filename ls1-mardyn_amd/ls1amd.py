@@ -252,10 +252,14 @@ class Context:
         """State in upload order (with outflow walls: the surviving molecules,
         ids tell which). keys: the arrays wanted (all of r, v, q, L, F, M, Vi,
         ids by default)."""
-        n = self.molecule_count() if self.open else self.n
         names = ("r", "v", "q", "L", "F", "M", "Vi", "ids")
+        keys = names if keys is None else tuple(keys)
+        unknown = [k for k in keys if k not in names]
+        if unknown:  # nothing would fill them
+            raise ValueError(f"download: no arrays {unknown}; there are {list(names)}")
+        n = self.molecule_count() if self.open else self.n
         out = {k: np.empty(n, np.uint64) if k == "ids" else np.empty((n, 4 if k == "q" else 3))
-               for k in (names if keys is None else keys)}
+               for k in keys}
         self._chk(self.L.mdx_download(self.h, n, *(_ptr(out.get(k)) for k in names)),
                   "mdx_download")
         return out
