@@ -270,8 +270,10 @@ int mdx_counters(mdx_context *ctx, int64_t *out);
  * FlopCounter counts one processor over all types, FlopCounter.cpp:19-76). */
 int mdx_kernel_stats(mdx_context *ctx, double *ms, int64_t *counters);
 
-/* Device-resident variants for callers that keep the state in HBM: device
- * pointers to n doubles / ints laid out as in mdx_upload. */
+/* Device-resident variant for callers that keep the state in HBM: device
+ * pointers, structure of arrays (r = [x(n) | y(n) | z(n)], q = [w | x | y | z],
+ * cid n ints). Waits for all work queued on the device, on any stream, before it
+ * reads them, and has read them when it returns: the caller orders nothing. */
 int mdx_upload_device(mdx_context *ctx, int64_t n, const double *r, const double *v,
                       const double *q, const double *L, const int32_t *cid);
 

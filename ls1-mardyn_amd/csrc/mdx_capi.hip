@@ -1635,6 +1635,9 @@ int mdx_upload_device(mdx_context *c, int64_t n, const double *r, const double *
     if (!c || !r || !v || !q || !L || !cid) return MDX_ERR_ARG;
     TRY(need(c, true, true, false));
     HIPCHK(c, hipSetDevice(c->device));
+    // the arrays may come from work on streams that the context's stream is not
+    // ordered behind
+    HIPCHK(c, hipDeviceSynchronize());
     std::vector<int32_t> hc((size_t)n);
     HIPCHK(c, hipMemcpy(hc.data(), cid, (size_t)n * 4, hipMemcpyDeviceToHost));
     TRY(state_setup(c, n, hc.data()));
