@@ -173,6 +173,7 @@ struct mdx_context {
     int site_forms = 0;  // site record forms built for the current re-bin (1 FP64, 2 FP32)
     double *macro_part = nullptr, *lf_part = nullptr, *red = nullptr, *step_out = nullptr;
     double *end_part = nullptr;  // k_step_end's block sums, tickets and step counts
+    int end_blocks = 1;          // its blocks for the replica with the most cells
     int *end_ticket = nullptr, *step_idx = nullptr;
     int cap_steps = 0;
     unsigned long long *d_counters = nullptr;
@@ -608,6 +609,9 @@ int upload_thermo(mdx_context *c) {
 // Replica geometries on the device; reduction buffers sized for nrep.
 int upload_reps(mdx_context *c) {
     const int R = c->nrep;
+    int most = 0;
+    for (int r = 0; r < R; ++r) most = std::max(most, c->cell_off[r + 1] - c->cell_off[r]);
+    c->end_blocks = std::max(1, std::min(kStepBlocks, (most + kStepRows - 1) / kStepRows));
     TRY(dalloc(c, &c->d_geoms, R));
     TRY(dalloc(c, &c->d_cell_off, R + 1));
     TRY(dalloc(c, &c->red, 8 * (size_t)R));
@@ -910,10 +914,8 @@ void launch_step_end(mdx_context *c, int what) {
     e.nrep = c->nrep;
     e.heuristics = c->heuristics;
     e.what = what;
-    int cells = 0;
-    for (int r = 0; r < c->nrep; ++r) cells = std::max(cells, c->cell_off[r + 1] - c->cell_off[r]);
-    const int nb = std::max(1, std::min(kStepBlocks, (cells + kStepRows - 1) / kStepRows));
-    hipLaunchKernelGGL(k_step_end, dim3(nb, c->nrep), dim3(256), 0, c->stream, e);
+    // (replicas on x: a batch may have more than the 65535 blocks that y takes)
+    hipLaunchKernelGGL(k_step_end, dim3(c->nrep, c->end_blocks), dim3(256), 0, c->stream, e);
 }
 
 // kick != 0 (reduced-memory mode): the pair kernel adds kick * F to the

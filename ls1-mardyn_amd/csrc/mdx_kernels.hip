@@ -989,10 +989,10 @@ __global__ __launch_bounds__(256) void k_velocity_scale(MolArrays s, double *F, 
 // that takes its last ticket, from the block sums in block order. Thread t of a
 // block adds rows t, t + 256, ..., the threads' sums go through one tree.
 __global__ __launch_bounds__(256) void k_step_end(StepEnd a) {
-    const int r = blockIdx.y, t = threadIdx.x;
+    const int r = blockIdx.x, t = threadIdx.x;
     const int m0 = a.cell_off[r], m1 = a.cell_off[r + 1];
     const int nb = max(1, min(kStepBlocks, (m1 - m0 + kStepRows - 1) / kStepRows));
-    const int b = blockIdx.x;
+    const int b = blockIdx.y;
     if (b >= nb) return;
     double v[8];
     for (int k = 0; k < 8; ++k) v[k] = 0.0;
