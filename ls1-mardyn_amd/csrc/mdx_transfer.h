@@ -22,9 +22,10 @@
 
 namespace mdx {
 
-// A context's ring: kSlots chunks of kChunk bytes, made on first use. 176 MB into
-// fresh 4 KB pages with 8 threads: 9.7 ms with 8 x 2 MB, 12.0 with 8 x 0.5 MB, 15
-// with 4 x 2 MB.
+// A context's ring: up to kSlots chunks of kChunk bytes, as many as the context's
+// largest transfer so far fills, made on first use and held while the context
+// lives. 176 MB into fresh 4 KB pages with 8 threads: 9.7 ms with 8 x 2 MB, 12.0
+// with 8 x 0.5 MB, 15 with 4 x 2 MB.
 struct PinnedRing {
     static constexpr size_t kChunk = 2u << 20;
     static constexpr int kSlots = 8;
@@ -33,14 +34,21 @@ struct PinnedRing {
     size_t size = 0;
     hipEvent_t ev[kSlots] = {};
 
-    // For transfers of at most `need` bytes in all: one slot of kSmall bytes for
-    // the small states (16 MB and their events take 0.1 to 0.2 ms).
+    // Bytes held for transfers of at most `need` bytes in all: one slot of kSmall
+    // bytes for the small states (16 MB and their events take 0.1 to 0.2 ms), else
+    // no more chunks than the transfer has.
+    static constexpr size_t bytes(size_t need) {
+        if (need <= kSmall) return kSmall;
+        const size_t chunks = need / kChunk + (need % kChunk != 0);
+        return kChunk * (chunks < (size_t)kSlots ? chunks : (size_t)kSlots);
+    }
     hipError_t open(size_t need) {
-        need = need <= kSmall ? kSmall : kChunk * kSlots;
+        need = bytes(need);
         if (mem && size >= need) return hipSuccess;
         if (mem) (void)hipHostFree(mem);
         mem = dev = nullptr;
-        for (int k = 0; k < (need > kSmall ? kSlots : 1); ++k)
+        size = need;
+        for (int k = 0; k < slots(); ++k)
             if (!ev[k]) {
                 const hipError_t r = hipEventCreateWithFlags(&ev[k], hipEventDisableTiming);
                 if (r != hipSuccess) return r;
@@ -56,10 +64,9 @@ struct PinnedRing {
         }
         mem = (char *)p;
         dev = (char *)d;
-        size = need;
         return hipSuccess;
     }
-    int slots() const { return size > kSmall ? kSlots : 1; }
+    int slots() const { return size > kSmall ? (int)(size / kChunk) : 1; }
     void close() {
         if (mem) (void)hipHostFree(mem);
         for (auto &e : ev)
