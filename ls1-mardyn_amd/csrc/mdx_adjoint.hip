@@ -46,7 +46,7 @@ template <bool MS, int CAP> struct AdjTile {
     Q4<double> p[CAP];  // site position, i cell frame; w = LJ id or charge
     Q4<double> m[MS ? 1 : CAP];  // molecule position, i cell frame (MS: = p)
     Q4<double> c[CAP];  // cotangent on the partner molecule's force
-    unsigned short lst[kAdjList][64];
+    alignas(4) unsigned short lst[kAdjList][64];  // hit lists, or the staging's marks
     // what the staged sites of a neighbour take: the image shift, and the site of
     // tile entry e, e + dj
     struct Nb {

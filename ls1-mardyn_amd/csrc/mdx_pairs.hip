@@ -101,7 +101,9 @@ template <int TI, typename R, bool MOLSITE, bool MULTI> struct Tile {
     static constexpr int SLOT =
         (int)sizeof(Q4<R>) * (1 + C::MOL + C::ORI) + (C::MOL && TI != T_LJ ? 3 : 0);
     alignas(32) unsigned char raw[C::CAP * SLOT];
-    unsigned short lst[C::LIST][64];  // per-lane hit lists (LDS addresses of site records)
+    // per-lane hit lists (LDS addresses of site records); the staging's marks, which
+    // are cleared a word at a time, lie in the same bytes
+    alignas(4) unsigned short lst[C::LIST][64];
     int pre[C::NB + 1];               // first tile entry of each neighbour
     NbrRec<R> nbr[C::NB];
 };
@@ -245,7 +247,8 @@ __device__ __forceinline__ void partner_pass(const PairArgs &a, const Geom &g, i
         // by DPP: 1 M-molecule slab FP32 397 -> 355 us, FP64 496 -> 440; 1 M
         // mixture, LJ 842 -> 800, charges 973 -> 936, quadrupoles 706 -> 653.
         unsigned char *mark = reinterpret_cast<unsigned char *>(T.lst);
-        static_assert(PT::CAP <= sizeof(T.lst), "marks");
+        static_assert(PT::CAP + 3 <= sizeof(T.lst), "marks");
+        static_assert(sizeof(T) < 65536, "LDS addresses in 16 bits");
         for (int z = 4 * lane; z < nst; z += 256) *reinterpret_cast<unsigned *>(mark + z) = 0u;
         __syncthreads();
         if (nk > 0 && pre < base + nst && incl > base)
