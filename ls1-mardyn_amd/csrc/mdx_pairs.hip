@@ -717,13 +717,20 @@ __global__ __launch_bounds__(64) __attribute__((
                 // edge exceeds the cutoff: the 9 cells of the common
                 // neighbourhood that are not neighbours of one of the two are
                 // then at least a cell edge, more than rc, from its sites, so
-                // testing them adds no pair that ls1's traversal leaves out
+                // testing them adds no pair that ls1's traversal leaves out.
+                // The cells 0 and 1, 2 and 3, ... of a row go together wherever
+                // the row lies in the launch (the item that holds the first one
+                // takes both), so a replica gives the bits that it gives alone
                 const Geom &g = a.R.geom[rep];
-                const int local = cell - a.R.cell_off[rep];
+                const int x = (cell - a.R.cell_off[rep]) % g.n[0];
                 const double rc2 = TI == T_LJ ? a.rclj2 : a.rc2;
-                if (cell + 1 < c1 && local % g.n[0] + 1 < g.n[0] &&
-                    g.cl[0] * g.cl[0] > rc2 * (1.0 + 1e-9))
-                    span = 2;
+                if (g.cl[0] * g.cl[0] > rc2 * (1.0 + 1e-9)) {
+                    if (x & 1) {
+                        ++cell;
+                        continue;
+                    }
+                    if (x + 1 < g.n[0]) span = 2;
+                }
             }
             if (pair_cell<TI, R, COUNT, MOLSITE, MULTI>(a, T, cell, span, lane, ntest, wmac))
                 last = cell + span - 1;
