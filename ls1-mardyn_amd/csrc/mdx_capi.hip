@@ -60,17 +60,24 @@ using namespace mdx;
 namespace {
 thread_local std::string g_create_error;
 constexpr int kBlock = 256;
-// Boxes of at most this many cells (one-centre systems: kSmallCellsPoint) run
-// the block pair kernels, four waves per cell. A box alone gains up to 512
-// cells and beyond (9001 mixture molecules, 512 cells, FP32: 310 -> 75 us; 500 LJ
-// molecules, 64 cells: 34 -> 13.5 us), but a batch of boxes fills the chip, where
-// a cell kernel does less work per pair, and the choice may depend on the box
-// alone (a replica gives the bits it gives alone). Full batches, block kernel
-// against cell kernel: multi-site 64 x 4000 molecules 924 / 914 us, 64 x 16000
-// (beyond the line) 3760 / 2613; one-centre 512 x 500 (64 cells) 175 / 113, 512
-// x 1500 (125 cells) 607 / 251: the one-centre line lies where a lone box gains
-// more than a full batch loses.
-constexpr long kSmallCells = 512, kSmallCellsPoint = 64;
+// Boxes of multi-site molecules with at most kSmallCells cells and, on average, at
+// least kSmallSites sites per cell and site type present run the block pair kernels,
+// four waves per cell (cells larger than kSmallVolume rc^3 count by volume). The
+// choice may depend on the box alone (a replica gives the bits it gives alone), so
+// it weighs a lone box, which leaves the chip idle, against a full batch of such
+// boxes, where the kernel that does less work per pair wins: what the block kernel
+// costs per cell pays off in dense cells only. us a step, block / cell kernel:
+//   2CLJQ + water mixture, FP32     alone      batch of 400 k molecules
+//    18 molecules a cell, 64 cells  106 / 298  1429 / 1341
+//    18 molecules, 512 cells        120 / 389  1409 / 1362
+//    30 molecules, 512 cells        185 / 674  1820 / 2086
+//    10 molecules, 512 cells         85 / 165  1590 /  882  (beyond the line)
+// FP64, 18 molecules, 512 cells: 147 / 516 and 2304 / 2335; water alone, FP32, 18
+// and 30 molecules: 136 / 275 and 1534 / 1221, 229 / 474 and 2279 / 1802. Boxes of
+// one-centre molecules lose in every batch (512 x 500 molecules: 167 / 104 us of
+// pair kernel FP32, 186 / 147 FP64; 512 x 60: 87 / 38) for 12 us against 25 alone.
+constexpr long kSmallCells = 512;
+constexpr double kSmallSites = 20.0, kSmallVolume = 1.5;
 inline int nblk(long n, int b = kBlock) { return (int)std::max<long>(1, (n + b - 1) / b); }
 
 // Scratch of the entry points that allocate nothing (mdx_adjoint_noalloc):
@@ -465,7 +472,7 @@ int make_geom(mdx_context *c, const double *box, double rc, int periodic, int ce
         g.reflect[d] = 0;
     }
     g.wall_rc = rc;
-    g.small = ncell <= (c->point_lj ? kSmallCellsPoint : kSmallCells);
+    g.small = 0;  // (upload: small_boxes)
     ncell_out = ncell;
     return MDX_OK;
 }
@@ -611,6 +618,7 @@ int upload_reps(mdx_context *c) {
     const int R = c->nrep;
     int most = 0;
     for (int r = 0; r < R; ++r) most = std::max(most, c->cell_off[r + 1] - c->cell_off[r]);
+    c->state_sig.clear();  // (no state: what is left of one belongs to other boxes)
     c->end_blocks = std::max(1, std::min(kStepBlocks, (most + kStepRows - 1) / kStepRows));
     TRY(dalloc(c, &c->d_geoms, R));
     TRY(dalloc(c, &c->d_cell_off, R + 1));
@@ -631,16 +639,6 @@ int upload_reps(mdx_context *c) {
             for (int k = c->cell_off[r]; k < c->cell_off[r + 1]; ++k) cr[k] = r;
         TRY(dalloc(c, &c->d_cell_rep, c->ncell));
         HIPCHK(c, hipMemcpy(c->d_cell_rep, cr.data(), 4 * cr.size(), hipMemcpyHostToDevice));
-    }
-    std::vector<int> small;
-    for (int r = 0; r < R; ++r)
-        if (c->geoms[r].small)
-            for (int k = c->cell_off[r]; k < c->cell_off[r + 1]; ++k) small.push_back(k);
-    c->nsmall = (int)small.size();
-    c->d_small_cell = nullptr;
-    if (c->nsmall > 0 && c->nsmall < c->ncell) {
-        TRY(dalloc(c, &c->d_small_cell, small.size()));
-        HIPCHK(c, hipMemcpy(c->d_small_cell, small.data(), 4 * small.size(), hipMemcpyHostToDevice));
     }
     return MDX_OK;
 }
@@ -1097,8 +1095,14 @@ int ensure_steps(mdx_context *c, int nsteps) {
     return MDX_OK;
 }
 
-// The state's arrays for n molecules.
-int state_alloc(mdx_context *c, int n) {
+// The state's arrays for n molecules. small: the global cells of the small boxes.
+int state_alloc(mdx_context *c, int n, const std::vector<int> &small) {
+    c->nsmall = (int)small.size();
+    c->d_small_cell = nullptr;
+    if (c->nsmall > 0 && c->nsmall < c->ncell) {
+        TRY(dalloc(c, &c->d_small_cell, small.size(), true));
+        HIPCHK(c, hipMemcpy(c->d_small_cell, small.data(), 4 * small.size(), hipMemcpyHostToDevice));
+    }
     TRY(alloc_mol(c, c->mol[0], n));
     TRY(alloc_mol(c, c->mol[1], n, c->point_lj ? &c->mol[0] : nullptr));
     TRY(dalloc(c, &c->F, 3 * (size_t)n, true));
@@ -1170,6 +1174,18 @@ int state_alloc(mdx_context *c, int n) {
     return MDX_OK;
 }
 
+// Whether a box with nsites sites of each type is small: the block pair kernels'.
+bool small_box(const mdx_context *c, const Geom &g, const long (&nsites)[kTypes]) {
+    const long ncell = (long)g.n[0] * g.n[1] * g.n[2];
+    if (c->point_lj || ncell > kSmallCells) return false;
+    long sites = 0;
+    int types = 0;
+    for (int t = 0; t < kTypes; ++t) sites += nsites[t], types += nsites[t] > 0;
+    const double cells =
+        std::max((double)ncell, g.L[0] * g.L[1] * g.L[2] / (kSmallVolume * c->rc * c->rc * c->rc));
+    return sites > 0 && sites >= kSmallSites * types * cells;
+}
+
 int state_setup(mdx_context *c, int64_t n64, const int32_t *cid_host) {
     if (n64 <= 0 || n64 > (1 << 27)) return fail(c, MDX_ERR_ARG, "molecule count out of range");
     if (c->nrep > 1) {
@@ -1178,11 +1194,25 @@ int state_setup(mdx_context *c, int64_t n64, const int32_t *cid_host) {
         if (tot != n64) return fail(c, MDX_ERR_ARG, "n differs from the sum of replica counts");
     }
     const int n = (int)n64;
+    // molecules of each component in each box, the sites of all and the small boxes
     long nsites[kTypes] = {0, 0, 0, 0};
-    for (int i = 0; i < n; ++i) {
-        int k = cid_host[i];
-        if (k < 0 || k >= c->model.ncomp) return fail(c, MDX_ERR_ARG, "component id out of range");
-        for (int t = 0; t < kTypes; ++t) nsites[t] += c->model.comp[k].n[t];
+    std::vector<char> small((size_t)c->nrep);
+    std::vector<int> small_cells;
+    for (int64_t r = 0, i = 0; r < c->nrep; ++r) {
+        long mols[4][kMaxComp] = {}, box[kTypes] = {0, 0, 0, 0};
+        for (const int64_t i1 = c->nrep > 1 ? i + c->rep_n[r] : n64; i < i1; ++i) {
+            const int k = cid_host[i];
+            if (k < 0 || k >= c->model.ncomp)
+                return fail(c, MDX_ERR_ARG, "component id out of range");
+            ++mols[i & 3][k];
+        }
+        for (int k = 0; k < c->model.ncomp; ++k)
+            for (int t = 0; t < kTypes; ++t)
+                box[t] += (mols[0][k] + mols[1][k] + mols[2][k] + mols[3][k]) * c->model.comp[k].n[t];
+        for (int t = 0; t < kTypes; ++t) nsites[t] += box[t];
+        small[r] = small_box(c, c->geoms[r], box);
+        if (small[r])
+            for (int k = c->cell_off[r]; k < c->cell_off[r + 1]; ++k) small_cells.push_back(k);
     }
     for (int t = 0; t < kTypes; ++t)
         if (nsites[t] >= (1 << 27)) return fail(c, MDX_ERR_CAPACITY, "too many sites");
@@ -1197,14 +1227,18 @@ int state_setup(mdx_context *c, int64_t n64, const int32_t *cid_host) {
     // A state of the same shape takes the arrays of the one before it (a fit
     // uploads new positions on every call: some 60 allocations and frees, 0.36
     // ms of a 500-molecule upload).
-    std::vector<long> sig = {n, c->ncell, c->nrep, c->point_lj, c->nsmall};
+    std::vector<long> sig = {n, c->ncell, c->nrep, c->point_lj};
     for (int t = 0; t < kTypes; ++t) sig.push_back(c->nsites[t]);
     if (c->nrep > 1) sig.insert(sig.end(), c->rep_n.begin(), c->rep_n.end());
+    sig.insert(sig.end(), small.begin(), small.end());
     if (sig != c->state_sig) {
         c->state_sig.clear();
         c->have_state = false;
         free_list(c->state_allocs);
-        TRY(state_alloc(c, n));
+        for (int r = 0; r < c->nrep; ++r) c->geoms[r].small = small[r];
+        HIPCHK(c, hipMemcpy(c->d_geoms, c->geoms.data(), sizeof(Geom) * c->nrep,
+                            hipMemcpyHostToDevice));
+        TRY(state_alloc(c, n, small_cells));
         c->state_sig = sig;
     }
     if (c->ring.open(22 * sizeof(double) * (size_t)n) != hipSuccess) (void)hipGetLastError();  // copies then are pageable

@@ -55,7 +55,7 @@ struct Geom {
                        // next re-bin moves them behind the last cell)
     double wall_rc;    // width of the wall slab checked for leaving molecules (rc)
     double rc2, rclj2, epsRFInvrc3;
-    int small;         // few cells: the block pair kernels' (mdx_pairs_block.hip)
+    int small;         // the block pair kernels (mdx_pairs_block.hip), set at the upload
 };
 
 // Site arrays of one type (device pointers).

@@ -1,7 +1,7 @@
 // mdx_pairs.hip -- site-pair traversal kernels (gfx950, wave64, no MFMA).
 //
-// The cell kernels, for boxes of many cells; mdx_pairs_block.hip holds the block
-// kernels of small boxes.
+// The cell kernels; mdx_pairs_block.hip holds the block kernels of small dense
+// boxes.
 //
 // The ten site-pair loops of VectorizedCellProcessor::_calculatePairs
 // (VectorizedCellProcessor.cpp:794-2730) with the seven bodies _loopBodyLJ ..

@@ -10,13 +10,13 @@
 // sites then share the list's entries among their lanes evenly. The cell
 // kernels test per site and leave a lane the hits of its own candidates.
 //
-// Small boxes are bound by latency (a few hundred cells leave most of the 1024
+// A small box alone is bound by latency (a few hundred cells leave most of the 1024
 // SIMDs one wave or none, and a cell kernel's wave walks its whole
 // neighbourhood alone): four waves per cell and lists shared evenly cut that
-// chain. Time of all pair kernels, cell -> block: 500 LJ molecules, FP64: 34 ->
-// 13.5 us; 9001 molecules of the 2CLJQ + water mixture (512 cells), FP32: 310 ->
-// 75, FP64: 376 -> 93; 3001 molecules of all site types, FP64: 112 -> 74. A
-// full chip is bound by VALU issue instead, and there the cell kernels win.
+// chain. Time of all pair kernels, cell -> block: 9001 molecules of the 2CLJQ + water
+// mixture (512 cells), FP32: 310 -> 75, FP64: 376 -> 93. A full chip is bound by VALU
+// issue instead, and there the cell kernels win unless the cells are dense (the
+// rule and both sides' figures stand with kSmallSites in mdx_capi.hip).
 #include "mdx_pair_common.h"
 
 namespace mdx {
@@ -679,23 +679,9 @@ __device__ __forceinline__ void pair_cell(BlockShared<TI, R, MOLSITE, MULTI> &T,
                 if (s.P > 1)
                     fold_phases<TI>(reinterpret_cast<double *>(T.lst[wv]), s.nI, s.P, own, lane, acc);
                 const int i = s.I.idx;
-                if (own && a.kvx) {
-                    // VCP1CLJRMM (VCP1CLJRMM.cpp:300-362): the site's force, times
-                    // dt/m, goes straight into its molecule's velocity
-                    a.kvx[i] = __dadd_rn(a.kvx[i], __dmul_rn(acc.f[0], a.kick));
-                    a.kvy[i] = __dadd_rn(a.kvy[i], __dmul_rn(acc.f[1], a.kick));
-                    a.kvz[i] = __dadd_rn(a.kvz[i], __dmul_rn(acc.f[2], a.kick));
-                } else if (own) {
+                if (own) {
                     S.Fx[i] = acc.f[0]; S.Fy[i] = acc.f[1]; S.Fz[i] = acc.f[2];
-                    double vv[3] = {__dmul_rn(a.vscale, acc.v[0]), __dmul_rn(a.vscale, acc.v[1]),
-                                    __dmul_rn(a.vscale, acc.v[2])};
-                    if (a.thermo) {  // Homogeneous.cpp:139-145, then calcFM's own sum
-                        const double w = constant(a.thermo, kThermoW * rep + kThVi);
-                        for (int k = 0; k < 3; ++k) vv[k] = __dadd_rn(vv[k], w);
-                    }
-                    S.Vx[i] = vv[0];
-                    S.Vy[i] = vv[1];
-                    S.Vz[i] = vv[2];
+                    S.Vx[i] = acc.v[0]; S.Vy[i] = acc.v[1]; S.Vz[i] = acc.v[2];
                     if constexpr (TI >= T_D) {
                         S.Mx[i] = acc.m[0]; S.My[i] = acc.m[1]; S.Mz[i] = acc.m[2];
                     }
