@@ -28,10 +28,10 @@ template <int TI, typename R, bool MOLSITE, int MULTI> struct BlockCfg {
     static constexpr bool LJID = TI == T_LJ && MULTI != kTableNone;  // several LJ centre types
     static constexpr bool F32 = sizeof(R) == 4;
     // Tile bytes, list entries per wave and rows of 64 candidates a wave keeps
-    // in registers. The LDS of a block lets four (one-centre FP32: eight)
-    // blocks share a CU, the register bound (WAVES) as many waves per SIMD; the
-    // FP64 multi-site kernels fit three waves (at four they spill: 842 -> 1017 us
-    // on a full chip).
+    // in registers. The register bound is WAVES waves per SIMD, and the LDS of a
+    // block (BlockShared) lets as many blocks of four waves share a CU; the FP64
+    // kernels with molecule records fit three waves (at four they spill: 842 ->
+    // 1017 us on a full chip).
     static constexpr int RAW = MOLSITE ? (F32 ? 10752 : 21504) : 32768;
     static constexpr int LCAP = MOLSITE ? 1280 : 768;
     // i sites per pass (the list entries hold a row of 64 hits for each): 12
@@ -50,6 +50,8 @@ template <int TI, typename R, bool MOLSITE, int MULTI> struct BlockShared {
     double mac[kPairWaves][3];
     Q4<R> tab[MULTI == kTableLds ? kTableIds * kTableIds : 1];
 };
+// blocks of LDS size `bytes` (given out in steps of 1280) that share a CU
+constexpr int blocks_per_cu(size_t bytes) { return (int)(160 * 1024 / ((bytes + 1279) / 1280 * 1280)); }
 
 // The records of one partner pass (partner type TJ) in a tile's bytes: p site
 // position (w = charge / moment or LJ table column), m molecule position, e
@@ -60,7 +62,7 @@ template <int TI, int TJ, typename R, bool MOLSITE, int MULTI> struct BlockTile 
     static constexpr bool ORIJ = TI != T_LJ && TJ >= T_D;
     static constexpr int REC = (int)sizeof(R) * (4 + 3 * C::MOL + 3 * ORIJ);
     static constexpr int CAP = C::RAW / REC / 16 * 16;
-    static_assert(CAP >= 64 && CAP < 65536, "tile capacity");
+    static_assert(CAP >= 64 && 4 * CAP < 65536, "tile capacity, 4 * index in 16 bits");
     Q4<R> *p;
     R *mx, *my, *mz, *ex, *ey, *ez;
     __device__ __forceinline__ explicit BlockTile(unsigned char *raw) {
@@ -745,6 +747,7 @@ template <typename R, bool COUNT, bool MOLSITE, int MULTI>
 __global__ __launch_bounds__(64 * kPairWaves) __attribute__((amdgpu_waves_per_eu(
     BlockCfg<T_LJ, R, MOLSITE, MULTI>::WAVES))) void k_block_lj(PairArgs a) {
     __shared__ BlockShared<T_LJ, R, MOLSITE, MULTI> T;
+    static_assert(blocks_per_cu(sizeof(T)) >= BlockCfg<T_LJ, R, MOLSITE, MULTI>::WAVES, "occupancy");
     block_cells<T_LJ, R, COUNT, MOLSITE, MULTI>(a, T);
 }
 
@@ -760,6 +763,7 @@ __global__ __launch_bounds__(64 * kPairWaves) __attribute__((amdgpu_waves_per_eu
     typedef BlockShared<T_D, R, false, kTableNone> TD;
     typedef BlockShared<T_Q, R, false, kTableNone> TQ;
     static_assert(sizeof(TC) == sizeof(TD) && sizeof(TC) == sizeof(TQ), "one LDS buffer");
+    static_assert(blocks_per_cu(sizeof(TC)) >= BlockCfg<T_C, R, false, kTableNone>::WAVES, "occupancy");
     __shared__ alignas(alignof(TC)) unsigned char buf[sizeof(TC)];
     const int t = a.es[blockIdx.y];
     if (t == T_C)
