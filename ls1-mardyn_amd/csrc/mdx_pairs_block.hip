@@ -490,12 +490,9 @@ __device__ __forceinline__ void partner_pass(const Cell &G, const Pass<R> &S,
                         (unsigned)(m[r] >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m[r], 0u));
                     unsigned end = lb + 2 * cnt;
                     asm("" : "+s"(end));  // scalar: one vector operation for the address
-                    // the row's hits store their entry behind the list's end:
-                    // one store under the hit mask, without the branch a
-                    // conditional store gets (all lanes are active here)
-                    asm volatile("s_mov_b64 exec, %2\n\tds_write_b16 %0, %1\n\ts_mov_b64 exec, -1"
-                                 :
-                                 : "v"((at << 1) + end), "v"(jid[r]), "s"(m[r]));
+                    // the row's hits store their entry behind the list's end
+                    if (__builtin_amdgcn_inverse_ballot_w64(m[r]))
+                        *(__attribute__((address_space(3))) unsigned short *)((at << 1) + end) = (unsigned short)jid[r];
                     cnt += pop;
                 };
                 int tot = 0, pop[C::RG];
