@@ -801,11 +801,11 @@ int rebin_forms(const mdx_context *c) {
     return c->precision == MDX_PREC_FP32_FP64ACC ? 2 : 1;
 }
 
+Bins bins(const mdx_context *c) { return {c->cell, c->rank, c->count, c->ls1id}; }
+
 // Re-bin (LinkedCells::update + exchangeMolecules' periodic wrap, which
 // leapfrog_pre already applied) and SoA cache build (setupSoACache).
 // counted: the drift has binned the molecules already (bins()).
-Bins bins(const mdx_context *c) { return {c->cell, c->rank, c->count, c->ls1id}; }
-
 int launch_update(mdx_context *c, bool counted = false) {
     const int n = c->n;
     if (c->point_lj) ++c->q_renorm;
@@ -2146,8 +2146,10 @@ size_t adjoint_table_width(const mdx_context *c) {
 }
 
 // The adjoint's one array each way goes with helping threads from 8 MB on (no
-// conversion of the caller's follows that would take their CPUs): 500 k molecules
-// 1700 -> 1280 us for a call.
+// conversion of the caller's follows that would take their CPUs). us a call without
+// / with two: 1.2 MB 289 / 368, 3 MB 497 / 522, 6 MB 834 / 777, 8 MB 1044 / 934, 12
+// MB (500 k molecules) 1498 / 1266: they pay from 4 MB on, and take two CPUs for it,
+// so the line lies where the gain is a tenth.
 constexpr size_t kAdjMany = 8u << 20;
 
 // The adjoint on the given buffers (no allocation): the LJ and charge

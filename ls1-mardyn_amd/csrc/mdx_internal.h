@@ -10,7 +10,7 @@
 //    arrays in molecule order; cell c owns sites [cstart_t[c], cstart_t[c+1]).
 //    Each site carries its position and its molecule's position (the mask is
 //    on molecule centres), FP64 absolute and FP32 relative to its cell's
-//    centre, its orientation (dipoles, quadrupoles) and its scalar parameter
+//    lower corner, its orientation (dipoles, quadrupoles) and its scalar parameter
 //    (LJ lookup id, charge, |mu|, |Q|), plus FP64 force / virial / torque
 //    outputs of the pair kernels.
 #pragma once

@@ -1,12 +1,18 @@
 // mdx_kernels.hip -- gfx950 kernels of the short-range force path.
 //
-// Step = leapfrog_pre (+ periodic wrap) -> bin_count -> scan -> bin_scatter
-//        -> bin_gather (stable counting sort) -> site scans -> build_sites
-//        -> pair kernels (one per i-site type) -> calc_fm -> leapfrog_post.
+// Step = leapfrog_pre (half kick, drift, periodic wrap, binning) -> scan ->
+//        bin_scatter -> bin_gather (stable counting sort) -> site scan ->
+//        build_sites -> pair kernels (one per i-site type) -> leapfrog_post (site
+//        sums = calcFM, half kick) -> step_end (the step's sums and record).
+// Consecutive steps without a thermostat take leapfrog_post and the next step's
+// leapfrog_pre in one pass (leapfrog_post_pre).
 // Systems of one-centre LJ molecules only: bin_gather_point (gather + site
 // cache) -> LJ pair kernel (writes molecule F, Vi) -> leapfrog_post.
+// Called one by one (re-bin, traversal, kicks) the same operations run unfused:
+// bin_count and calc_fm are then passes of their own.
 //
-// Pair kernels: one 64-lane wavefront per cell. Lane = (i-site, j-phase):
+// Pair kernels (mdx_pairs.hip; small dense boxes: mdx_pairs_block.hip): one
+// 64-lane wavefront per cell. Lane = (i-site, j-phase):
 // the cell's n sites of the i type occupy n lanes per phase and the
 // min(floor(64/n), 8) phases stride over the j sites of the 27 neighbour cells
 // (periodic images through shift vectors, no halo copies). Stage A tests the
@@ -982,7 +988,7 @@ __global__ __launch_bounds__(256) void k_velocity_scale(MolArrays s, double *F, 
 // pair kernels' cell rows and of the leapfrog chunks' rows, the step record, the
 // thermostat's factors and the step count (before: two reductions of one or two
 // launches, two final kernels and the count, 4 to 5 us each; a batch's two
-// segmented sums 17 us each; now 4 us for 64 cells, 6 for 2744, 10 for a batch of
+// segmented sums 17 us each; now 4 us for 27 cells, 6 for 2744, 10 for a batch of
 // 64 boxes, 15 for 1 M molecules). Replica r's rows go to min(rows / kStepRows,
 // kStepBlocks) blocks (its own rows alone decide, so a replica's sums do not
 // depend on the batch); a replica of several blocks is finished by the block
