@@ -2145,12 +2145,11 @@ size_t adjoint_table_width(const mdx_context *c) {
     return std::max(nl * 4 * nl, (size_t)c->model.ncomp * kMaxSite * 2);
 }
 
-// The adjoint's one array each way goes as a plain copy below 8 MB, and through the
-// ring with helping threads from there on (no conversion of the caller's follows
-// that would take their CPUs). us a call, plain / ring alone / ring with two
-// threads: 0.2 MB 146 / 168 / -, 0.8 MB 189 / 210 / -, 3 MB 465 / 495 / 522, 6 MB 805
-// / 830 / 777, 8 MB 1014 / 1040 / 934, 12 MB (500 k molecules) 1534 / 1490 / 1260: the
-// line lies where the threads, which take two CPUs for it, gain a tenth.
+// The adjoint's one array each way goes with helping threads from 8 MB on (no
+// conversion of the caller's follows that would take their CPUs). us a call without
+// / with two: 1.2 MB 289 / 368, 3 MB 497 / 522, 6 MB 834 / 777, 8 MB 1044 / 934, 12
+// MB (500 k molecules) 1498 / 1266: they pay from 4 MB on, and take two CPUs for it,
+// so the line lies where the gain is a tenth.
 constexpr size_t kAdjMany = 8u << 20;
 
 // The adjoint on the given buffers (no allocation): the LJ and charge
@@ -2165,15 +2164,10 @@ int adjoint_run(mdx_context *c, const double *cot, double *dU_deps, double *dU_d
     const int nn = c->n, ncomp = c->model.ncomp;
     const int nsl = c->nsites[T_LJ], nsc = c->nsites[T_C];
     MolArrays &m = c->mol[c->cur];
-    const size_t rows = (size_t)nn * 3 * 8;
     if (cot) {
-        if (rows < kAdjMany) {
-            HIPCHK(c, hipMemcpyAsync(c->dl_tmp, cot, rows, hipMemcpyHostToDevice, c->stream));
-        } else {
-            HostTransfer tr(b.ring, c->stream, c->device, rows, kAdjMany);
-            tr.to_device((char *)c->dl_tmp, {{(char *)cot, rows}});
-            HIPCHK(c, tr.finish());
-        }
+        HostTransfer tr(b.ring, c->stream, c->device, (size_t)nn * 3 * 8, kAdjMany);
+        tr.to_device((char *)c->dl_tmp, {{(char *)cot, (size_t)nn * 3 * 8}});
+        HIPCHK(c, tr.finish());
         hipLaunchKernelGGL(gather_orig3_kernel(), dim3(nblk(nn)), dim3(kBlock), 0, c->stream, nn,
                            m.orig, c->dl_tmp, b.cot);
     }
@@ -2241,13 +2235,9 @@ int adjoint_run(mdx_context *c, const double *cot, double *dU_deps, double *dU_d
     }
     if (c->timing) HIPCHK(c, hipEventRecord(c->ev[3], c->stream));
     if (vjp) {
-        if (rows < kAdjMany) {
-            HIPCHK(c, hipMemcpyAsync(vjp, b.cot, rows, hipMemcpyDeviceToHost, c->stream));
-        } else {
-            HostTransfer tr(b.ring, c->stream, c->device, rows, kAdjMany);
-            tr.to_host((const char *)b.cot, {{(char *)vjp, rows}});
-            HIPCHK(c, tr.finish());
-        }
+        HostTransfer tr(b.ring, c->stream, c->device, (size_t)nn * 3 * 8, kAdjMany);
+        tr.to_host((const char *)b.cot, {{(char *)vjp, (size_t)nn * 3 * 8}});
+        HIPCHK(c, tr.finish());
     }
     HIPCHK(c, hipStreamSynchronize(c->stream));
     if (c->timing) {
