@@ -2146,10 +2146,12 @@ size_t adjoint_table_width(const mdx_context *c) {
 }
 
 // The adjoint's one array each way goes with helping threads from 8 MB on (no
-// conversion of the caller's follows that would take their CPUs). us a call without
-// / with two: 1.2 MB 289 / 368, 3 MB 497 / 522, 6 MB 834 / 777, 8 MB 1044 / 934, 12
-// MB (500 k molecules) 1498 / 1266: they pay from 4 MB on, and take two CPUs for it,
-// so the line lies where the gain is a tenth.
+// conversion of the caller's follows that would take their CPUs). us a call, ring
+// alone / with two threads: 3 MB 495 / 522, 6 MB 830 / 777, 8 MB 1040 / 934, 12 MB
+// (500 k molecules) 1490 / 1260: the line lies where the threads, which take two
+// CPUs for it, gain a tenth. (Plain copies of the caller's pages, once the runtime
+// has made some 75 of them, take 10 to 30 us less than the ring alone: 4000 molecules
+// 137 / 157 us a call; before that 50 to 550 us more, 210 / 160, 770 / 215 for 32000.)
 constexpr size_t kAdjMany = 8u << 20;
 
 // The adjoint on the given buffers (no allocation): the LJ and charge
