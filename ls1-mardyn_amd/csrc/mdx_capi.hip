@@ -62,22 +62,33 @@ thread_local std::string g_create_error;
 constexpr int kBlock = 256;
 // Boxes of multi-site molecules with at most kSmallCells cells and, on average, at
 // least kSmallSites sites per cell and site type present run the block pair kernels,
-// four waves per cell (cells larger than kSmallVolume rc^3 count by volume). The
+// four waves per cell (cells larger than kSmallVolume rc^3 count by volume), and so
+// do those with kLiquidSites of each type and kLiquidMols molecules per rc^3. The
 // choice may depend on the box alone (a replica gives the bits it gives alone), so
 // it weighs a lone box, which leaves the chip idle, against a full batch of such
 // boxes, where the kernel that does less work per pair wins: what the block kernel
-// costs per cell pays off in dense cells only. us a step, block / cell kernel:
+// costs per cell pays off in dense cells only, with fewer sites where there are more
+// molecules (it tests those, not their sites). us a step, block / cell kernel:
 //   2CLJQ + water mixture, FP32     alone      batch of 400 k molecules
-//    18 molecules a cell, 64 cells  106 / 298  1429 / 1341
+//    30 molecules a cell, 512 cells 185 / 674  1820 / 2086
+//    18 molecules, 64 cells         106 / 298  1429 / 1341
 //    18 molecules, 512 cells        120 / 389  1409 / 1362
-//    30 molecules, 512 cells        185 / 674  1820 / 2086
+//    14 molecules, 512 cells        109 / 287  1431 / 1133
+//    14 molecules, 27 cells          75 / 211  1360 /  938  (the largest loss)
 //    10 molecules, 512 cells         85 / 165  1590 /  882  (beyond the line)
-// FP64, 18 molecules, 512 cells: 147 / 516 and 2304 / 2335; water alone, FP32, 18
-// and 30 molecules: 136 / 275 and 1534 / 1221, 229 / 474 and 2279 / 1802. Boxes of
-// one-centre molecules lose in every batch (512 x 500 molecules: 167 / 104 us of
-// pair kernel FP32, 186 / 147 FP64; 512 x 60: 87 / 38) for 12 us against 25 alone.
+//   the same FP64
+//    18 molecules, 512 cells        147 / 516  2304 / 2335
+//    14 molecules, 512 cells        131 / 377  2310 / 1877
+//   water, FP32, 512 cells
+//    30 molecules                   229 / 474  2279 / 1802
+//    18 molecules                   136 / 275  1534 / 1221
+//   2CLJQ, FP32, 512 cells
+//    11 molecules, 16 sites a type                1003 / 702   (beyond the line)
+// Boxes of one-centre molecules lose in every batch (512 x 500 molecules: 167 / 104
+// us of pair kernel FP32, 186 / 147 FP64; 512 x 60: 87 / 38) for 12 us against 25 alone.
 constexpr long kSmallCells = 512;
 constexpr double kSmallSites = 20.0, kSmallVolume = 1.5;
+constexpr double kLiquidSites = 15.0, kLiquidMols = 13.0;
 inline int nblk(long n, int b = kBlock) { return (int)std::max<long>(1, (n + b - 1) / b); }
 
 // Scratch of the entry points that allocate nothing (mdx_adjoint_noalloc):
@@ -1174,16 +1185,18 @@ int state_alloc(mdx_context *c, int n, const std::vector<int> &small) {
     return MDX_OK;
 }
 
-// Whether a box with nsites sites of each type is small: the block pair kernels'.
-bool small_box(const mdx_context *c, const Geom &g, const long (&nsites)[kTypes]) {
+// Whether a box with n molecules and nsites sites of each type is small: the block
+// pair kernels'.
+bool small_box(const mdx_context *c, const Geom &g, int64_t n, const long (&nsites)[kTypes]) {
     const long ncell = (long)g.n[0] * g.n[1] * g.n[2];
     if (c->point_lj || ncell > kSmallCells) return false;
     long sites = 0;
     int types = 0;
     for (int t = 0; t < kTypes; ++t) sites += nsites[t], types += nsites[t] > 0;
-    const double cells =
-        std::max((double)ncell, g.L[0] * g.L[1] * g.L[2] / (kSmallVolume * c->rc * c->rc * c->rc));
-    return sites > 0 && sites >= kSmallSites * types * cells;
+    const double volume = g.L[0] * g.L[1] * g.L[2] / (c->rc * c->rc * c->rc);
+    const double cells = std::max((double)ncell, volume / kSmallVolume);
+    return sites > 0 && (sites >= kSmallSites * types * cells ||
+                         (sites >= kLiquidSites * types * volume && n >= kLiquidMols * volume));
 }
 
 int state_setup(mdx_context *c, int64_t n64, const int32_t *cid_host) {
@@ -1210,7 +1223,7 @@ int state_setup(mdx_context *c, int64_t n64, const int32_t *cid_host) {
             for (int t = 0; t < kTypes; ++t)
                 box[t] += (mols[0][k] + mols[1][k] + mols[2][k] + mols[3][k]) * c->model.comp[k].n[t];
         for (int t = 0; t < kTypes; ++t) nsites[t] += box[t];
-        small[r] = small_box(c, c->geoms[r], box);
+        small[r] = small_box(c, c->geoms[r], c->nrep > 1 ? c->rep_n[r] : n64, box);
         if (small[r])
             for (int k = c->cell_off[r]; k < c->cell_off[r + 1]; ++k) small_cells.push_back(k);
     }

@@ -1,6 +1,7 @@
 """Which boxes run the block pair kernels (four waves per cell): at most 512 cells
 and, on average, at least 20 sites per cell and site type present, multi-site
-molecules (cells larger than 1.5 rc^3 count by volume). Every case says on which
+molecules (cells larger than 1.5 rc^3 count by volume), or 15 sites of each type
+and 13 molecules per rc^3. Every case says on which
 side of the rule its box lies, so that none moves to the other kernel unseen:
 dense boxes against the oracle where the block kernels' split can go wrong, and
 sparse and one-centre ones, which lost time to them, for the time of a batch.
@@ -32,7 +33,9 @@ def blocks(s):
     ncell = int(np.prod(cells(s)))
     if ncell > 512:
         return False
-    return sum(n) >= 20 * sum(x > 0 for x in n) * max(ncell, np.prod(s.box) / (1.5 * s.rc**3))
+    volume, types = np.prod(s.box) / s.rc**3, sum(x > 0 for x in n)
+    return (sum(n) >= 20 * types * max(ncell, volume / 1.5)
+            or sum(n) >= 15 * types * volume and s.n >= 13 * volume)
 
 
 def check(s, periodic=True, cell_mode=0):
@@ -103,7 +106,8 @@ def crowd(s, corner, share, seed):
     return s
 
 
-@pytest.mark.parametrize("n,rho", [(500, .5), (1500, .5), (4000, .5), (9001, .5), (1777, .9)])
+@pytest.mark.parametrize("n,rho", [(500, .5), (1500, .5), (4000, .5), (9001, .5), (1777, .9),
+                                   (3468, .5), (499, .49), (7000, .49)])
 def test_mixture(n, rho):
     print("mixture", n, rho, flush=True)
     s = scenarios.mixture(n=n, rho=rho, seed=n)
